@@ -66,12 +66,13 @@ typedef struct tdc_conv_desc {
  * as many rows as fit in the workgroup's mf*nb*wn pixel lanes); its wm*wn*wk
  * computing wavefronts split output channels, pixels and input channels; input channels
  * are staged through LDS `cch` at a time, double-buffered (alg 0-2), or requested from
- * global memory into registers all at once (alg 3-6). */
+ * global memory into registers all at once (alg 3-6) or a run ahead (alg 7). */
 typedef struct tdc_tile {
     int32_t mf;   /* MFMA block edge: 32 (v_mfma_f32_32x32x2_f32) or 16 (16x16x4) */
     int32_t mb;   /* MFMA blocks per wave along output channels (1 or 2)        */
     int32_t nb;   /* MFMA blocks per wave along pixels (1 or 2; alg 4 and 6 also 4: the
-                     workgroup's tile is nb 16-pixel blocks side by side along a row)  */
+                     workgroup's tile is nb 16-pixel blocks side by side along a row;
+                     alg 7: 2 or 4)                                              */
     int32_t wm;   /* waves along output channels                               */
     int32_t wn;   /* waves along pixels                                        */
     int32_t wk;   /* waves along input channels (in-workgroup split-K)          */
@@ -113,6 +114,11 @@ typedef struct tdc_tile {
                          from there.  3x3 / dilation 1, pad <= 1, stride <= 2; same shapes, cch / wk / ks rules and
                          fused tail as alg 4 (nb = 4: at most two channel groups per wave).  The input base address
                          and row pitch need not be 16-byte aligned: the requests are element-masked at the row ends.
+                     7 = 1x1 / pad 0 convolution (any stride) for batches: 16 * mb channels x 16 * nb pixels per wave (mb 1 or 2,
+                         nb 2 or 4), operands straight into registers one run of 16 channels ahead of the MFMAs; wm x wn
+                         waves over channels and pixels, wk over input channels (at most 8 together; cch = C rounded up to
+                         16 * wk); the pixels of all images in one row, so grid_x counts them and grid_z is 1; tw = 1,
+                         ks = 1, wl = 0.  Carries the input affine, not a fused tail.
                      The model offers 3 to 6 where launch and latency dominate (few channels or few pixels); the
                      staged paths keep the layers whose operands are worth sharing through the LDS. */
 } tdc_tile;

@@ -163,7 +163,9 @@ int tdc_model_select_with_tail(const tdc_conv_desc *desc, int32_t tail_N, tdc_ti
 int tdc_model_kernel_info(const tdc_conv_desc *desc, const tdc_tile *tile, int32_t extras, char *name_out, int32_t cap,
                           int32_t *vgprs_out, int32_t *waves_per_simd_out) {
     if (!desc || !tile || (cap > 0 && !name_out)) return fail(TDC_ERR_INVALID, "null argument");
-    const KernelId k = kernel_id_for(*tile, desc->KH, desc->KW, desc->dilation, desc->stride, extras != 0);
+    Geometry g;
+    const bool single_pixels = tile->alg == 7 && make_geometry(*desc, *tile, g, nullptr) && g.gen;
+    const KernelId k = kernel_id_for(*tile, desc->KH, desc->KW, desc->dilation, desc->stride, extras != 0, single_pixels);
     if (k.family == KernelId::NONE) return fail(TDC_ERR_UNSUPPORTED, "no kernel instantiated for this tile");
     const std::string name = kernel_name(k);
     if (cap > 0) {
@@ -371,10 +373,12 @@ static void refresh_launch_params(tdc_conv_plan *plan) {
     kp.fd_tw = make_fastdiv(g.TW);
     kp.fd_ntx = make_fastdiv(g.ntx);
     kp.fd_pt = make_fastdiv(g.PT);
-    kp.fd_wtw = make_fastdiv(g.wino ? g.TWt : (plan->tile.alg == 3 && d.stride > 1) ? g.Wo : 1);
+    kp.fd_wtw = make_fastdiv(g.wino ? g.TWt : ((plan->tile.alg == 3 && d.stride > 1) || plan->tile.alg == 7) ? g.Wo : 1);
     kp.fd_wk = make_fastdiv(plan->tile.wk);
     kp.fd_wn = make_fastdiv(plan->tile.wn);
     kp.fd_ks = make_fastdiv(g.ks);
+    kp.units = g.units;
+    kp.fd_units = make_fastdiv(std::max(g.units_image, 1));
     kp.grid_x = g.grid_x; kp.grid_y = g.grid_y;
     kp.n_wg = g.grid_x * g.grid_y * g.grid_z;
     kp.xcd_chunk = (kp.n_wg + 7) / 8;
@@ -421,7 +425,7 @@ int tdc_conv_plan_create_with_tail(const tdc_conv_desc *desc, int32_t tail_N, in
     }
     p->tile = p->info.tile;
     if (!make_geometry(*desc, p->tile, p->geo, &why, tail_N)) return fail(TDC_ERR_INVALID, why);
-    p->kernel = conv_kernel_for(p->tile, desc->KH, desc->KW, desc->dilation, desc->stride, tail_N > 0);
+    p->kernel = conv_kernel_for(p->tile, desc->KH, desc->KW, desc->dilation, desc->stride, tail_N > 0, p->geo.gen);
     if (!p->kernel) return fail(TDC_ERR_UNSUPPORTED, "no kernel instantiated for this tile");
     int he = prepare_conv_kernel(p->kernel, p->geo, &p->kernel_handle);
     if (he) return hip_fail("kernel set-up (hipFuncSetAttribute / hipGetFuncBySymbol)", he);
@@ -530,7 +534,7 @@ int tdc_conv_plan_set_input_affine(tdc_conv_plan *plan, const float *scale, cons
     if (e == hipSuccess) e = hipMemcpy(plan->d_in_aff, packed.data(), n * sizeof(float), hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail("input affine upload", e);
     // from now on this plan needs the kernel instantiation that carries the extras
-    plan->kernel = conv_kernel_for(plan->tile, d.KH, d.KW, d.dilation, d.stride, true);
+    plan->kernel = conv_kernel_for(plan->tile, d.KH, d.KW, d.dilation, d.stride, true, plan->geo.gen);
     if (!plan->kernel) return fail(TDC_ERR_UNSUPPORTED, "no kernel instantiated for this tile");
     if (int he = prepare_conv_kernel(plan->kernel, plan->geo, &plan->kernel_handle)) return hip_fail("kernel set-up (hipFuncSetAttribute / hipGetFuncBySymbol)", he);
     plan->in_relu = relu != 0;
@@ -675,8 +679,23 @@ static int forward_impl(tdc_conv_plan *plan, const float *d_in, int64_t in_batch
         kp.fd_csv = plan->fd_csv1;
         kp.fd_rsv = plan->fd_rsv1;
     }
-    int he = launch_conv(plan->kernel_handle, g, kp, stream);
-    if (he) return hip_fail("kernel launch", he);
+    // tile.alg = 7 addresses the images that one wave's pixels lie in through 32-bit offsets from the first of them: where
+    // they are too far apart for that (a slice of a much wider buffer), the images are launched one by one.
+    const bool one_by_one = plan->tile.alg == 7 && (g.unit_images * kp.in_bstride + in_image) * 4 >= (1LL << 31);
+    const int images = one_by_one ? d.batch : 1;
+    if (one_by_one) {
+        kp.units = g.units_image;
+        kp.grid_x = (g.units_image + 16 * (g.gen ? plan->tile.nb : 1) * plan->tile.wn - 1) / (16 * (g.gen ? plan->tile.nb : 1) * plan->tile.wn);
+        kp.n_wg = kp.grid_x * kp.grid_y;
+        kp.xcd_chunk = (kp.n_wg + 7) / 8;
+        if (kp.channel_major) kp.fd_g1 = make_fastdiv(kp.grid_x);
+    }
+    for (int b = 0; b < images; ++b) {
+        if (int he = launch_conv(plan->kernel_handle, g, kp, stream)) return hip_fail("kernel launch", he);
+        kp.in += kp.in_bstride;
+        kp.out += kp.out_bstride;
+        if (kp.resid) kp.resid += kp.resid_bstride;
+    }
     return TDC_OK;
 }
 

@@ -63,6 +63,10 @@ struct Geometry {
     int nstage = 1;
     int lds_bytes = 0;
     int max_waves_kernel = 0;        // launch bound of the instantiated kernel
+    // tile.alg = 7: the pixels of the whole batch in one row of units (groups of nb pixels of one image, or single pixels)
+    int units = 0, units_image = 0;
+    int gen = 0;                     // single pixels
+    int unit_images = 0;             // images that the units of one wave reach past the first one's
     int channel_major = 0;           // which logical workgroup order costs fewer L2 fills (see conv_staged.hip)
     double b_ways = 1.0;             // serialisation of the B-operand LDS read by bank conflicts (1 = none)
 };
@@ -148,6 +152,8 @@ struct ConvKParams {
     FastDiv fd_tw, fd_ntx, fd_pt;
     FastDiv fd_wtw;            // Winograd: 2x2 tiles per row of the workgroup tile; streamed 1x1 with stride > 1: output row length
     FastDiv fd_wk, fd_wn, fd_ks;
+    int units;                 // tile.alg = 7: pixel groups of the whole batch, and per image (see Geometry)
+    FastDiv fd_units;
     unsigned wpk_bytes;
     unsigned in_image_bytes;   // C*H*W*4: reads at or past it return zero
     long long in_bstride;      // floats between consecutive images of the input (C*H*W when dense)
@@ -168,13 +174,15 @@ enum : int { TAPS_GENERIC = 0, TAPS_1x1 = 1, TAPS_3x3 = 9, TAPS_3x3G = 10, TAPS_
 //   STREAM_3x3  tdc_conv3x3_stream_kernel<CG, INP, MODE>              p = {CG, INP, MODE, 1}   (INP: 0 taps, 1 row shifts, 2 window in LDS)
 //               tdc_conv3x3_stream_rownb_kernel<CG, NB>               p = {CG, 1, 0, NB}   (NB = 2 or 4 pixel blocks per wave)
 //   STREAM_WINO tdc_wino3x3_stream_kernel<CG, MAXW>                   p = {CG, MAXW}
+//   BLOCK_1x1   tdc_conv1x1_block_kernel<MB, NJ, AFF, GEN>            p = {MB, NJ, AFF, GEN}
 struct KernelId {
-    enum Family : int { NONE = 0, STAGED = 1, STREAM_1x1 = 2, STREAM_3x3 = 3, STREAM_WINO = 4 };
+    enum Family : int { NONE = 0, STAGED = 1, STREAM_1x1 = 2, STREAM_3x3 = 3, STREAM_WINO = 4, BLOCK_1x1 = 5 };
     int family = NONE;
     int p[6] = {0, 0, 0, 0, 0, 0};
 };
 // `extras`: the instantiation that also carries the input affine and the fused 1x1 tail.  family == NONE: no kernel.
-KernelId kernel_id_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras);
+// `single_pixels`: tile.alg = 7 addresses its pixels one by one (Geometry::gen).
+KernelId kernel_id_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras, bool single_pixels);
 KernelId kernel_id_with_head(const tdc_tile &t);
 // Streamed Winograd kernel (tile.alg = 5): waves per workgroup it is built for, by groups of four channels per wave (0 = none).
 int wino_stream_max_waves(int groups);   // streamed 3x3 with fused 1x1 head and tail
@@ -188,12 +196,13 @@ int kernel_vgprs(const KernelId &k);
 int kernel_waves_per_simd(const KernelId &k);
 // The function itself (nullptr if not instantiated).
 const void *kernel_function(const KernelId &k);
-// (its parts, one per translation unit that holds kernels: conv_staged.hip, conv_stream.hip, conv_wino_stream.hip)
+// (its parts, one per translation unit that holds kernels: conv_staged.hip, conv_stream.hip, conv_wino_stream.hip, conv_block.hip)
 const void *staged_kernel_function(const KernelId &k);
 const void *stream_kernel_function(const KernelId &k);
 const void *wino_stream_kernel_function(const KernelId &k);
-inline const void *conv_kernel_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras) {
-    return kernel_function(kernel_id_for(t, KH, KW, dilation, stride, extras));
+const void *block_kernel_function(const KernelId &k);
+inline const void *conv_kernel_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras, bool single_pixels) {
+    return kernel_function(kernel_id_for(t, KH, KW, dilation, stride, extras, single_pixels));
 }
 inline const void *conv_kernel_with_head(const tdc_tile &t) { return kernel_function(kernel_id_with_head(t)); }
 // One-time per-plan set-up: the dynamic-LDS attribute (above 64 KiB) and the kernel's module function handle on the

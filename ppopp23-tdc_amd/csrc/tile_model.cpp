@@ -14,6 +14,7 @@
 #include <map>
 #include <mutex>
 #include <shared_mutex>
+#include <unordered_map>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -114,8 +115,9 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     };
     if (!check_desc(d, why)) return false;
     if (t.mf != 32 && t.mf != 16) return fail("tile.mf must be 16 or 32");
-    if (t.mb < 1 || t.mb > 2 || t.nb < 1 || (t.nb > 2 && !((t.alg == 4 || t.alg == 6) && t.nb == 4)))
-        return fail("tile.mb / tile.nb must be 1 or 2 (tile.nb may be 4 for tile.alg = 4)");
+    if (t.mb < 1 || t.mb > 2 || t.nb < 1 ||
+        (t.nb > 2 && !((t.alg == 4 || t.alg == 6 || t.alg == 7) && t.nb == 4)))
+        return fail("tile.mb / tile.nb must be 1 or 2 (tile.nb may be 4 for tile.alg = 4, 6 and 7)");
     if (t.wm < 1 || t.wn < 1 || t.wk < 1) return fail("tile.wm / wn / wk must be >= 1");
     g = Geometry();
     // (256 registers per lane for the 2x2 block grid, 168 for the Winograd path)
@@ -126,6 +128,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         g.max_waves_kernel = wino_stream_max_waves(groups);
         if (!g.max_waves_kernel) return fail("tile.alg = 5 needs cch = 4 * wk * {1, 2, 3, 4}");
     }
+    if (t.alg == 7) g.max_waves_kernel = 8;
     if (t.wl < 0 || t.wl > 8) return fail("tile.wl must be in [0, 8]");
     if ((long long)t.wm * t.wn * t.wk + t.wl > g.max_waves_kernel) return fail("too many waves per workgroup for this tile");
     g.waves = t.wm * t.wn * t.wk + t.wl;
@@ -142,7 +145,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     g.taps = d.KH * d.KW;
     g.ktaps = g.taps;
     g.MT = t.mf * t.mb * t.wm;
-    if (t.alg < 0 || t.alg > 6) return fail("tile.alg must be in [0, 6]");
+    if (t.alg < 0 || t.alg > 7) return fail("tile.alg must be in [0, 7]");
     if (t.alg == 5) {
         // Winograd F(2x2,3x3) streamed from global memory: 16*wm channels of one tile row block (2 rows x 28 columns) per
         // workgroup, the input channels split over wk waves in groups of four, everything in one pass
@@ -192,6 +195,25 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         if (t.tw != std::min(16, g.P)) return fail("tile.alg = 3 needs tw = min(16, pixels)");
         if ((long long)t.cch * g.We * 4 >= (1LL << 31)) return fail("image too large for tile.alg = 3");
     }
+    if (t.alg == 7) {
+        // register-blocked 1x1 convolution: 16*mb channels x 16*nb pixels per wave, the pixels of the whole batch in one
+        // row of groups of nb (or single pixels, where a group does not fit an image or the convolution has a stride)
+        if (d.KH != 1 || d.KW != 1 || d.pad != 0) return fail("tile.alg = 7 needs a 1x1 / pad 0 convolution");
+        if (t.mf != 16 || (t.nb != 2 && t.nb != 4)) return fail("tile.alg = 7 needs mf = 16 and nb = 2 or 4");
+        if (t.wl != 0 || t.ks != 1) return fail("tile.alg = 7 has no loader waves and no split across workgroups");
+        if (tail_N > 0) return fail("tile.alg = 7 cannot carry a fused tail");
+        if (t.wk > 1 && t.wk > 4 * t.mb) return fail("tile.alg = 7: more channel slices than rows to finish");
+        if (t.cch % (16 * t.wk) != 0 || t.cch < d.C || t.cch - d.C >= 16 * t.wk)
+            return fail("tile.alg = 7 takes all input channels in one pass: cch = C rounded up to 16 * wk");
+        g.gen = !flat || g.P < t.nb;
+        g.units_image = g.gen ? g.P : ceil_div(g.P, t.nb);
+        if (t.tw != 1) return fail("tile.alg = 7 needs tw = 1");
+        const long long units = (long long)d.batch * g.units_image;
+        if (units * g.units_image >= (1LL << 32) || units >= (1LL << 30)) return fail("batch too large for tile.alg = 7");
+        g.units = (int)units;
+        g.unit_images = std::min(d.batch - 1, (16 * (g.gen ? t.nb : 1) - 2) / g.units_image + 1);
+        if ((long long)d.H * d.W * std::max(d.C, t.cch) * 4 >= (1LL << 31)) return fail("image too large for tile.alg = 7");
+    }
     if (t.alg == 2) {
         // direct 3x3 convolution with the weights read from global memory into registers, a pair of channel groups at a time
         if (d.KH != 3 || d.KW != 3 || d.dilation != 1) return fail("tile.alg = 2 needs a 3x3 / dilation 1 convolution");
@@ -218,6 +240,10 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         g.TW = 28;
         g.TH = 2;
         g.PT = 64;          // two rows of 32 columns in the parked tile (28 of them real)
+    } else if (t.alg == 7) {
+        g.PT = t.mf * t.nb * t.wn;
+        g.TW = std::min(g.PT, g.P);
+        g.TH = 1;
     } else {
         g.PT = t.mf * t.nb * t.wn;
         // (the streamed 1x1 kernel walks the output in runs of 16 consecutive pixels, whatever the image's rows are)
@@ -234,15 +260,19 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         g.ntx = ceil_div(g.P, 16);
         g.nty = 1;
     }
+    if (t.alg == 7) {
+        g.ntx = ceil_div(g.units, 16 * (g.gen ? t.nb : 1) * t.wn);
+        g.nty = 1;
+    }
     // (the kernel divides the tile index by ntx with a 32-bit multiply-high)
-    if ((long long)g.ntx * g.nty > 65535 * 16) return fail("grid too large");
-    if ((long long)g.ntx * g.nty * g.ntx >= (1LL << 32)) return fail("grid too large");
+    if (t.alg != 7 && (long long)g.ntx * g.nty > 65535 * 16) return fail("grid too large");
+    if (t.alg != 7 && (long long)g.ntx * g.nty * g.ntx >= (1LL << 32)) return fail("grid too large");
     g.grid_x = g.ntx * g.nty;
     g.grid_y = ceil_div(d.N, g.MT);
     if (t.ks < 1 || t.ks > 64) return fail("tile.ks must be in [1, 64]");
     g.ks = t.ks;
     if ((long long)d.batch * t.ks > 65535) return fail("grid too large");
-    g.grid_z = d.batch * t.ks;
+    g.grid_z = t.alg == 7 ? 1 : d.batch * t.ks;   // (alg 7: grid_x counts the pixels of all images)
     if (g.grid_y > 65535) return fail("grid too large");
     const int granule = g.kc * t.wk;
     if (t.cch < granule || t.cch % granule != 0) return fail("tile.cch must be a positive multiple of kc*wk");
@@ -323,7 +353,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     // Bytes the eight die-private L2s fill in total, for the two logical workgroup orders: with the channel
     // tiles of a pixel tile adjacent a die reads its share of the input and every weight; with the pixel tiles
     // of a channel tile adjacent it reads every input pixel of min(channel tiles, 8) ... and its own weights.
-    const double in_bytes = 4.0 * d.C * d.H * d.W, w_bytes = 4.0 * d.N * d.C * g.taps;
+    const double in_bytes = 4.0 * d.C * d.H * d.W * (t.alg == 7 ? d.batch : 1), w_bytes = 4.0 * d.N * d.C * g.taps;
     const double dies = (double)std::min<long long>(8, n_wg);
     const double pixel_major = in_bytes + dies * w_bytes;
     const double channel_major = std::min<double>(g.grid_y, dies) * in_bytes + std::max(1.0, dies / g.grid_y) * w_bytes;
@@ -356,11 +386,11 @@ void pack_weights(const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, 
                             }
         return;
     }
-    if (t.alg == 3) {
+    if (t.alg == 3 || t.alg == 7) {
         // per (channel block, run of 16 input channels): [lane][s], lane (n = l % 16, k = l / 16) holding
         // w[block*16 + n][16*run + 4*k + s]; the runs of all slices of a split across workgroups follow each other
         const int runs = g.nchunks * (t.cch / 16);
-        for (int by = 0; by < g.grid_y; ++by)
+        for (int by = 0; by < g.grid_y * mbw; ++by)
             for (int r = 0; r < runs; ++r)
                 for (int l = 0; l < 64; ++l)
                     for (int e = 0; e < 4; ++e) {
@@ -479,8 +509,16 @@ static const CompiledKernel *compiled_kernel(const KernelId &k) {
         for (const CompiledKernel &c : compiled_kernels) m[c.name] = &c;
         return m;
     }();
-    const auto it = by_name.find(kernel_name(k));
-    return it == by_name.end() ? nullptr : it->second;
+    // (a selection asks for the same hundred kernels tens of thousands of times: the name is spelt out once per thread)
+    static thread_local std::unordered_map<uint64_t, const CompiledKernel *> known;
+    uint64_t key = (uint64_t)k.family;
+    for (int v : k.p) key = key << 8 | (uint64_t)(v & 255);
+    auto hit = known.find(key);
+    if (hit == known.end()) {
+        const auto it = by_name.find(kernel_name(k));
+        hit = known.emplace(key, it == by_name.end() ? nullptr : it->second).first;
+    }
+    return hit->second;
 }
 
 // Waves of this kernel that fit one SIMD, as the compiler works it out from the registers of the compiled kernel:
@@ -509,8 +547,15 @@ KernelId kernel_id_with_head(const tdc_tile &t) {
 
 int wino_stream_max_waves(int groups) { return (groups >= 1 && groups <= 4) ? 16 : 0; }
 
-KernelId kernel_id_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras) {
+KernelId kernel_id_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras, bool single_pixels) {
     KernelId k;
+    if (t.alg == 7) {
+        // (`extras` here can only mean the input affine)
+        if (KH != 1 || KW != 1 || t.mf != 16 || (t.mb != 1 && t.mb != 2) || (t.nb != 2 && t.nb != 4)) return k;
+        k.family = KernelId::BLOCK_1x1;
+        k.p[0] = t.mb; k.p[1] = t.nb; k.p[2] = extras; k.p[3] = single_pixels;
+        return k;
+    }
     if (t.alg == 5) {
         if (extras || KH != 3 || KW != 3 || dilation != 1 || stride != 1 || t.mf != 16 || t.mb != 1 || t.nb != 1 || t.wn != 1 ||
             t.wm < 1 || t.wk < 1 || t.ks != 1 || t.cch % (4 * t.wk) != 0)
@@ -593,6 +638,9 @@ std::string kernel_name(const KernelId &k) {
         case KernelId::STREAM_WINO:
             std::snprintf(buf, sizeof buf, "tdc_wino3x3_stream_kernel<%d, %d>", k.p[0], k.p[1]);
             break;
+        case KernelId::BLOCK_1x1:
+            std::snprintf(buf, sizeof buf, "tdc_conv1x1_block_kernel<%d, %d, %s, %s>", k.p[0], k.p[1], tf[k.p[2] != 0], tf[k.p[3] != 0]);
+            break;
         default: return "";
     }
     return buf;
@@ -622,7 +670,7 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
     info.nchunks = g.nchunks;
     info.th = g.TH;
     // (a fused tail needs the instantiation with the extras; an input affine, which the model does not know of, too)
-    const KernelId kid = kernel_id_for(t, d.KH, d.KW, d.dilation, d.stride, tail_N > 0);
+    const KernelId kid = kernel_id_for(t, d.KH, d.KW, d.dilation, d.stride, tail_N > 0, g.gen);
     info.vgpr_estimate = kernel_vgprs(kid);
     if (info.vgpr_estimate <= 0) {
         if (why) *why = "no kernel instantiated for this tile";
@@ -800,6 +848,28 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
         }
         return clk;
     };
+    if (t.alg == 7) {
+        // Register-blocked 1x1: the whole launch at once, the largest of what the matrix pipes, a wave's own chain of runs,
+        // the address paths and the L2 need, + launch and first operands, + a share of the memory traffic that does not
+        // overlap (mostly the stores, which end together).  Fitted to 8000 timed tiles of 190 shapes, 7 % mean error, 1.5 %
+        // mean loss of the pick within the family.  The factor in front: the formulas of the other 1x1 families are some
+        // 8 % kind to launches of 4 us and more, and the pick between families has to fall at the measured crossover
+        // (there, at about 4 us, both run equally fast; at 10 us this one needs 0.8, at 30 us and more 0.6 of the time).
+        const double runs = (double)(t.cch / 16 / t.wk), run_clk = 4.0 * t.mb * t.nb * mfma_clk;
+        const double wgs_cu = (double)((n_wg + m.cus - 1) / m.cus);
+        const double waves_simd = std::max(1.0, (double)n_wg * g.waves / (m.cus * m.simds_per_cu));
+        const double waves_simd_most = std::ceil(wgs_cu * g.waves / m.simds_per_cu);
+        const double pipe = 1.366 * runs * run_clk * 0.5 * (waves_simd + waves_simd_most);
+        const double chain = runs * std::max(run_clk, 396.0);
+        const double requests = 18.6 * wgs_cu * g.waves * runs * (t.mb + (g.gen ? 4 * t.nb : 4));
+        const double l2 = (double)n_wg * t.wk * runs * (t.wm * t.mb + t.wn * t.nb) * 1024.0 / std::min<double>(m.cus, (double)n_wg) / 29.3;
+        double clk = 307.0 + std::max(std::max(pipe, chain), std::max(requests, l2));
+        if (t.wk > 1) clk += 232.0 + 20.5 * g.waves * t.mb * t.nb * std::min(wgs_cu, 4.0);
+        const double traffic = 4.0 * (d.batch * P * ((double)d.C + d.N) + (double)d.C * d.N);
+        info.pred_us = 0.92 * (2.67 + clk / (m.clock_ghz * 1e3) + traffic / 11.95e6);
+        info.pred_l2_bytes = 0.0;   // nothing is staged
+        return true;
+    }
     const long long slots = (long long)m.cus * wg_per_cu;
     const long long full = n_wg / slots;
     const long long rem = n_wg % slots;
@@ -840,6 +910,20 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
             }
         }
     }
+    // register-blocked 1x1 candidates
+    if (d.KH == 1 && d.KW == 1 && d.pad == 0 && tail_N == 0 && !std::getenv("TDC_EXPERIMENT_NO_BLOCKED_1X1")) {
+        for (int mb : {1, 2})
+            for (int nb : {2, 4})
+                for (int wm : wms)
+                    for (int wn : wns)
+                        for (int wk : {1, 2, 4, 8}) {
+                            // (the waves of a workgroup of two share a pair of SIMDs with those of the next one)
+                            if (wm * wn * wk > 8 || wm * wn * wk == 2 || 16 * mb * wm > round_up(d.N, 16 * mb)) continue;
+                            tdc_tile t{16, mb, nb, wm, wn, wk, round_up(d.C, 16 * wk), 1, 1, 0, 7};
+                            Geometry g;
+                            if (make_geometry(d, t, g, nullptr, 0)) out.push_back(t);
+                        }
+    }
     // streamed 3x3 candidates: 1, 2 or 4 groups of four channels per wave, a few shapes of the 16-pixel tile
     if (d.KH == 3 && d.KW == 3 && d.dilation == 1 && !std::getenv("TDC_EXPERIMENT_NO_STREAMED_3X3")) {
         std::vector<int> tws;
@@ -878,14 +962,14 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
                             if (ceil_div(Wo, 14) < nb) continue;
                             t.nb = nb;
                             if (make_geometry(d, t, g, nullptr, 0) &&
-                                kernel_id_for(t, 3, 3, 1, 1, false).family != KernelId::NONE)
+                                kernel_id_for(t, 3, 3, 1, 1, false, false).family != KernelId::NONE)
                                 out.push_back(t);
                             // ... and with the rows of all blocks loaded as one window through LDS
                             if (d.pad <= 1 && !std::getenv("TDC_EXPERIMENT_NO_STREAMED_WINDOW")) {
                                 tdc_tile t6 = t;
                                 t6.alg = 6;
                                 if (make_geometry(d, t6, g, nullptr, 0) &&
-                                    kernel_id_for(t6, 3, 3, 1, 1, false).family != KernelId::NONE)
+                                    kernel_id_for(t6, 3, 3, 1, 1, false, false).family != KernelId::NONE)
                                     out.push_back(t6);
                             }
                         }

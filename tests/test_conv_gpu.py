@@ -908,3 +908,70 @@ def test_errors():
     bad = tdc_amd.Tile(32, 1, 1, 1, 1, 1, 3, 4)  # cch not a multiple of kc
     with pytest.raises(tdc_amd.TdcError):
         tdc_amd.Conv2dPlan(1, 4, 4, 6, 6, 3, 3, 1, 1, tile=bad)
+
+
+@pytest.mark.parametrize("shape,stride", [((1, 64, 16, 7, 7), 1), ((3, 19, 5, 3, 3), 1), ((2, 100, 40, 5, 6), 1), ((35, 33, 70, 1, 1), 1),
+                                          ((4, 48, 33, 1, 3), 1), ((40, 16, 20, 2, 2), 1), ((2, 260, 64, 12, 11), 1),
+                                          ((2, 100, 40, 9, 11), 2), ((3, 19, 5, 7, 5), 3), ((9, 33, 17, 1, 9), 2)])
+def test_every_blocked_1x1_tile(shape, stride):
+    """The register-blocked 1x1 path (tile.alg = 7), every launchable tile: groups that straddle neither image end (49, 30,
+    132 pixels), end inside one (9 and 3 pixels), images smaller than a group (1 and 2x2 pixels: single pixels and groups),
+    a stride, ragged channels (a last run of 1, 3 and 4), more waves than runs; plain, then bias + residual + ReLU with
+    input, residual and output as channel slices that are only 4-byte aligned and the residual in place, then the input
+    affine."""
+    from ctypes import c_void_p
+    B, C, N, H, W = shape
+    x, w = case(8600 + C + N + H, B, C, N, H, W, 1)
+    g = seeded(8601)
+    bias = torch.randn(N, generator=g)
+    scale = torch.rand(C, generator=g) * 2 - 0.5
+    shift = torch.randn(C, generator=g) * 0.3
+    want = ref.conv2d_c(x.numpy(), w.numpy(), stride=stride)
+    Ho, Wo = want.shape[2], want.shape[3]
+    resid = torch.randn(B, N, Ho, Wo, generator=g)
+    want_full = ref.conv2d_c(x.numpy(), w.numpy(), bias.numpy(), resid.numpy(), stride=stride, relu=True)
+    xt = (x * scale.view(1, C, 1, 1) + shift.view(1, C, 1, 1)).clamp_min(0)
+    want_aff = ref.conv2d_c(xt.numpy(), w.numpy(), bias.numpy(), stride=stride, relu=True)
+    tiles = [t for t in tdc_amd.model_enumerate(tdc_amd.conv_desc(B, C, N, H, W, 1, 1, stride, 0)) if t.alg == 7]
+    assert {t.nb for t in tiles} == {2, 4} and {t.wk for t in tiles} >= {1, 4}
+    for t in tiles:
+        announce("blocked 1x1", shape, stride, t)
+        assert_close(run_conv(x, w, stride=stride, tile=t), want, f"{shape} s{stride} {t}")
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, 1, 1, stride, 0, 1, True, True, tile=t).set_weights(w, bias)
+        xin = torch.full((B, C + 3, H, W), float("nan"), device="cuda"); xin[:, 1:1 + C] = x.cuda()
+        obuf = torch.full((B, N + 5, Ho, Wo), 7.0, device="cuda"); obuf[:, 4:4 + N] = resid.cuda()
+        o = c_void_p(obuf[:, 4:].data_ptr())
+        tdc_amd._lib.check(tdc_amd.lib().tdc_conv_forward_strided(
+            plan._h, c_void_p(xin[:, 1:].data_ptr()), (C + 3) * H * W, o, (N + 5) * Ho * Wo, o, (N + 5) * Ho * Wo,
+            c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        got = obuf.cpu()
+        assert_close(got[:, 4:4 + N].numpy(), want_full, f"slices {shape} s{stride} {t}")
+        assert (got[:, :4] == 7.0).all() and (got[:, 4 + N:] == 7.0).all()
+        plan.set_input_affine(scale, shift, relu=True)
+        out = torch.full((B, N, Ho, Wo), float("nan"), device="cuda")
+        plan.forward(x.cuda(), out=out)
+        torch.cuda.synchronize()
+        plan.close()
+        assert_close(out.cpu().numpy(), want_aff, f"input affine {shape} s{stride} {t}")
+
+
+def test_blocked_1x1_with_images_far_apart():
+    """tile.alg = 7 reaches the images of one wave through 32-bit offsets; images 2 GiB apart are launched one by one."""
+    from ctypes import c_void_p
+    B, C, N, H, W = 3, 20, 24, 3, 5
+    x, w = case(8650, B, C, N, H, W, 1)
+    far = 1 << 29
+    buf = torch.empty(2 * far + C * H * W, device="cuda")
+    for b in range(B):
+        buf[b * far:b * far + C * H * W] = x[b].reshape(-1).cuda()
+    for t in [t for t in tdc_amd.model_enumerate(tdc_amd.conv_desc(B, C, N, H, W, 1, 1, 1, 0)) if t.alg == 7]:
+        announce("blocked 1x1 far apart", t)
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, 1, 1, tile=t).set_weights(w)
+        out = torch.full((B, N, H, W), float("nan"), device="cuda")
+        tdc_amd._lib.check(tdc_amd.lib().tdc_conv_forward_strided(
+            plan._h, c_void_p(buf.data_ptr()), far, None, 0, c_void_p(out.data_ptr()), 0,
+            c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        plan.close()
+        assert_close(out.cpu().numpy(), ref.conv2d_c(x.numpy(), w.numpy()), f"{t}")
