@@ -87,6 +87,10 @@ typedef struct tdc_tile {
                      1 = Winograd F(2x2,3x3) for 3x3 / stride 1 / dilation 1 convolutions: the pixel lanes hold
                          2x2-pixel output tiles (tw counts those tiles), 16 MFMAs per four input channels and 16
                          tiles instead of 36; weights read from global memory into registers; mf = 16, mb = nb = 1.
+                         With tw = 0 (pad <= 1, images of 8 pixels and more) the output tiles of the whole batch are counted
+                         in one row: 16 * mb channels (mb 1 or 2) x 16 tiles per wave, wn = 2 or 4 waves over tiles that
+                         share the weights through LDS, wk teams of them over input channels (at most 8 waves; cch = C
+                         rounded up to 8 * wk), input straight into registers; wm = nb = ks = 1, wl = 0, grid_z = 1.
                      2 = direct 3x3 / dilation 1 convolution with the weights read from global memory straight
                          into registers (the LDS holds input only, so a pass can take more input channels);
                          mb = nb = 1, an even number of channel groups per wave and pass.

@@ -377,6 +377,7 @@ static void refresh_launch_params(tdc_conv_plan *plan) {
     kp.fd_wk = make_fastdiv(plan->tile.wk);
     kp.fd_wn = make_fastdiv(plan->tile.wn);
     kp.fd_ks = make_fastdiv(g.ks);
+    kp.batch = d.batch;
     kp.units = g.units;
     kp.fd_units = make_fastdiv(std::max(g.units_image, 1));
     kp.grid_x = g.grid_x; kp.grid_y = g.grid_y;
@@ -679,13 +680,16 @@ static int forward_impl(tdc_conv_plan *plan, const float *d_in, int64_t in_batch
         kp.fd_csv = plan->fd_csv1;
         kp.fd_rsv = plan->fd_rsv1;
     }
-    // tile.alg = 7 addresses the images that one wave's pixels lie in through 32-bit offsets from the first of them: where
-    // they are too far apart for that (a slice of a much wider buffer), the images are launched one by one.
-    const bool one_by_one = plan->tile.alg == 7 && (g.unit_images * kp.in_bstride + in_image) * 4 >= (1LL << 31);
+    // The kernels that count the pixels (tiles) of the whole batch in one row address the images that one wave's pixels lie
+    // in through 32-bit offsets from the first of them: where they are too far apart for that (a slice of a much wider
+    // buffer), the images are launched one by one.
+    const bool one_by_one = g.units > 0 && (g.unit_images * kp.in_bstride + in_image) * 4 >= (1LL << 31) - 16;
     const int images = one_by_one ? d.batch : 1;
     if (one_by_one) {
+        const int per_wg = 16 * plan->tile.wn * (g.gen ? plan->tile.nb : 1);
+        kp.batch = 1;
         kp.units = g.units_image;
-        kp.grid_x = (g.units_image + 16 * (g.gen ? plan->tile.nb : 1) * plan->tile.wn - 1) / (16 * (g.gen ? plan->tile.nb : 1) * plan->tile.wn);
+        kp.grid_x = (g.units_image + per_wg - 1) / per_wg;
         kp.n_wg = kp.grid_x * kp.grid_y;
         kp.xcd_chunk = (kp.n_wg + 7) / 8;
         if (kp.channel_major) kp.fd_g1 = make_fastdiv(kp.grid_x);

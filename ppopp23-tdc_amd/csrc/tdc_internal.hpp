@@ -63,7 +63,8 @@ struct Geometry {
     int nstage = 1;
     int lds_bytes = 0;
     int max_waves_kernel = 0;        // launch bound of the instantiated kernel
-    // tile.alg = 7: the pixels of the whole batch in one row of units (groups of nb pixels of one image, or single pixels)
+    // tile.alg = 7: the pixels of the whole batch in one row of units (groups of nb pixels of one image, or single pixels);
+    // tile.alg = 1 with tw = 0: its 2x2 output tiles likewise
     int units = 0, units_image = 0;
     int gen = 0;                     // single pixels
     int unit_images = 0;             // images that the units of one wave reach past the first one's
@@ -152,7 +153,8 @@ struct ConvKParams {
     FastDiv fd_tw, fd_ntx, fd_pt;
     FastDiv fd_wtw;            // Winograd: 2x2 tiles per row of the workgroup tile; streamed 1x1 with stride > 1: output row length
     FastDiv fd_wk, fd_wn, fd_ks;
-    int units;                 // tile.alg = 7: pixel groups of the whole batch, and per image (see Geometry)
+    int batch;
+    int units;                 // tile.alg = 7, tile.tw = 0: pixel groups / tiles of the whole batch, and per image (see Geometry)
     FastDiv fd_units;
     unsigned wpk_bytes;
     unsigned in_image_bytes;   // C*H*W*4: reads at or past it return zero
@@ -174,9 +176,10 @@ enum : int { TAPS_GENERIC = 0, TAPS_1x1 = 1, TAPS_3x3 = 9, TAPS_3x3G = 10, TAPS_
 //   STREAM_3x3  tdc_conv3x3_stream_kernel<CG, INP, MODE>              p = {CG, INP, MODE, 1}   (INP: 0 taps, 1 row shifts, 2 window in LDS)
 //               tdc_conv3x3_stream_rownb_kernel<CG, NB>               p = {CG, 1, 0, NB}   (NB = 2 or 4 pixel blocks per wave)
 //   STREAM_WINO tdc_wino3x3_stream_kernel<CG, MAXW>                   p = {CG, MAXW}
+//   BLOCK_WINO  tdc_wino3x3_block_kernel<MB, WN>                      p = {MB, WN}
 //   BLOCK_1x1   tdc_conv1x1_block_kernel<MB, NJ, AFF, GEN>            p = {MB, NJ, AFF, GEN}
 struct KernelId {
-    enum Family : int { NONE = 0, STAGED = 1, STREAM_1x1 = 2, STREAM_3x3 = 3, STREAM_WINO = 4, BLOCK_1x1 = 5 };
+    enum Family : int { NONE = 0, STAGED = 1, STREAM_1x1 = 2, STREAM_3x3 = 3, STREAM_WINO = 4, BLOCK_1x1 = 5, BLOCK_WINO = 6 };
     int family = NONE;
     int p[6] = {0, 0, 0, 0, 0, 0};
 };
@@ -196,11 +199,12 @@ int kernel_vgprs(const KernelId &k);
 int kernel_waves_per_simd(const KernelId &k);
 // The function itself (nullptr if not instantiated).
 const void *kernel_function(const KernelId &k);
-// (its parts, one per translation unit that holds kernels: conv_staged.hip, conv_stream.hip, conv_wino_stream.hip, conv_block.hip)
+// (its parts, one per translation unit that holds kernels: conv_staged.hip, conv_stream.hip, conv_wino_stream.hip, conv_block.hip, conv_wino_block.hip)
 const void *staged_kernel_function(const KernelId &k);
 const void *stream_kernel_function(const KernelId &k);
 const void *wino_stream_kernel_function(const KernelId &k);
 const void *block_kernel_function(const KernelId &k);
+const void *wino_block_kernel_function(const KernelId &k);
 inline const void *conv_kernel_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras, bool single_pixels) {
     return kernel_function(kernel_id_for(t, KH, KW, dilation, stride, extras, single_pixels));
 }

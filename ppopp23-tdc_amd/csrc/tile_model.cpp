@@ -128,7 +128,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         g.max_waves_kernel = wino_stream_max_waves(groups);
         if (!g.max_waves_kernel) return fail("tile.alg = 5 needs cch = 4 * wk * {1, 2, 3, 4}");
     }
-    if (t.alg == 7) g.max_waves_kernel = 8;
+    if (t.alg == 7 || (t.alg == 1 && t.tw == 0)) g.max_waves_kernel = 8;
     if (t.wl < 0 || t.wl > 8) return fail("tile.wl must be in [0, 8]");
     if ((long long)t.wm * t.wn * t.wk + t.wl > g.max_waves_kernel) return fail("too many waves per workgroup for this tile");
     g.waves = t.wm * t.wn * t.wk + t.wl;
@@ -179,7 +179,34 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         if (ceil_div(d.C, t.cch) != t.ks) return fail("tile.alg = 4 takes its input channels in one pass: ks slices of cch channels must cover them exactly");
         if ((long long)t.cch * d.H * d.W * 4 >= (1LL << 31)) return fail("image too large for tile.alg = 4");
     }
+    const bool wino_batch = t.alg == 1 && t.tw == 0;
     g.wino = t.alg == 1;
+    if (wino_batch) {
+        // Winograd over the 2x2 tiles of the whole batch: 16*mb channels x 16*wn tiles per workgroup, wk teams of wn waves
+        // split the input channels, two groups of four channels per step
+        if (d.KH != 3 || d.KW != 3 || d.stride != 1 || d.dilation != 1 || d.pad > 1)
+            return fail("tile.alg = 1 with tw = 0 needs a 3x3 / stride 1 / dilation 1 / pad <= 1 convolution");
+        if (t.mf != 16 || t.wm != 1 || (t.wn != 2 && t.wn != 4) || t.nb != 1)
+            return fail("tile.alg = 1 with tw = 0 needs mf = 16, wm = nb = 1, wn = 2 or 4");
+        if (t.wl != 0 || t.ks != 1) return fail("tile.alg = 1 with tw = 0 has no loader waves and no split across workgroups");
+        if (tail_N > 0) return fail("tile.alg = 1 cannot carry a fused tail");
+        if (t.wk > 4 * t.mb) return fail("tile.alg = 1 with tw = 0: more teams than rows to finish");
+        const int granule = 8 * t.wk;
+        if (t.cch % granule != 0 || t.cch < d.C || t.cch - d.C >= granule)
+            return fail("tile.alg = 1 with tw = 0 takes all input channels: cch = C rounded up to 8 * wk");
+        g.ktaps = 16;
+        g.TWt = ceil_div(g.Wo, 2);
+        g.THt = ceil_div(g.Ho, 2);
+        g.units_image = g.TWt * g.THt;
+        const long long units = (long long)d.batch * g.units_image;
+        if (units * g.units_image >= (1LL << 32) || units >= (1LL << 30)) return fail("batch too large for tile.alg = 1 with tw = 0");
+        if (d.H * d.W < 8) return fail("tile.alg = 1 with tw = 0 needs images of at least 8 pixels");
+        g.units = (int)units;
+        g.unit_images = std::min(d.batch - 1, 14 / g.units_image + 1);
+        g.TW = 2 * std::min(g.TWt, 16 * t.wn);
+        g.TH = 2;
+        g.PT = 64 * t.wn;
+    }
     if (t.alg == 3) {
         // 1x1 convolution streamed from global memory: a 16x16 output block per workgroup, the input channels split
         // over wk waves in runs of 16, everything in one pass
@@ -221,7 +248,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         if (tail_N > 0) return fail("tile.alg = 2 cannot carry a fused tail");
         if (t.cch % (2 * g.kc * t.wk) != 0) return fail("tile.alg = 2 needs an even number of channel groups per wave and pass");
     }
-    if (t.alg == 1) {
+    if (t.alg == 1 && !wino_batch) {
         // Winograd F(2x2,3x3): a pixel lane holds one 2x2 output tile; the workgroup tile is THt x TWt such tiles.
         if (d.KH != 3 || d.KW != 3 || d.stride != 1 || d.dilation != 1) return fail("tile.alg needs a 3x3 / stride 1 / dilation 1 convolution");
         if (t.mf != 16 || t.mb != 1 || t.nb != 1) return fail("tile.alg needs mf = 16, mb = nb = 1");
@@ -235,6 +262,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         g.TW = 2 * g.TWt;
         g.TH = 2 * g.THt;
         g.PT = 4 * lanes;   // pixels the workgroup's lanes stand for
+    } else if (wino_batch) {
     } else if (t.alg == 5) {
         g.ktaps = 16;
         g.TW = 28;
@@ -264,19 +292,24 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         g.ntx = ceil_div(g.units, 16 * (g.gen ? t.nb : 1) * t.wn);
         g.nty = 1;
     }
+    if (wino_batch) {
+        g.ntx = ceil_div(g.units, 16 * t.wn);
+        g.nty = 1;
+    }
+    const bool flat_batch = t.alg == 7 || wino_batch;   // grid_x counts the pixels (tiles) of all images
     // (the kernel divides the tile index by ntx with a 32-bit multiply-high)
-    if (t.alg != 7 && (long long)g.ntx * g.nty > 65535 * 16) return fail("grid too large");
-    if (t.alg != 7 && (long long)g.ntx * g.nty * g.ntx >= (1LL << 32)) return fail("grid too large");
+    if (!flat_batch && (long long)g.ntx * g.nty > 65535 * 16) return fail("grid too large");
+    if (!flat_batch && (long long)g.ntx * g.nty * g.ntx >= (1LL << 32)) return fail("grid too large");
     g.grid_x = g.ntx * g.nty;
     g.grid_y = ceil_div(d.N, g.MT);
     if (t.ks < 1 || t.ks > 64) return fail("tile.ks must be in [1, 64]");
     g.ks = t.ks;
     if ((long long)d.batch * t.ks > 65535) return fail("grid too large");
-    g.grid_z = t.alg == 7 ? 1 : d.batch * t.ks;   // (alg 7: grid_x counts the pixels of all images)
+    g.grid_z = flat_batch ? 1 : d.batch * t.ks;
     if (g.grid_y > 65535) return fail("grid too large");
     const int granule = g.kc * t.wk;
     if (t.cch < granule || t.cch % granule != 0) return fail("tile.cch must be a positive multiple of kc*wk");
-    if (t.alg < 3 && t.cch > round_up(d.C, granule)) return fail("tile.cch exceeds the (padded) channel count");
+    if (t.alg < 3 && !wino_batch && t.cch > round_up(d.C, granule)) return fail("tile.cch exceeds the (padded) channel count");
     g.cpw = t.cch / t.wk;
     g.nchunks = ceil_div(d.C, t.cch);
     g.c_pad = g.nchunks * t.cch;
@@ -308,13 +341,15 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     g.aff_floats = (d.KH == 1 && d.KW == 1 && d.pad == 0) ? round_up(2 * t.cch, 256) : 0;
     // (the Winograd path reads its weights straight from global memory into registers: the LDS holds input only)
     g.stage_floats = g.in_stage_floats + (t.alg ? 0 : round_up(g.wslab_floats, 256)) + g.aff_floats;   // (wino = 2 likewise)
-    if (t.alg >= 3) g.in_stage_floats = g.aff_floats = g.stage_floats = 0;   // nothing is staged
+    if (t.alg >= 3 || wino_batch) g.in_stage_floats = g.aff_floats = g.stage_floats = 0;   // nothing is staged
     g.nstage = g.cps > 1 ? 2 : 1;
     const long long stage_bytes = (long long)g.nstage * g.stage_floats * 4;
     // (the Winograd path always parks its output tiles in LDS, also without a split over waves)
     // (... and so does the streamed 3x3 kernel with several pixel blocks per wave: all its threads share the final store)
     const long long red_bytes = (t.wk > 1 || t.alg == 1 || t.alg == 5 || ((t.alg == 4 || t.alg == 6) && t.nb > 1)) ? (long long)t.wk * g.MT * g.PT * 4 : 0;
     long long lds = std::max(stage_bytes, red_bytes);
+    if (wino_batch)   // two buffers of transformed weights per team, or the outputs of all teams
+        lds = std::max<long long>(2LL * t.wk * t.mb * 2 * 4096, t.wk > 1 ? (long long)t.wk * t.wn * t.mb * 4096 : 0);
     if (tail_N > 0) {
         // A fused 1x1 tail needs every output channel of the convolution in one workgroup; its tile is parked
         // in LDS behind the split-K partials with a row stride that keeps the four channel quarters of a
@@ -353,7 +388,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     // Bytes the eight die-private L2s fill in total, for the two logical workgroup orders: with the channel
     // tiles of a pixel tile adjacent a die reads its share of the input and every weight; with the pixel tiles
     // of a channel tile adjacent it reads every input pixel of min(channel tiles, 8) ... and its own weights.
-    const double in_bytes = 4.0 * d.C * d.H * d.W * (t.alg == 7 ? d.batch : 1), w_bytes = 4.0 * d.N * d.C * g.taps;
+    const double in_bytes = 4.0 * d.C * d.H * d.W * (flat_batch ? d.batch : 1), w_bytes = 4.0 * d.N * d.C * g.taps;
     const double dies = (double)std::min<long long>(8, n_wg);
     const double pixel_major = in_bytes + dies * w_bytes;
     const double channel_major = std::min<double>(g.grid_y, dies) * in_bytes + std::max(1.0, dies / g.grid_y) * w_bytes;
@@ -549,6 +584,14 @@ int wino_stream_max_waves(int groups) { return (groups >= 1 && groups <= 4) ? 16
 
 KernelId kernel_id_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras, bool single_pixels) {
     KernelId k;
+    if (t.alg == 1 && t.tw == 0) {
+        if (extras || KH != 3 || KW != 3 || dilation != 1 || stride != 1 || t.mf != 16 || t.wm != 1 || (t.wn != 2 && t.wn != 4) ||
+            (t.mb != 1 && t.mb != 2) || t.nb != 1)
+            return k;
+        k.family = KernelId::BLOCK_WINO;
+        k.p[0] = t.mb; k.p[1] = t.wn;
+        return k;
+    }
     if (t.alg == 7) {
         // (`extras` here can only mean the input affine)
         if (KH != 1 || KW != 1 || t.mf != 16 || (t.mb != 1 && t.mb != 2) || (t.nb != 2 && t.nb != 4)) return k;
@@ -637,6 +680,9 @@ std::string kernel_name(const KernelId &k) {
             break;
         case KernelId::STREAM_WINO:
             std::snprintf(buf, sizeof buf, "tdc_wino3x3_stream_kernel<%d, %d>", k.p[0], k.p[1]);
+            break;
+        case KernelId::BLOCK_WINO:
+            std::snprintf(buf, sizeof buf, "tdc_wino3x3_block_kernel<%d, %d>", k.p[0], k.p[1]);
             break;
         case KernelId::BLOCK_1x1:
             std::snprintf(buf, sizeof buf, "tdc_conv1x1_block_kernel<%d, %d, %s, %s>", k.p[0], k.p[1], tf[k.p[2] != 0], tf[k.p[3] != 0]);
@@ -848,6 +894,25 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
         }
         return clk;
     };
+    if (t.alg == 1 && t.tw == 0) {
+        // Winograd over the tiles of the batch: like the register-blocked 1x1 below (the largest of matrix pipes, a wave's
+        // own chain of channel groups and the L2, + launch and first operands, + the end of every workgroup, + the memory
+        // traffic).  Fitted to 1160 timed tiles of 145 shapes, 7 % mean error, 1.7 % mean loss of the pick within the
+        // family.  The factor in front puts the pick between families at the measured crossover, about 6 us: below it the
+        // streamed kernels, whose formulas are kind to launches of this length, have the shorter start.
+        const double groups = (double)t.cch / (4.0 * t.wk);
+        const double wgs_cu = (double)((n_wg + m.cus - 1) / m.cus);
+        const double load = std::ceil(wgs_cu * g.waves / m.simds_per_cu);
+        const double pipe = groups * (16.0 * t.mb * mfma_clk + 182.0) * load;
+        const double chain = groups * (16.0 * t.mb * mfma_clk + 394.0);
+        const double l2 = (double)n_wg * groups * (t.wk * t.mb * 4096.0 + g.waves * 1100.0) / std::min<double>(m.cus, (double)n_wg) / 20.2;
+        double clk = std::max(std::max(pipe, chain), l2) + 620.0 * t.mb * load;
+        if (t.wk > 1) clk += 707.0 + 58.0 * g.waves * t.mb * std::min(wgs_cu, 3.0);
+        const double traffic = 4.0 * (d.batch * ((double)d.C * d.H * d.W + (double)d.N * P) + 16.0 * d.C * d.N);
+        info.pred_us = 0.85 * (3.12 + clk / (m.clock_ghz * 1e3) + traffic / 4.45e6);
+        info.pred_l2_bytes = 0.0;
+        return true;
+    }
     if (t.alg == 7) {
         // Register-blocked 1x1: the whole launch at once, the largest of what the matrix pipes, a wave's own chain of runs,
         // the address paths and the L2 need, + launch and first operands, + a share of the memory traffic that does not
@@ -997,8 +1062,25 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
             }
         }
     }
+    // Winograd over the tiles of the whole batch: batches, and single images of more than 64x64 pixels (224x224 17.3 -> 15.0
+    // us, 96x96 14.6 -> 12.4; at 56x56 the streamed Winograd kernel is as fast).  It leaves nothing to the staged one there.
+    const bool wino_batch = (d.batch > 1 || P > 4096) && d.KH == 3 && d.KW == 3 && d.stride == 1 && d.dilation == 1 && d.pad <= 1 &&
+                            d.H * d.W >= 8 && tail_N == 0 && !std::getenv("TDC_EXPERIMENT_NO_WINOGRAD");
+    if (wino_batch)
+        for (int mb : {1, 2})
+            for (int wn : {2, 4})
+                for (int wk : {1, 2, 4}) {
+                    if (wn * wk > 8 || wn * wk < 4 || 16 * mb > round_up(d.N, 16)) continue;
+                    tdc_tile t{16, mb, 1, 1, wn, wk, round_up(d.C, 8 * wk), 0, 1, 0, 1};
+                    Geometry g;
+                    if (!make_geometry(d, t, g, nullptr, 0)) continue;
+                    // (32 channels x 32 tiles, the weights shared by two waves only: deep layers of small images, whose
+                    //  workgroups fit the chip at once; 256 -> 256 @7 batch 64 25.8 us against 28.2)
+                    if (mb == 2 && wn == 2 && (wk < 4 || g.grid_x * g.grid_y > machine().cus)) continue;
+                    out.push_back(t);
+                }
     // Winograd candidates for 3x3 / stride 1 convolutions with enough pixels to fill tile lanes
-    if (d.KH == 3 && d.KW == 3 && d.stride == 1 && d.dilation == 1 && tail_N == 0 && !std::getenv("TDC_EXPERIMENT_NO_WINOGRAD")) {
+    if (!wino_batch && d.KH == 3 && d.KW == 3 && d.stride == 1 && d.dilation == 1 && tail_N == 0 && !std::getenv("TDC_EXPERIMENT_NO_WINOGRAD")) {
         const int Wt = ceil_div(Wo, 2), Ht = ceil_div(Ho, 2);
         for (int wm : wms)
             for (int wn : wns)

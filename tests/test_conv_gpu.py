@@ -975,3 +975,39 @@ def test_blocked_1x1_with_images_far_apart():
         torch.cuda.synchronize()
         plan.close()
         assert_close(out.cpu().numpy(), ref.conv2d_c(x.numpy(), w.numpy()), f"{t}")
+
+
+@pytest.mark.parametrize("shape,pad", [((2, 13, 20, 9, 11), 1), ((5, 8, 16, 3, 4), 1), ((40, 7, 33, 3, 3), 1), ((3, 40, 24, 14, 14), 0),
+                                       ((2, 33, 17, 1, 9), 1), ((2, 65, 48, 8, 31), 1), ((4, 19, 40, 10, 3), 0), ((9, 4, 5, 4, 2), 1),
+                                       ((1, 20, 36, 60, 70), 1)])
+def test_every_batched_winograd_tile(shape, pad):
+    """The Winograd kernel that counts the 2x2 output tiles of the whole batch in one row (tile.alg = 1, tile.tw = 0), every
+    launchable tile: one step, two and several, a ragged last step, more teams than channel groups, odd and even sizes, images
+    of 8 pixels and of one row or two columns, 16 tiles of one wave in several images; plain, then bias + residual + ReLU with
+    input and output as channel slices that are only 4-byte aligned, NaN around the input slice and the residual in place."""
+    from ctypes import c_void_p
+    B, C, N, H, W = shape
+    x, w = case(8700 + C * N + H, B, C, N, H, W, 3)
+    g = seeded(8701)
+    bias = torch.randn(N, generator=g)
+    want = ref.conv2d_c(x.numpy(), w.numpy(), pad=pad)
+    Ho, Wo = want.shape[2], want.shape[3]
+    resid = torch.randn(B, N, Ho, Wo, generator=g)
+    want_full = ref.conv2d_c(x.numpy(), w.numpy(), bias.numpy(), resid.numpy(), pad=pad, relu=True)
+    tiles = [t for t in tdc_amd.model_enumerate(tdc_amd.conv_desc(B, C, N, H, W, 3, 3, 1, pad)) if t.alg == 1]
+    assert all(t.tw == 0 for t in tiles) and {(t.wn, t.wk) for t in tiles} >= {(4, 1), (2, 2), (2, 4)}
+    for t in tiles:
+        announce("batched winograd", shape, pad, t)
+        assert_close(run_conv(x, w, pad=pad, tile=t), want, f"{shape} pad {pad} {t}")
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, 3, 3, 1, pad, 1, True, True, tile=t).set_weights(w, bias)
+        xin = torch.full((B, C + 3, H, W), float("nan"), device="cuda"); xin[:, 1:1 + C] = x.cuda()
+        obuf = torch.full((B, N + 5, Ho, Wo), 7.0, device="cuda"); obuf[:, 4:4 + N] = resid.cuda()
+        o = c_void_p(obuf[:, 4:].data_ptr())
+        tdc_amd._lib.check(tdc_amd.lib().tdc_conv_forward_strided(
+            plan._h, c_void_p(xin[:, 1:].data_ptr()), (C + 3) * H * W, o, (N + 5) * Ho * Wo, o, (N + 5) * Ho * Wo,
+            c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        plan.close()
+        got = obuf.cpu()
+        assert_close(got[:, 4:4 + N].numpy(), want_full, f"slices {shape} pad {pad} {t}")
+        assert (got[:, :4] == 7.0).all() and (got[:, 4 + N:] == 7.0).all()
