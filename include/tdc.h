@@ -66,13 +66,15 @@ typedef struct tdc_conv_desc {
  * as many rows as fit in the workgroup's mf*nb*wn pixel lanes); its wm*wn*wk
  * computing wavefronts split output channels, pixels and input channels; input channels
  * are staged through LDS `cch` at a time, double-buffered (alg 0-2), or requested from
- * global memory into registers all at once (alg 3-6) or a run ahead (alg 7). */
+ * global memory into registers all at once (alg 3-6) or a run ahead (alg 7);
+ * alg 8 stages them as three bf16 parts each. */
 typedef struct tdc_tile {
     int32_t mf;   /* MFMA block edge: 32 (v_mfma_f32_32x32x2_f32) or 16 (16x16x4) */
-    int32_t mb;   /* MFMA blocks per wave along output channels (1 or 2)        */
+    int32_t mb;   /* MFMA blocks per wave along output channels (1 or 2; alg 8
+                     also 4)                                                     */
     int32_t nb;   /* MFMA blocks per wave along pixels (1 or 2; alg 4 and 6 also 4: the
                      workgroup's tile is nb 16-pixel blocks side by side along a row;
-                     alg 7: 2 or 4)                                              */
+                     alg 7: 2 or 4; alg 8: 4, with tw = 0 also 2)                */
     int32_t wm;   /* waves along output channels                               */
     int32_t wn;   /* waves along pixels                                        */
     int32_t wk;   /* waves along input channels (in-workgroup split-K)          */
@@ -123,6 +125,15 @@ typedef struct tdc_tile {
                          waves over channels and pixels, wk over input channels (at most 8 together; cch = C rounded up to
                          16 * wk); the pixels of all images in one row, so grid_x counts them and grid_z is 1; tw = 1,
                          ks = 1, wl = 0.  Carries the input affine, not a fused tail.
+                     8 = fp32 as three bf16 parts per operand and six products on v_mfma_f32_16x16x32_bf16, accumulated in fp32
+                         (the error against 64-bit sums is below that of the fp32 MFMAs; sums that come out NaN or under 2^-90,
+                         where the split does not hold, are computed again without it).  16 * mb channels x 16 * nb pixels per
+                         wave.  tw = 0: 1x1 / stride 1 / pad 0, the pixels of all images in one row of groups of nb, wk
+                         waves over input channels (mb 1 or 2, cch = 32 * wm * wk, at most 8 waves).  tw > 0: filters larger than
+                         1x1, any stride and dilation, nb = 4, wk = 1: tiles of tw columns and as many output rows, counted through the
+                         batch, as fit in 64 * wn pixels; cch = 8, 16 or 32 input channels per pass, or 4 (at most four
+                         input channels, even stride, dilation 1).  ks = 1, wl = 0.  The 1x1 form carries the input
+                         affine; no fused tail.
                      The model offers 3 to 6 where launch and latency dominate (few channels or few pixels); the
                      staged paths keep the layers whose operands are worth sharing through the LDS. */
 } tdc_tile;

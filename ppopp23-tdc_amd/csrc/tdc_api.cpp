@@ -377,6 +377,13 @@ static void refresh_launch_params(tdc_conv_plan *plan) {
     kp.fd_wk = make_fastdiv(plan->tile.wk);
     kp.fd_wn = make_fastdiv(plan->tile.wn);
     kp.fd_ks = make_fastdiv(g.ks);
+    if (plan->tile.alg == 8) {
+        kp.KS = d.stride;
+        kp.win_nreq = g.oct_shift; kp.win_ns = g.ksteps;
+        kp.fd_npx = make_fastdiv(std::max(g.nrows * g.ncols, 1));
+        kp.fd_hww = make_fastdiv(std::max(g.ncols, 1));
+        kp.fd_wtw = make_fastdiv(g.row_taps);
+    }
     kp.batch = d.batch;
     kp.units = g.units;
     kp.fd_units = make_fastdiv(std::max(g.units_image, 1));
@@ -689,7 +696,7 @@ static int forward_impl(tdc_conv_plan *plan, const float *d_in, int64_t in_batch
         const int per_wg = 16 * plan->tile.wn * (g.gen ? plan->tile.nb : 1);
         kp.batch = 1;
         kp.units = g.units_image;
-        kp.grid_x = (g.units_image + per_wg - 1) / per_wg;
+        kp.grid_x = plan->tile.alg == 8 ? g.ntx * ((g.units_image + g.units_wg - 1) / g.units_wg) : (g.units_image + per_wg - 1) / per_wg;
         kp.n_wg = kp.grid_x * kp.grid_y;
         kp.xcd_chunk = (kp.n_wg + 7) / 8;
         if (kp.channel_major) kp.fd_g1 = make_fastdiv(kp.grid_x);

@@ -67,7 +67,11 @@ struct Geometry {
     // tile.alg = 1 with tw = 0: its 2x2 output tiles likewise
     int units = 0, units_image = 0;
     int gen = 0;                     // single pixels
-    int unit_images = 0;             // images that the units of one wave reach past the first one's
+    int unit_images = 0;             // images that the units of one wave (tile.alg = 8: workgroup) reach past the first one's
+    // tile.alg = 8 (units are groups of nb pixels, or output rows): units per workgroup, octets of input channels per stage (as a
+    // power of two), K-steps per stage, taps (pairs
+    // of taps with at most four channels) per filter row.  win_L = window rows of one image, RS / CS = slots per row / octet.
+    int units_wg = 0, oct_shift = 0, ksteps = 0, row_taps = 1;
     int channel_major = 0;           // which logical workgroup order costs fewer L2 fills (see conv_staged.hip)
     double b_ways = 1.0;             // serialisation of the B-operand LDS read by bank conflicts (1 = none)
 };
@@ -178,8 +182,9 @@ enum : int { TAPS_GENERIC = 0, TAPS_1x1 = 1, TAPS_3x3 = 9, TAPS_3x3G = 10, TAPS_
 //   STREAM_WINO tdc_wino3x3_stream_kernel<CG, MAXW>                   p = {CG, MAXW}
 //   BLOCK_WINO  tdc_wino3x3_block_kernel<MB, WN>                      p = {MB, WN}
 //   BLOCK_1x1   tdc_conv1x1_block_kernel<MB, NJ, AFF, GEN>            p = {MB, NJ, AFF, GEN}
+//   SPLIT       tdc_conv_split_kernel<MB, NB, MODE, AFF>              p = {MB, NB, MODE, AFF}   (MODE: 0 flat, 1 window, 2 few channels)
 struct KernelId {
-    enum Family : int { NONE = 0, STAGED = 1, STREAM_1x1 = 2, STREAM_3x3 = 3, STREAM_WINO = 4, BLOCK_1x1 = 5, BLOCK_WINO = 6 };
+    enum Family : int { NONE = 0, STAGED = 1, STREAM_1x1 = 2, STREAM_3x3 = 3, STREAM_WINO = 4, BLOCK_1x1 = 5, BLOCK_WINO = 6, SPLIT = 7 };
     int family = NONE;
     int p[6] = {0, 0, 0, 0, 0, 0};
 };
@@ -199,12 +204,13 @@ int kernel_vgprs(const KernelId &k);
 int kernel_waves_per_simd(const KernelId &k);
 // The function itself (nullptr if not instantiated).
 const void *kernel_function(const KernelId &k);
-// (its parts, one per translation unit that holds kernels: conv_staged.hip, conv_stream.hip, conv_wino_stream.hip, conv_block.hip, conv_wino_block.hip)
+// (its parts, one per translation unit that holds kernels: conv_staged.hip, conv_stream.hip, conv_wino_stream.hip, conv_block.hip, conv_wino_block.hip, conv_split.hip)
 const void *staged_kernel_function(const KernelId &k);
 const void *stream_kernel_function(const KernelId &k);
 const void *wino_stream_kernel_function(const KernelId &k);
 const void *block_kernel_function(const KernelId &k);
 const void *wino_block_kernel_function(const KernelId &k);
+const void *split_kernel_function(const KernelId &k);
 inline const void *conv_kernel_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras, bool single_pixels) {
     return kernel_function(kernel_id_for(t, KH, KW, dilation, stride, extras, single_pixels));
 }

@@ -108,12 +108,133 @@ static int pad_channel_stride(int raw, int mf, int vw, int PT, int TW, int TH, i
     return hit->second.first;
 }
 
+// Which logical workgroup order costs fewer L2 fills.  Bytes the eight die-private L2s fill in total, for the two orders: with
+// the channel tiles of a pixel tile adjacent a die reads its share of the input and every weight; with the pixel tiles of a
+// channel tile adjacent it reads every input pixel of min(channel tiles, 8) ... and its own weights.
+static int channel_major_order(double in_bytes, double w_bytes, long long n_wg, int grid_y) {
+    const double dies = (double)std::min<long long>(8, n_wg);
+    const double pixel_major = in_bytes + dies * w_bytes;
+    const double channel_major = std::min<double>(grid_y, dies) * in_bytes + std::max(1.0, dies / grid_y) * w_bytes;
+    if (const char *e = std::getenv("TDC_EXPERIMENT_XCD_ORDER")) return std::atoi(e) != 0;
+    return channel_major < pixel_major ? 1 : 0;
+}
+
+// tile.alg = 8: fp32 operands as three bf16 parts each (conv_split.hip).
+static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::string *why, int tail_N) {
+    auto fail = [&](const char *m) {
+        if (why) *why = m;
+        return false;
+    };
+    const bool flat = t.tw == 0, few = t.cch == 4, one = d.KH == 1 && d.KW == 1;
+    if (t.mf != 16 || (t.nb != 4 && !(t.nb == 2 && flat)) || (t.mb != 1 && t.mb != 2 && t.mb != 4))
+        return fail("tile.alg = 8 needs mf = 16, mb = 1, 2 or 4, nb = 4 (with tw = 0 also 2)");
+    if (t.wm < 1 || t.wn < 1 || t.wk < 1 || (long long)t.wm * t.wn * t.wk > 8) return fail("tile.alg = 8 needs 1 to 8 waves");
+    if ((t.wk != 1 && !flat) || t.ks != 1 || t.wl != 0)
+        return fail("tile.alg = 8 has no split across workgroups and no loader waves, and splits input channels over waves only with tw = 0");
+    if (tail_N > 0) return fail("tile.alg = 8 cannot carry a fused tail");
+    g = Geometry();
+    g.Ho = (d.H + 2 * d.pad - d.dilation * (d.KH - 1) - 1) / d.stride + 1;
+    g.Wo = (d.W + 2 * d.pad - d.dilation * (d.KW - 1) - 1) / d.stride + 1;
+    g.P = g.Ho * g.Wo;
+    g.He = d.H;
+    g.We = d.W;
+    g.kc = 32;
+    g.taps = g.ktaps = d.KH * d.KW;
+    g.max_waves_kernel = 8;
+    g.waves = t.wm * t.wn * t.wk;
+    g.threads = 64 * g.waves;
+    g.MT = 16 * t.mb * t.wm;
+    g.PT = 16 * t.nb * t.wn;
+    g.cpw = t.cch / t.wk;
+    g.nchunks = ceil_div(d.C, t.cch);
+    g.cps = g.nchunks;
+    g.c_pad = g.nchunks * t.cch;
+    long long lds, units;
+    int cols = 1;
+    if (flat) {
+        if (!one || d.stride != 1 || d.pad != 0) return fail("tile.alg = 8 with tw = 0 needs a 1x1 / stride 1 / pad 0 convolution");
+        if (g.P < t.nb) return fail("tile.alg = 8 with tw = 0 needs images of at least nb pixels");
+        const int kw = t.wm * t.wk;             // K-steps of a stage: every thread of the workgroup loads one octet
+        if (kw != 1 && kw != 2 && kw != 4 && kw != 8) return fail("tile.alg = 8 with tw = 0 needs wm * wk = 1, 2, 4 or 8");
+        if (t.mb > 2) return fail("tile.alg = 8 with tw = 0 needs mb = 1 or 2");
+        if (4 * t.mb % t.wk != 0) return fail("tile.alg = 8: more channel slices than rows to finish");
+        if (t.cch != 32 * kw) return fail("tile.alg = 8 with tw = 0 needs cch = 32 * wm * wk");
+        g.units_image = ceil_div(g.P, t.nb);
+        units = (long long)d.batch * g.units_image;
+        g.units_wg = 16 * t.wn;
+        g.unit_images = std::min(d.batch - 1, (g.units_wg - 2) / g.units_image + 1);
+        g.TW = std::min(g.PT, g.P);
+        g.TH = 1;
+        while ((1 << g.oct_shift) < 4 * kw) ++g.oct_shift;
+        g.ksteps = kw;
+        g.RS = 1;
+        g.CS = g.PT;
+        g.win_L = 1;
+        lds = std::max(3LL * (4 * kw) * g.CS * 16, 1024LL * g.waves * t.mb * t.nb);   // the staged octets, or the sums of all waves
+    } else {
+        if (few) {
+            if (d.C > 4 || d.dilation != 1 || d.stride % 2 != 0)
+                return fail("tile.alg = 8 with cch = 4 needs at most four input channels, an even stride and dilation 1");
+        } else if (t.cch != 8 && t.cch != 16 && t.cch != 32) {
+            return fail("tile.alg = 8 needs cch = 8, 16 or 32 (4: at most four input channels)");
+        }
+        if (one) return fail("tile.alg = 8 takes 1x1 convolutions with tw = 0 only");
+        if (t.tw < 1 || t.tw > g.PT || t.tw > g.Wo) return fail("tile.alg = 8: tile.tw does not fit");
+        units = (long long)d.batch * g.Ho;
+        g.TW = t.tw;
+        g.TH = (int)std::min<long long>(g.PT / t.tw, units);
+        g.units_image = g.Ho;
+        g.units_wg = g.TH;
+        while ((8 << g.oct_shift) < t.cch) ++g.oct_shift;
+        g.row_taps = few ? ceil_div(d.KW, 2) : d.KW;
+        g.ksteps = few ? ceil_div(d.KH * g.row_taps, 4) : ceil_div(g.taps << g.oct_shift, 4);
+        const long long columns = (long long)(g.TW - 1) * d.stride + (few ? 2 * g.row_taps : (d.KW - 1) * d.dilation + 1);
+        const long long image_rows = (long long)(g.Ho - 1) * d.stride + (long long)(d.KH - 1) * d.dilation + 1;
+        // the most window rows any tile of output rows needs (the tiles repeat their place in the images after Ho of them)
+        long long rows = 0;
+        const long long tiles = (units + g.TH - 1) / g.TH;
+        for (long long i = 0; i < std::min<long long>(tiles, g.Ho); ++i) {
+            const long long a = i * g.TH, b = std::min(a + g.TH, units) - 1;
+            rows = std::max(rows, (b / g.Ho - a / g.Ho) * image_rows + (b % g.Ho - a % g.Ho) * d.stride + (long long)(d.KH - 1) * d.dilation + 1);
+            g.unit_images = std::max(g.unit_images, (int)(b / g.Ho - a / g.Ho));
+        }
+        g.unit_images = std::min(d.batch - 1, g.unit_images + 1);   // (the last rows of a window may lie in an image that no output needs)
+        if (columns > 8192 || rows > 8192 || rows * columns > 65536 || image_rows + rows > 65535) return fail("tile.alg = 8: input window too large");
+        g.ncols = (int)columns;
+        g.nrows = (int)rows;
+        g.win_L = (int)image_rows;
+        g.win_off = (g.ncols + 1) / 2;
+        g.RS = !few && d.stride == 2 ? 2 * g.win_off : g.ncols;
+        g.CS = g.nrows * g.RS;
+        lds = few ? 3LL * g.CS * 8 : (3LL * g.CS * 16) << g.oct_shift;
+        cols = ceil_div(g.Wo, g.TW);
+    }
+    if (units * std::max(g.units_image, 16) >= (1LL << 32) || units >= (1LL << 30)) return fail("batch too large for tile.alg = 8");
+    if ((long long)d.H * d.W * (g.c_pad + 8) * 4 >= (1LL << 31)) return fail("image too large for tile.alg = 8");
+    if (lds > machine().lds_bytes_per_cu) return fail("tile needs more than 160 KiB of LDS");
+    g.units = (int)units;
+    g.lds_bytes = (int)lds;
+    g.ntx = cols;
+    g.nty = (int)((units + g.units_wg - 1) / g.units_wg);
+    g.grid_y = ceil_div(d.N, g.MT);
+    g.grid_z = 1;
+    const long long gx = (long long)g.ntx * g.nty, n_wg = gx * g.grid_y;
+    if (gx * g.ntx >= (1LL << 32) || n_wg + 8 >= (1LL << 28) || n_wg * std::max<long long>(gx, g.grid_y) >= (1LL << 32) || g.grid_y > 65535)
+        return fail("grid too large");
+    g.grid_x = (int)gx;
+    g.wslab_floats = t.wm * t.mb * g.ksteps * 3 * 256;
+    if ((long long)g.grid_y * g.nchunks * g.wslab_floats * 4 >= (1LL << 31)) return fail("packed weights exceed 2 GiB");
+    g.channel_major = channel_major_order(4.0 * d.batch * d.C * d.H * d.W, 6.0 * d.N * d.C * g.taps, n_wg, g.grid_y);
+    return true;
+}
+
 bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::string *why, int tail_N) {
     auto fail = [&](const std::string &m) {
         if (why) *why = m;
         return false;
     };
     if (!check_desc(d, why)) return false;
+    if (t.alg == 8) return make_split_geometry(d, t, g, why, tail_N);
     if (t.mf != 32 && t.mf != 16) return fail("tile.mf must be 16 or 32");
     if (t.mb < 1 || t.mb > 2 || t.nb < 1 ||
         (t.nb > 2 && !((t.alg == 4 || t.alg == 6 || t.alg == 7) && t.nb == 4)))
@@ -145,7 +266,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     g.taps = d.KH * d.KW;
     g.ktaps = g.taps;
     g.MT = t.mf * t.mb * t.wm;
-    if (t.alg < 0 || t.alg > 7) return fail("tile.alg must be in [0, 7]");
+    if (t.alg < 0 || t.alg > 7) return fail("tile.alg must be in [0, 8]");
     if (t.alg == 5) {
         // Winograd F(2x2,3x3) streamed from global memory: 16*wm channels of one tile row block (2 rows x 28 columns) per
         // workgroup, the input channels split over wk waves in groups of four, everything in one pass
@@ -385,15 +506,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     // (the kernel decodes a one-dimensional launch index with 32-bit multiply-high divisions)
     const long long n_wg = (long long)g.grid_x * g.grid_y * g.grid_z;
     if (n_wg + 8 >= (1LL << 28) || n_wg * std::max(g.grid_x, g.grid_y) >= (1LL << 32)) return fail("grid too large");
-    // Bytes the eight die-private L2s fill in total, for the two logical workgroup orders: with the channel
-    // tiles of a pixel tile adjacent a die reads its share of the input and every weight; with the pixel tiles
-    // of a channel tile adjacent it reads every input pixel of min(channel tiles, 8) ... and its own weights.
-    const double in_bytes = 4.0 * d.C * d.H * d.W * (flat_batch ? d.batch : 1), w_bytes = 4.0 * d.N * d.C * g.taps;
-    const double dies = (double)std::min<long long>(8, n_wg);
-    const double pixel_major = in_bytes + dies * w_bytes;
-    const double channel_major = std::min<double>(g.grid_y, dies) * in_bytes + std::max(1.0, dies / g.grid_y) * w_bytes;
-    g.channel_major = channel_major < pixel_major ? 1 : 0;
-    if (const char *e = std::getenv("TDC_EXPERIMENT_XCD_ORDER")) g.channel_major = std::atoi(e) != 0;
+    g.channel_major = channel_major_order(4.0 * d.C * d.H * d.W * (flat_batch ? d.batch : 1), 4.0 * d.N * d.C * g.taps, n_wg, g.grid_y);
     return true;
 }
 
@@ -401,11 +514,63 @@ size_t packed_weight_floats(const Geometry &g) {
     return (size_t)g.grid_y * (size_t)g.nchunks * (size_t)g.wslab_floats;
 }
 
+static uint16_t to_bf16(float v) {   // nearest even; a finite value never becomes infinite
+    uint32_t u;
+    std::memcpy(&u, &v, 4);
+    if ((u & 0x7f800000u) == 0x7f800000u) return (uint16_t)((u >> 16) | ((u & 0xffffu) ? 0x40u : 0u));
+    const uint32_t r = u + 0x7fffu + ((u >> 16) & 1u);
+    return (uint16_t)(((r & 0x7f800000u) == 0x7f800000u ? u : r) >> 16);
+}
+static float from_bf16(uint16_t h) {
+    const uint32_t u = (uint32_t)h << 16;
+    float v;
+    std::memcpy(&v, &u, 4);
+    return v;
+}
+
+// tile.alg = 8: per (16 channels, pass, K-step, part): [lane][8], lane (n = l % 16, k = l / 16) holding part 0, 1 or 2 of the
+// weights of channel block*16 + n and K octet 4*step + k.  An octet is eight input channels of one tap, or (cch = 4) four
+// channels of two neighbouring taps of a filter row.
+static void pack_split_weights(const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, const float *w, float *packed) {
+    uint16_t *const dst = reinterpret_cast<uint16_t *>(packed);
+    const bool few = t.tw != 0 && t.cch == 4;
+    const int octets = t.cch / 8, blocks = g.grid_y * t.wm * t.mb;
+    size_t base = 0;
+    for (int blk = 0; blk < blocks; ++blk)
+        for (int pass = 0; pass < g.nchunks; ++pass)
+            for (int ks = 0; ks < g.ksteps; ++ks, base += 3 * 512)
+                for (int l = 0; l < 64; ++l)
+                    for (int e = 0; e < 8; ++e) {
+                        const int idx = 4 * ks + l / 16, n = blk * 16 + l % 16;
+                        int c, ky, kx;
+                        if (few) {
+                            c = e & 3;
+                            ky = idx / g.row_taps;
+                            kx = 2 * (idx % g.row_taps) + (e >> 2);
+                        } else {
+                            const int tap = idx / octets;
+                            c = pass * t.cch + 8 * (idx % octets) + e;
+                            ky = tap / d.KW;
+                            kx = tap % d.KW;
+                        }
+                        float v = (n < d.N && c < d.C && ky < d.KH && kx < d.KW) ? w[(((size_t)n * d.C + c) * d.KH + ky) * d.KW + kx] : 0.0f;
+                        for (int s = 0; s < 3; ++s) {
+                            const uint16_t h = to_bf16(v);
+                            dst[base + (size_t)s * 512 + l * 8 + e] = h;
+                            v = std::isfinite(v) ? v - from_bf16(h) : 0.0f;
+                        }
+                    }
+}
+
 void pack_weights(const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, const float *w, float *packed) {
     const int mbw = t.wm * t.mb;
     const int ncg = t.cch / g.kc;
     const int taps = g.taps;
     float *dst = packed;
+    if (t.alg == 8) {
+        pack_split_weights(d, t, g, w, packed);
+        return;
+    }
     if (t.alg == 2 || t.alg == 4 || t.alg == 6) {
         // per (channel tile, pass, M block, channel group): [taps 0-3][lane][4] [taps 4-7][lane][4] [tap 8][lane]
         for (int by = 0; by < g.grid_y; ++by)
@@ -584,6 +749,17 @@ int wino_stream_max_waves(int groups) { return (groups >= 1 && groups <= 4) ? 16
 
 KernelId kernel_id_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras, bool single_pixels) {
     KernelId k;
+    if (t.alg == 8) {
+        if (t.mf != 16 || (t.nb != 2 && t.nb != 4) || (t.mb != 1 && t.mb != 2 && t.mb != 4)) return k;
+        // (`extras` here can only mean the input affine of a 1x1 convolution)
+        const int mode = t.tw == 0 ? 0 : t.cch == 4 ? 2 : 1;
+        if (mode == 0 ? t.mb > 2 : t.nb != 4) return k;
+        if ((mode == 0) != (KH == 1 && KW == 1)) return k;
+        if ((mode != 0 && extras) || (mode == 2 && dilation != 1)) return k;
+        k.family = KernelId::SPLIT;
+        k.p[0] = t.mb; k.p[1] = t.nb; k.p[2] = mode; k.p[3] = extras;
+        return k;
+    }
     if (t.alg == 1 && t.tw == 0) {
         if (extras || KH != 3 || KW != 3 || dilation != 1 || stride != 1 || t.mf != 16 || t.wm != 1 || (t.wn != 2 && t.wn != 4) ||
             (t.mb != 1 && t.mb != 2) || t.nb != 1)
@@ -686,6 +862,9 @@ std::string kernel_name(const KernelId &k) {
             break;
         case KernelId::BLOCK_1x1:
             std::snprintf(buf, sizeof buf, "tdc_conv1x1_block_kernel<%d, %d, %s, %s>", k.p[0], k.p[1], tf[k.p[2] != 0], tf[k.p[3] != 0]);
+            break;
+        case KernelId::SPLIT:
+            std::snprintf(buf, sizeof buf, "tdc_conv_split_kernel<%d, %d, %d, %s>", k.p[0], k.p[1], k.p[2], tf[k.p[3] != 0]);
             break;
         default: return "";
     }
@@ -913,6 +1092,36 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
         info.pred_l2_bytes = 0.0;
         return true;
     }
+    if (t.alg == 8) {
+        // Split operands on the bf16 matrix pipe: the largest of what the matrix pipes, a workgroup's own chain of stages and
+        // the L2 need, + LDS reads + the end of every workgroup + launch and memory traffic.  Fitted to 4500 timed tiles of 90
+        // 1x1 shapes (6 % mean error, 2.2 % mean loss of the pick within the family) and 4100 tiles of 60 3x3 and 7x7 shapes
+        // (6 %, 2.5 %).  The factor in front of the 1x1 and 3x3 forms: as measured, the formulas of the other families are 15 to
+        // 25 % kind to the launches this one competes with (7 us and more), those for the 7x7 stems are not.  At 0.91 no 1x1
+        // shape of the 90 loses more than 2 % to its former pick and the mean gain is 9 % (0.85: 10 %, but three lose 8 to 12 %;
+        // 1.0: 6 %); the lines fall at 7 to 9 us from 64 channels up, and about 25 us at 3x3 / stride 2.
+        const bool flat = t.tw == 0;
+        const double wgs = (double)n_wg / m.cus, load = 0.5 * (std::ceil(wgs) + std::max(wgs, 1.0)), rounds = std::ceil(wgs / wg_per_cu);
+        const double simd = std::max(1.0, (double)g.waves / m.simds_per_cu), epi = load * g.waves * t.mb * t.nb;
+        const double mfmas = (double)g.nchunks * g.ksteps / t.wk * t.mb * t.nb * 6.0 * 16.0;
+        const double lds_reads = load * g.waves * g.nchunks * t.nb * 3.0 * 8.0;
+        const double traffic = 4.0 * (d.batch * ((double)d.C * d.H * d.W + (double)d.N * P)) + 6.0 * d.C * d.N * g.taps;
+        if (flat) {
+            const double l2 = (double)n_wg * g.nchunks * (g.waves * t.wm * t.mb * 3072.0 + (double)t.cch * g.PT * 4.0) / std::min<double>(m.cus, (double)n_wg) / 105.9;
+            double clk = std::max(std::max(0.807 * load * simd * mfmas, rounds * (1859.0 * g.nchunks + mfmas)), l2);
+            clk += 1.443 * lds_reads * (t.wm + 1) + 92.1 * epi;
+            if (t.wk > 1) clk += 815.0 + 5.6 * epi;
+            info.pred_us = 0.91 * (2.859 + clk / (m.clock_ghz * 1e3) + traffic / 17.67e6);
+        } else {
+            const bool few = t.cch == 4;
+            const double staged = g.nchunks * std::ceil((double)(g.CS << g.oct_shift) / g.threads) * (few ? 0.5 : 1.0);
+            double clk = std::max(load * simd * (0.906 * mfmas + 757.0 * staged), rounds * (3232.0 * g.nchunks + 912.0 * staged + 1.164 * mfmas));
+            clk += 1.293 * lds_reads * g.ksteps + 181.5 * epi;
+            info.pred_us = (few ? 1.0 : 0.85) * (3.527 + clk / (m.clock_ghz * 1e3) + traffic / 15.3e6);
+        }
+        info.pred_l2_bytes = 0.0;
+        return true;
+    }
     if (t.alg == 7) {
         // Register-blocked 1x1: the whole launch at once, the largest of what the matrix pipes, a wave's own chain of runs,
         // the address paths and the L2 need, + launch and first operands, + a share of the memory traffic that does not
@@ -974,6 +1183,34 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
                 out.push_back(t);
             }
         }
+    }
+    // split-operand candidates (bf16 matrix pipe); below 0.1 and 0.3 GFLOP (1x1, larger filters) they never came within 10 % of the
+    // other families, which have the shorter start
+    const bool one = d.KH == 1 && d.KW == 1;
+    const double flops = 2.0 * d.batch * P * d.C * d.N * d.KH * d.KW;
+    if (tail_N == 0 && flops >= (one ? 1e8 : 3e8) && !(one && (d.stride != 1 || d.pad != 0)) && !std::getenv("TDC_EXPERIMENT_NO_SPLIT")) {
+        const bool few = d.C <= 4 && d.dilation == 1 && d.stride % 2 == 0;
+        auto offer = [&](const tdc_tile &t) {
+            Geometry g;
+            if (make_geometry(d, t, g, nullptr, 0)) out.push_back(t);
+        };
+        std::vector<int> tws;
+        for (int tw : {Wo, ceil_div(Wo, 2), ceil_div(Wo, 4), 8, 16, 32, 64})
+            if (tw <= Wo && std::find(tws.begin(), tws.end(), tw) == tws.end()) tws.push_back(tw);
+        for (int mb : {1, 2, 4})
+            for (int wm : {1, 2, 4, 8})
+                for (int wn : {1, 2, 4, 8}) {
+                    if (wm * wn > 8 || 16 * mb * wm > round_up(d.N, 16 * mb)) continue;
+                    if (one) {
+                        for (int nb : {2, 4})
+                            for (int wk : {1, 2, 4, 8})
+                                if (mb <= 2 && (wm * wn * wk == 4 || wm * wn * wk == 8)) offer({16, mb, nb, wm, wn, wk, 32 * wm * wk, 0, 1, 0, 8});
+                    } else if (wm * wn >= 4) {
+                        for (int tw : tws)
+                            for (int cch : {4, 8, 16, 32})
+                                if ((cch == 4) == few && cch < 2 * d.C + 8) offer({16, mb, 4, wm, wn, 1, cch, tw, 1, 0, 8});
+                    }
+                }
     }
     // register-blocked 1x1 candidates
     if (d.KH == 1 && d.KW == 1 && d.pad == 0 && tail_N == 0 && !std::getenv("TDC_EXPERIMENT_NO_BLOCKED_1X1")) {
@@ -1182,6 +1419,8 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
                                         }
                         }
     }
+    // (the other families' addressing limits hold for the library as a whole: a shape that none of them takes is refused)
+    if (std::all_of(out.begin(), out.end(), [](const tdc_tile &t) { return t.alg == 8; })) out.clear();
     return out;
 }
 

@@ -1011,3 +1011,134 @@ def test_every_batched_winograd_tile(shape, pad):
         got = obuf.cpu()
         assert_close(got[:, 4:4 + N].numpy(), want_full, f"slices {shape} pad {pad} {t}")
         assert (got[:, :4] == 7.0).all() and (got[:, 4 + N:] == 7.0).all()
+
+
+def split_tiles(B, C, N, H, W, K, stride, pad, dil=1):
+    """Every launchable tile of the split-operand kernel (tile.alg = 8), also those the model does not offer at this size."""
+    d = tdc_amd.conv_desc(B, C, N, H, W, K, K, stride, pad, dil)
+    Wo = (W + 2 * pad - dil * (K - 1) - 1) // stride + 1
+    out = []
+    for mb in (1, 2, 4):
+        for wm, wn, wk in ((1, 4, 1), (2, 2, 1), (4, 1, 1), (8, 1, 1), (1, 1, 4), (2, 1, 2), (1, 2, 2), (1, 1, 8), (1, 1, 1), (1, 8, 1)):
+            for nb in (2, 4):
+                for tw in ((0,) if K == 1 else sorted({Wo, -(-Wo // 2), min(Wo, 8)})):
+                    for cch in ((32 * wm * wk,) if K == 1 else (4, 8, 16, 32)):
+                        t = tdc_amd.Tile(16, mb, nb, wm, wn, wk, cch, tw, 1, 0, 8)
+                        try:
+                            tdc_amd.model_evaluate(d, t)
+                        except tdc_amd.TdcError:
+                            continue
+                        out.append(t)
+    return out
+
+
+def run_slices(plan, x, resid, N, Ho, Wo):
+    """Input, residual and output as channel slices that are only 4-byte aligned, the residual in place."""
+    from ctypes import c_void_p
+    B, C, H, W = x.shape
+    xin = torch.full((B, C + 3, H, W), float("nan"), device="cuda"); xin[:, 1:1 + C] = x.cuda()
+    obuf = torch.full((B, N + 5, Ho, Wo), 7.0, device="cuda"); obuf[:, 4:4 + N] = resid.cuda()
+    o = c_void_p(obuf[:, 4:].data_ptr())
+    tdc_amd._lib.check(tdc_amd.lib().tdc_conv_forward_strided(
+        plan._h, c_void_p(xin[:, 1:].data_ptr()), (C + 3) * H * W, o, (N + 5) * Ho * Wo, o, (N + 5) * Ho * Wo,
+        c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    got = obuf.cpu()
+    assert (got[:, :4] == 7.0).all() and (got[:, 4 + N:] == 7.0).all()
+    return got[:, 4:4 + N].numpy()
+
+
+@pytest.mark.parametrize("shape,K,stride,pad,dil", [
+    ((3, 20, 24, 7, 5), 1, 1, 0, 1), ((2, 33, 40, 9, 9), 1, 1, 0, 1), ((5, 300, 70, 7, 7), 1, 1, 0, 1), ((9, 64, 130, 2, 2), 1, 1, 0, 1),
+    ((3, 70, 17, 1, 3), 1, 1, 0, 1), ((2, 260, 64, 12, 11), 1, 1, 0, 1), ((3, 16, 20, 7, 7), 3, 1, 1, 1), ((2, 40, 36, 13, 9), 3, 2, 1, 1),
+    ((7, 9, 70, 5, 6), 3, 1, 1, 1), ((2, 24, 33, 11, 12), 3, 3, 0, 1), ((2, 17, 16, 10, 11), 5, 2, 2, 1), ((2, 20, 18, 12, 13), 3, 2, 2, 2),
+    ((2, 3, 64, 23, 21), 7, 2, 3, 1), ((3, 4, 18, 15, 17), 3, 2, 1, 1), ((2, 1, 30, 20, 17), 4, 2, 1, 1)])
+def test_every_split_tile(shape, K, stride, pad, dil):
+    """The split-operand path (tile.alg = 8), every launchable tile: pixel groups that end inside an image and images of fewer
+    pixels than a wave's, several images per workgroup, ragged channels and stages, tiles of rows that cross images, strides
+    (even and odd columns apart at 2), dilation, few input channels with odd and even filters; plain, then bias + residual +
+    ReLU on channel slices, for 1x1 then the input affine.  The error against 64-bit sums is bounded by 4e-7 of the norm, the
+    level of one chain of fp32 MFMAs at K = 512 (measured: 3.9e-8 ... 7e-8), beside the usual tolerance per element."""
+    B, C, N, H, W = shape
+    x, w = case(8700 + C + N + H, B, C, N, H, W, K)
+    g = seeded(8701)
+    bias = torch.randn(N, generator=g)
+    want = ref.conv2d_c(x.numpy(), w.numpy(), stride=stride, pad=pad, dil=dil)
+    exact = torch.nn.functional.conv2d(x.double(), w.double(), None, stride, pad, dil)
+    Ho, Wo = want.shape[2], want.shape[3]
+    resid = torch.randn(B, N, Ho, Wo, generator=g)
+    want_full = ref.conv2d_c(x.numpy(), w.numpy(), bias.numpy(), resid.numpy(), stride=stride, pad=pad, dil=dil, relu=True)
+    tiles = split_tiles(B, C, N, H, W, K, stride, pad, dil)
+    assert tiles
+    if K == 1:
+        scale, shift = torch.rand(C, generator=g) * 2 - 0.5, torch.randn(C, generator=g) * 0.3
+        xt = (x * scale.view(1, C, 1, 1) + shift.view(1, C, 1, 1)).clamp_min(0)
+        want_aff = ref.conv2d_c(xt.numpy(), w.numpy(), bias.numpy(), relu=True)
+    for t in tiles:
+        announce("split", shape, K, stride, pad, dil, t)
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, K, K, stride, pad, dil, tile=t).set_weights(w)
+        out = torch.full((B, N, Ho, Wo), float("nan"), device="cuda")
+        plan.forward(x.cuda(), out=out)
+        torch.cuda.synchronize()
+        plan.close()
+        assert_close(out.cpu().numpy(), want, f"{shape} {t}")
+        assert (out.cpu().double() - exact).norm() <= 4e-7 * exact.norm(), f"{shape} {t}"
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, K, K, stride, pad, dil, True, True, tile=t).set_weights(w, bias)
+        assert_close(run_slices(plan, x, resid, N, Ho, Wo), want_full, f"slices {shape} {t}")
+        if K == 1:
+            plan.set_input_affine(scale, shift, relu=True)
+            got = plan.forward(x.cuda()).cpu().numpy()
+            assert_close(got, want_aff, f"input affine {shape} {t}")
+        plan.close()
+
+
+@pytest.mark.parametrize("shape,K,stride,pad", [((2, 40, 36, 8, 8), 1, 1, 0), ((2, 70, 20, 7, 7), 1, 1, 0), ((2, 40, 36, 9, 9), 3, 2, 1),
+                                                ((2, 3, 20, 12, 12), 7, 2, 3)])
+def test_split_tiles_with_special_values(shape, K, stride, pad):
+    """Infinities, NaN and values that round to a bf16 infinity, in the input and in the weights, come out as fp32 sums of the
+    unsplit operands give them; so do inputs near the smallest normal numbers, whose lower parts bf16 cannot hold."""
+    B, C, N, H, W = shape
+    g = seeded(8750)
+    x, w = torch.rand(B, C, H, W, generator=g) + 0.1, torch.rand(N, C, K, K, generator=g) + 0.1
+    w[3] = -w[3]
+    w[5, 1, 0, 0] = float("inf")
+    x[0, 1, 2, 3], x[0, 2, 5, 5], x[1, 0, 4, 4], x[1, 1, 6, 6] = float("inf"), -float("inf"), float("nan"), 3.4e38
+    resid, bias = torch.rand(B, N, (H + 2 * pad - K) // stride + 1, (W + 2 * pad - K) // stride + 1, generator=g), torch.rand(N, generator=g)
+    want = (torch.nn.functional.conv2d(x.double(), w.double(), bias.double(), stride, pad) + resid).float()
+    assert torch.isinf(want).any() and torch.isnan(want).any() and torch.isfinite(want).any()
+    tiny, tiny_w = (torch.rand(B, C, H, W, generator=g) + 0.5) * 1e-35, torch.rand(N, C, K, K, generator=g) + 0.5
+    want_tiny = torch.nn.functional.conv2d(tiny.double(), tiny_w.double(), None, stride, pad)
+    for t in split_tiles(B, C, N, H, W, K, stride, pad):
+        announce("split special values", shape, K, t)
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, K, K, stride, pad, 1, True, tile=t).set_weights(w, bias)
+        got = plan.forward(x.cuda(), resid.cuda()).cpu()
+        plan.close()
+        assert torch.allclose(got, want, rtol=1e-5, atol=1e-5, equal_nan=True), f"{shape} {t}"
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, K, K, stride, pad, tile=t).set_weights(tiny_w)
+        got = plan.forward(tiny.cuda()).cpu().double()
+        plan.close()
+        # (positive fp32 sums of at most 360 products, a rounding of 2^-24 each: 2.2e-5)
+        assert ((got - want_tiny).abs() <= 2.2e-5 * want_tiny.abs()).all(), f"tiny {shape} {t}"
+
+
+@pytest.mark.parametrize("K,stride,C", [(1, 1, 20), (3, 2, 20), (3, 2, 3)])
+def test_split_tiles_with_images_far_apart(K, stride, C):
+    """tile.alg = 8 reaches the images of one workgroup through 32-bit offsets; images 2 GiB apart are launched one by one."""
+    from ctypes import c_void_p
+    B, N, H, W, pad = 3, 24, 3, 5, K // 2
+    x, w = case(8760, B, C, N, H, W, K)
+    want = ref.conv2d_c(x.numpy(), w.numpy(), stride=stride, pad=pad)
+    far = 1 << 29
+    buf = torch.empty(2 * far + C * H * W, device="cuda")
+    for b in range(B):
+        buf[b * far:b * far + C * H * W] = x[b].reshape(-1).cuda()
+    for t in split_tiles(B, C, N, H, W, K, stride, pad):
+        announce("split far apart", K, C, t)
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, K, K, stride, pad, tile=t).set_weights(w)
+        out = torch.full(want.shape, float("nan"), device="cuda")
+        tdc_amd._lib.check(tdc_amd.lib().tdc_conv_forward_strided(
+            plan._h, c_void_p(buf.data_ptr()), far, None, 0, c_void_p(out.data_ptr()), 0,
+            c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        plan.close()
+        assert_close(out.cpu().numpy(), want, f"{t}")
