@@ -62,7 +62,8 @@ static __device__ __forceinline__ bool suspect(float sum) { return !(fabsf(sum) 
 //   SPLIT_FEW     at most four input channels (RGB stems): 8 bytes per pixel, a K octet is a pair of neighbouring taps.
 // Infinite and NaN operands (and finite ones above 3.39e38) make the split invalid: an infinity less itself is NaN.  Operands
 // below 2^-110 lose their last bits, because bf16 has no subnormals under 2^-133.  A wave that finds a NaN among its sums, or
-// one under 2^-90 other than zero, computes its outputs again, one by one, in fp32 from the unsplit input.
+// one under 2^-90 other than zero, computes its outputs again, one by one, in fp32 from the unsplit input.  Channels of very small
+// or very large weights are packed times a power of two (pack_split_weights) and their sums multiplied by p.w_scale.
 // AFF: per-channel affine (+ ReLU) on the input of a 1x1 convolution.
 // Bound: no single one.  512 -> 128 @28 batch 32 takes 26 us: 9 us of MFMAs at the 390 TFLOP/s of fp32 products that a bare MFMA
 // loop reaches, 13 us of memory traffic, and between them LDS reads (a half of the MFMA time at mb = 2), the splitting (6
@@ -252,6 +253,9 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
         for (int j = 0; j < NB; ++j) lead[m][j] = rest[m][j] = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
     const int steps_all = p.nchunks * ksteps;
+    // (requested here and looked at behind the last stage.  Read from memory and not passed: new weights may come under a captured graph)
+    const float scaled_flag = *p.w_scale;
+    const float *const w_scale = p.w_scale + 4;
     const int mblk0 = (by * p.WM + wm) * MB;
     struct A {
         bf8_t h[3];
@@ -332,6 +336,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 
     // ---- results ---------------------------------------------------------------------------------------------------------
     const int ch_base = mblk0 * 16 + 4 * k;
+    const bool scaled = __builtin_amdgcn_readfirstlane(__float_as_int(scaled_flag)) == 0x3f800000;
     const bool has_resid = p.resid != nullptr;
     // One sum in fp32 from the unsplit input (see above): channel ch, pixel pix of image img.
     auto exact_sum = [&](int ch, int img, int pix) {
@@ -385,12 +390,21 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
                 if ((MODE == SPLIT_FLAT ? j < px.fresh : px.fresh != 0) || ch >= p.N) continue;
                 const int pix = px.pix + (MODE == SPLIT_FLAT ? j : 0);
                 float sum = exact_sum(ch, px.img, pix);
+                if (scaled) sum *= w_scale[ch];
                 if (p.bias) sum += p.bias[ch];
                 if (has_resid) sum += p.resid[(long long)px.img * p.resid_bstride + (long long)ch * p.P + pix];
                 if (p.relu) sum = fmaxf(sum, 0.0f);
                 p.out[(long long)px.img * p.out_bstride + (long long)ch * p.P + pix] = sum;
             }
             return;
+        }
+        if (__builtin_expect(scaled, 0)) {
+#pragma unroll
+            for (int m = 0; m < MB; ++m) {
+                const f4_t s = *reinterpret_cast<const f4u_t *>(w_scale + ch_base + 16 * m);   // (padded to whole blocks)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) lead[m][j] *= s;
+            }
         }
     }
     if constexpr (MODE == SPLIT_FLAT) {
@@ -476,6 +490,10 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
                     for (int x = 0; x < 2 * NB; ++x) v[x / NB][x % NB] = x == r ? s : v[x / NB][x % NB];
                 }
+            }
+            if (__builtin_expect(scaled, 0)) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) v[i] *= w_scale[ch[i]];
             }
             finish(v[0], ch[0], bv[0], rv[0]);
             if (r0 + 1 < rows) finish(v[1], ch[1], bv[1], rv[1]);

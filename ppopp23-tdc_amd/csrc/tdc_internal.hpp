@@ -72,6 +72,7 @@ struct Geometry {
     // power of two), K-steps per stage, taps (pairs
     // of taps with at most four channels) per filter row.  win_L = window rows of one image, RS / CS = slots per row / octet.
     int units_wg = 0, oct_shift = 0, ksteps = 0, row_taps = 1;
+    int scale_floats = 0;            // tile.alg = 8, behind the packed weights: 1 if any of the following is not 1, 3 unused, a factor per (padded) output channel
     int channel_major = 0;           // which logical workgroup order costs fewer L2 fills (see conv_staged.hip)
     double b_ways = 1.0;             // serialisation of the B-operand LDS read by bank conflicts (1 = none)
 };
@@ -117,6 +118,7 @@ inline FastDiv make_fastdiv(int d) {
 struct ConvKParams {
     const float *in;
     const float *wpk;
+    const float *w_scale;      // tile.alg = 8: factors of the output channels (see Geometry::scale_floats)
     const float *bias;
     const float *resid;
     const float *in_aff;       // optional per-input-channel affine in front of a 1x1 convolution: [pass][scale(CCH) | shift(CCH)]

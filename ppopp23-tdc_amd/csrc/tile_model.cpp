@@ -223,7 +223,8 @@ static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geome
         return fail("grid too large");
     g.grid_x = (int)gx;
     g.wslab_floats = t.wm * t.mb * g.ksteps * 3 * 256;
-    if ((long long)g.grid_y * g.nchunks * g.wslab_floats * 4 >= (1LL << 31)) return fail("packed weights exceed 2 GiB");
+    g.scale_floats = 4 + g.grid_y * g.MT;
+    if ((long long)packed_weight_floats(g) * 4 >= (1LL << 31)) return fail("packed weights exceed 2 GiB");
     g.channel_major = channel_major_order(4.0 * d.batch * d.C * d.H * d.W, 6.0 * d.N * d.C * g.taps, n_wg, g.grid_y);
     return true;
 }
@@ -511,7 +512,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
 }
 
 size_t packed_weight_floats(const Geometry &g) {
-    return (size_t)g.grid_y * (size_t)g.nchunks * (size_t)g.wslab_floats;
+    return (size_t)g.grid_y * (size_t)g.nchunks * (size_t)g.wslab_floats + (size_t)g.scale_floats;
 }
 
 static uint16_t to_bf16(float v) {   // nearest even; a finite value never becomes infinite
@@ -531,7 +532,27 @@ static float from_bf16(uint16_t h) {
 // tile.alg = 8: per (16 channels, pass, K-step, part): [lane][8], lane (n = l % 16, k = l / 16) holding part 0, 1 or 2 of the
 // weights of channel block*16 + n and K octet 4*step + k.  An octet is eight input channels of one tap, or (cch = 4) four
 // channels of two neighbouring taps of a filter row.
+// The last of the three parts is exact only above 2^-110, and sums below 2^-90 cost the kernel a second pass.  Trained networks
+// hold whole channels that weight decay left near nothing, so a channel whose largest weight is outside 2^-40 ... 2^20 is packed
+// times the power of two that brings it to 1, and its sums are multiplied by the inverse, which follows the weights.
+static float split_channel_scale(const tdc_conv_desc &d, const float *w, int n) {
+    const size_t per = (size_t)d.C * d.KH * d.KW;
+    float largest = 0.0f;
+    for (size_t i = 0; i < per; ++i)
+        if (std::isfinite(w[n * per + i])) largest = std::max(largest, std::fabs(w[n * per + i]));
+    return largest == 0.0f || (largest >= 0x1p-40f && largest <= 0x1p20f) ? 1.0f : std::ldexp(1.0f, std::ilogb(largest));
+}
+
 static void pack_split_weights(const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, const float *w, float *packed) {
+    float *const scales = packed + (packed_weight_floats(g) - g.scale_floats);
+    std::vector<int> shift((size_t)g.scale_floats - 4, 0);
+    std::fill(scales, scales + 4, 0.0f);
+    for (int n = 0; n < g.scale_floats - 4; ++n) {
+        const float s = n < d.N ? split_channel_scale(d, w, n) : 1.0f;
+        scales[4 + n] = s;
+        shift[n] = -std::ilogb(s);
+        if (shift[n]) scales[0] = 1.0f;
+    }
     uint16_t *const dst = reinterpret_cast<uint16_t *>(packed);
     const bool few = t.tw != 0 && t.cch == 4;
     const int octets = t.cch / 8, blocks = g.grid_y * t.wm * t.mb;
@@ -554,6 +575,7 @@ static void pack_split_weights(const tdc_conv_desc &d, const tdc_tile &t, const 
                             kx = tap % d.KW;
                         }
                         float v = (n < d.N && c < d.C && ky < d.KH && kx < d.KW) ? w[(((size_t)n * d.C + c) * d.KH + ky) * d.KW + kx] : 0.0f;
+                        if (shift[n]) v = std::ldexp(v, shift[n]);
                         for (int s = 0; s < 3; ++s) {
                             const uint16_t h = to_bf16(v);
                             dst[base + (size_t)s * 512 + l * 8 + e] = h;

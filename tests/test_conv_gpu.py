@@ -1121,6 +1121,40 @@ def test_split_tiles_with_special_values(shape, K, stride, pad):
         assert ((got - want_tiny).abs() <= 2.2e-5 * want_tiny.abs()).all(), f"tiny {shape} {t}"
 
 
+@pytest.mark.parametrize("shape,K,stride,pad", [((2, 40, 36, 8, 8), 1, 1, 0), ((2, 70, 20, 7, 7), 1, 1, 0), ((2, 40, 36, 9, 9), 3, 2, 1),
+                                                ((2, 3, 20, 12, 12), 7, 2, 3)])
+def test_split_tiles_with_channels_of_extreme_weights(shape, K, stride, pad):
+    """Channels whose weights are next to nothing (also subnormal) or very large come out as accurate as the others, alone and
+    beside an input whose own lower parts bf16 cannot hold; weights that replace others reach a captured graph."""
+    B, C, N, H, W = shape
+    g = seeded(8770)
+    x, w0 = torch.rand(B, C, H, W, generator=g) + 0.5, torch.rand(N, C, K, K, generator=g) + 0.5
+    w = w0.clone()
+    for n, s in ((1, 1e-13), (2, 1e-30), (3, 1e-37), (17, 1e20), (18, 1e30), (19, 0.0)):
+        w[n] *= s
+    tiny = x * 1e-36
+    wants = [torch.nn.functional.conv2d(v.double(), w.double(), None, stride, pad) for v in (x, tiny)]
+    for t in split_tiles(B, C, N, H, W, K, stride, pad):
+        announce("split extreme weights", shape, K, t)
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, K, K, stride, pad, tile=t).set_weights(w0)
+        xd, out = x.cuda(), torch.empty(wants[0].shape, device="cuda")
+        plan.forward(xd, out=out)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            plan.forward(xd, out=out)
+        plan.set_weights(w)
+        for v, want in zip((x, tiny), wants):
+            xd.copy_(v)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, plan.forward(xd)), f"graph {shape} {t}"
+            # (positive fp32 sums of at most 360 products, a rounding of 2^-24 each: 2.2e-5; a subnormal result is off by 2^-150
+            # at every rounding)
+            assert ((out.cpu().double() - want).abs() <= 2.2e-5 * want.abs() + 400 * 2.0 ** -150).all(), f"{shape} {t}"
+        plan.close()
+
+
 @pytest.mark.parametrize("K,stride,C", [(1, 1, 20), (3, 2, 20), (3, 2, 3)])
 def test_split_tiles_with_images_far_apart(K, stride, C):
     """tile.alg = 8 reaches the images of one workgroup through 32-bit offsets; images 2 GiB apart are launched one by one."""
