@@ -39,6 +39,30 @@ def check_features(net, feats, what):
         net_close(net.read(tid).numpy(), ref, f"{what} {name}")
 
 
+@pytest.mark.parametrize("B,C,H,W", [(1, 1, 1, 4), (2, 3, 2, 4), (3, 5, 7, 8), (2, 37, 13, 12), (2, 6, 16, 260), (1, 2, 9, 6), (2, 3, 5, 7)])
+def test_max_pool_3x3_stride_2(B, C, H, W):
+    """Rows of whole quads (the 128-bit kernel: one quad a row, one row, odd heights, a partly empty last block) and others; the
+    output as a tensor of its own, and as a slice of a wider buffer whose planes may leave it without 8-byte alignment.  Equal to
+    the reference bit for bit, negative values, infinities and signed zeros among them."""
+    g = torch.Generator().manual_seed(17)
+    x = torch.randn(B, C, H, W, generator=g) - 1.0
+    x.view(-1)[::7] = float("inf")
+    x.view(-1)[::5] = 0.0
+    want = torch.nn.functional.max_pool2d(x, 3, 2, 1)
+    Ho, Wo = want.shape[2], want.shape[3]
+    net = nets.Net(B, C, H, W)
+    a = net.pool(0, "max", 3, 2, 1)
+    cat = net.tensor(C + 1, Ho, Wo)
+    net.pool(0, "max", 3, 2, 1, dst=net.view(cat, 1, C))
+    net.pool(0, "max", 3, 2, 1, dst=net.view(cat, 0, C))
+    net.pool(0, "max", 3, 2, 1, dst=net.view(cat, 1, C))
+    net.finalize(a)
+    out = net(x.cuda()).cpu()
+    assert torch.equal(out, want) and torch.equal(net.read(a), want)
+    got = net.read(cat)
+    assert torch.equal(got[:, 1:], want) and torch.equal(got[:, :1], want[:, :1])
+
+
 def test_pool_and_concat_ops():
     g = torch.Generator().manual_seed(3)
     x = torch.randn(2, 6, 13, 11, generator=g)
