@@ -1027,6 +1027,10 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
                 const double blocks = std::ceil((double)ceil_div(tail_N, 16) / g.waves);
                 clk += MC.sync_clk + MC.stream_latency_clk + blocks * (g.tail_ng * 40.0 + 64.0) +
                        (double)tail_N * d.N * 4.0 * r / rate + (double)tail_N * 64.0 * r / 200.0;
+                // More than eight slices cost another 0.5 to 0.6 us here (timed, 12 to 16 slices against half as many with twice the
+                // channel groups each: 64 -> 16 -> 32 @14 4.73 against 4.21 us, 48 -> 16 -> 96 @20 4.74 against 4.24, 100 -> 16 -> 40
+                // @21 5.46 against 5.22, 128 -> 16 -> 64 @14 5.58 against 5.35); up to eight, also times two channel blocks, nothing.
+                if (t.wk > 8) clk += 1300.0;
                 return clk;
             }
             if (t.ks > 1) clk += MC.ksplit_clk + 1000.0 * (t.ks - 2) + (double)t.ks * 1024.0 * r / rate;   // (timed: each slice past the second adds 0.4 us)
