@@ -1326,7 +1326,7 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
         }
     }
     // Winograd over the tiles of the whole batch: batches, and single images of more than 64x64 pixels (224x224 17.3 -> 15.0
-    // us, 96x96 14.6 -> 12.4; at 56x56 the streamed Winograd kernel is as fast).  It leaves nothing to the staged one there.
+    // us, 96x96 14.6 -> 12.4; at 56x56 the streamed Winograd kernel is as fast).
     const bool wino_batch = (d.batch > 1 || P > 4096) && d.KH == 3 && d.KW == 3 && d.stride == 1 && d.dilation == 1 && d.pad <= 1 &&
                             d.H * d.W >= 8 && tail_N == 0 && !std::getenv("TDC_EXPERIMENT_NO_WINOGRAD");
     if (wino_batch)
@@ -1342,8 +1342,10 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
                     if (mb == 2 && wn == 2 && (wk < 4 || g.grid_x * g.grid_y > machine().cus)) continue;
                     out.push_back(t);
                 }
-    // Winograd candidates for 3x3 / stride 1 convolutions with enough pixels to fill tile lanes
-    if (!wino_batch && d.KH == 3 && d.KW == 3 && d.stride == 1 && d.dilation == 1 && tail_N == 0 && !std::getenv("TDC_EXPERIMENT_NO_WINOGRAD")) {
+    // Winograd candidates for 3x3 / stride 1 convolutions with enough pixels to fill tile lanes.  Batches keep them beside the
+    // tiles above: those stop where batch * tiles * tiles reaches 2^32 (224x224 from 28 images, 512x512 from one), and deep
+    // layers with few output channels are cheaper with eight waves over channels.
+    if (d.KH == 3 && d.KW == 3 && d.stride == 1 && d.dilation == 1 && tail_N == 0 && !std::getenv("TDC_EXPERIMENT_NO_WINOGRAD")) {
         const int Wt = ceil_div(Wo, 2), Ht = ceil_div(Ho, 2);
         for (int wm : wms)
             for (int wn : wns)
@@ -1465,15 +1467,30 @@ bool model_set_constants(const double *in, int n) {
     return true;
 }
 
+// The price of a staged Winograd tile stands too low against the tiles over the whole batch, except where its workgroups have
+// a compute unit each and eight slices of the input channels, or where four workgroups share those.  Timed against the best
+// other tile, 126 shapes where its price is the lowest: outside of these two 1.21 times as long on average (up to 2.2 times),
+// inside 0.85 of the time (0.65 to 1.13).
+static double staged_winograd_handicap(const tdc_tile_info &info) {
+    const tdc_tile &t = info.tile;
+    if (t.alg != 1 || t.tw == 0) return 1.0;
+    const long long n_wg = (long long)info.grid_x * info.grid_y * info.grid_z;
+    return t.wl == 0 && (t.ks >= 4 ? t.wk >= 4 : t.wk >= 8 && n_wg <= machine().cus) ? 1.0 : 1.35;
+}
+
 bool model_select(const tdc_conv_desc &d, tdc_tile_info &best, std::string *why, int tail_N) {
     if (!check_desc(d, why)) return false;
     std::vector<tdc_tile> cands = model_enumerate(d, tail_N);
+    const bool batched = std::any_of(cands.begin(), cands.end(), [](const tdc_tile &t) { return t.alg == 1 && t.tw == 0; });
     bool have = false;
+    double best_us = 0.0;
     for (const tdc_tile &t : cands) {
         tdc_tile_info info;
         if (!model_evaluate(d, t, info, nullptr, tail_N)) continue;
-        if (!have || info.pred_us < best.pred_us) {
+        const double us = info.pred_us * (batched ? staged_winograd_handicap(info) : 1.0);
+        if (!have || us < best_us) {
             best = info;
+            best_us = us;
             have = true;
         }
     }

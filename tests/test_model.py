@@ -155,6 +155,19 @@ def test_winograd_tiles_only_where_the_algorithm_applies():
     assert not any(t.alg == 1 for t in tdc_amd.model_enumerate(conv3(64, 64, 56, stride=2)))
 
 
+@pytest.mark.parametrize("batch,C,N,H,W", [(27, 64, 32, 224, 224), (28, 64, 32, 224, 224), (1, 64, 32, 512, 512), (2, 944, 512, 16, 16),
+                                           (5, 688, 32, 32, 32)])
+def test_batches_keep_the_staged_winograd_tiles(batch, C, N, H, W):
+    """The Winograd tiles over the whole batch (tw = 0) stop at 2^32 = batch * tiles * tiles (224x224: 27 images still have them,
+    28 do not) and are dear for deep layers with few pixels: the staged ones are offered beside them, and picked where they
+    were timed faster (944 -> 512 @16 batch 2 35 against 46 us, 688 -> 32 @32 batch 5 22 against 30)."""
+    d = tdc_amd.conv_desc(batch, C, N, H, W, 3, 3, 1, 1)
+    tiles = [t for t in tdc_amd.model_enumerate(d) if t.alg == 1]
+    assert any(t.tw > 0 for t in tiles) and any(t.tw == 0 for t in tiles) == (batch * (H // 2 * (W // 2)) ** 2 < 1 << 32)
+    if C > 64:
+        assert tdc_amd.model_select(d).tile.alg == 1 and tdc_amd.model_select(d).tile.tw > 0
+
+
 def test_algorithmic_work_and_roofline_of_config1():
     i = tdc_amd.model_select(conv3(32, 32, 56))
     assert i.flops == 2 * 56 * 56 * 32 * 32 * 9 == 57802752
