@@ -158,4 +158,47 @@ __device__ __forceinline__ ImageBase image_base(const ConvKParams &p, int img) {
     return b;
 }
 
+// A block of 16 channels x 16 pixels as plain fp32 sums over the weights as the caller gave them (p.w_raw, OIHW): for the rare
+// outputs that a transform or a split of the operands cannot represent.  Lane (k = l / 16, n = l % 16) names channel `ch` (row n
+// of the block; past N: any) and output pixel (oy, ox) of image `img` (column n); it gets rows 4k .. 4k + 3 of its pixel.  Every
+// lane of the wave must call it.  Padding counts (0 * inf).  AFF: the input affine of a 1x1 convolution.
+// Bound: latency, sixteen channels in flight; a wave in which it runs takes several times as long.
+template <bool AFF>
+__device__ __forceinline__ f4_t direct_block(const ConvKParams &p, int ch, int img, int oy, int ox) {
+    const int k = (threadIdx.x >> 4) & 3;
+    const int taps = p.KH * p.KW, plane = p.H * p.W;
+    const float *const w = p.w_raw + (size_t)min(ch, p.N - 1) * p.C * taps;
+    const float *const src = p.in + (long long)img * p.in_bstride;
+    f4_t part[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) part[u] = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 1
+    for (int tap = 0; tap < taps; ++tap) {
+        const int kr = tap / p.KW;
+        const int y = oy * p.stride + kr * p.dil - p.pad, x = ox * p.stride + (tap - kr * p.KW) * p.dil - p.pad;
+        const bool inside = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.W;
+        const int pix = inside ? y * p.W + x : 0;
+#pragma unroll 1
+        for (int c0 = k; c0 < p.C + k; c0 += 16) {      // (the same number of turns for every lane)
+            float a[4], b[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int c = c0 + 4 * u, cc = min(c, p.C - 1);
+                a[u] = w[(size_t)cc * taps + tap];
+                b[u] = src[(size_t)cc * plane + pix];
+                if constexpr (AFF) {
+                    const float *const aff = p.in_aff + (size_t)(cc / p.CCH) * 2 * p.CCH + cc % p.CCH;
+                    b[u] = b[u] * aff[0] + aff[p.CCH];
+                    if (p.in_relu) b[u] = fmaxf(b[u], 0.0f);
+                }
+                a[u] = c < p.C ? a[u] : 0.0f;
+                b[u] = c < p.C && inside ? b[u] : 0.0f;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) part[u] = Mfma<16>::run(a[u], b[u], part[u]);
+        }
+    }
+    return (part[0] + part[1]) + (part[2] + part[3]);
+}
+
 }  // namespace tdc

@@ -28,6 +28,8 @@ typedef float f2u_t __attribute__((ext_vector_type(2), aligned(4)));
 // batch 64 35.3 -> 25.9, 128 -> 128 @14 batch 32 20.1 -> 15.3, 32 -> 32 @56 batch 32 20.1 -> 15.7; on sizes the tiles of
 // that kernel do not divide 1.3 to 2 times as fast (64 -> 176 @59 batch 13 103 -> 50, 145 random shapes 1.5 on average).
 // WK teams of WN waves split the input channels; their 2x2 outputs are added through LDS in team order.
+// Outputs that come out infinite or NaN are computed as plain sums (direct_block); the look at them costs at most 0.1 us
+// (60 -> 84 @35 batch 5 10.3 -> 10.4, 128 -> 128 @56 batch 64 within 1 %).
 // ---------------------------------------------------------------------------
 template <int MB, int WN>
 __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKParams p) {
@@ -257,8 +259,16 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
         v[3] = two_cols && two_rows ? r[p.Wo + 1] : v[0];
         return v;
     };
-    auto store = [&](f4_t v, int ch) {
-        if (!live || ch >= p.N) return;
+    // The transform makes more sums infinite or NaN than those whose own window holds such a value, and sums of four inputs
+    // overflow early: rows of a lane with one among their outputs are left out here and computed as plain sums at the end.
+    int left_out = 0;
+    auto unusual = [&](f4_t v, int row) {
+        const bool bad = !((fabsf(v[0]) + fabsf(v[1])) + (fabsf(v[2]) + fabsf(v[3])) < __builtin_inff());
+        left_out |= (bad ? 1 : 0) << row;
+        return bad;
+    };
+    auto store = [&](f4_t v, int ch, bool skip) {
+        if (!live || ch >= p.N || skip) return;
         float *o = out + (long long)ch * p.P;
         if (two_cols) {
             *reinterpret_cast<f2u_t *>(o) = (f2_t){v[0], v[1]};
@@ -293,25 +303,48 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
                 for (int i = 0; i < 4; ++i) rv[i] = load_resid(ch0 + i);
             }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) store(finish(output(m, i), bv[i], rv[i]), ch0 + i);
+            for (int i = 0; i < 4; ++i) {
+                const f4_t v = output(m, i);
+                store(finish(v, bv[i], rv[i]), ch0 + i, unusual(v, 4 * m + i));
+            }
         }
-        return;
+    } else {
+        // the teams leave their outputs in LDS, [wn][team][row = 4m + i][lane], and finish every WK-th row each
+        f4_t *part = reinterpret_cast<f4_t *>(lds) + (size_t)(wn * p.WK) * (4 * MB * 64) + lane;
+#pragma unroll
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part[(slice * 4 * MB + 4 * m + i) * 64] = output(m, i);
+        __syncthreads();
+        for (int row = slice; row < 4 * MB; row += p.WK) {
+            const int ch = ch_base + 16 * (row >> 2) + (row & 3);
+            f4_t rv = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
+            if (has_resid) rv = load_resid(ch);
+            const float bv = p.bias ? p.bias[min(ch, p.N - 1)] : 0.0f;
+            f4_t v = part[row * 64];
+            for (int s = 1; s < p.WK; ++s) v += part[(s * 4 * MB + row) * 64];
+            store(finish(v, bv, rv), ch, unusual(v, row));
+        }
     }
-    // the teams leave their outputs in LDS, [wn][team][row = 4m + i][lane], and finish every WK-th row each
-    f4_t *part = reinterpret_cast<f4_t *>(lds) + (size_t)(wn * p.WK) * (4 * MB * 64) + lane;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(left_out != 0) == 0, 1)) return;
+#pragma unroll 1
+    for (int m = 0; m < MB; ++m) {
+        f4_t sums[4];                           // of the four pixels of the tile, rows 4m .. 4m + 3
+        if (__builtin_amdgcn_ballot_w64((left_out >> (4 * m) & 15) != 0) == 0) continue;
+#pragma unroll 1
+        for (int e = 0; e < 4; ++e) {
+            const f4_t s = direct_block<false>(p, ch_base - 4 * k + 16 * m + n, img, min(oy + (e >> 1), p.Ho - 1), min(ox + (e & 1), p.Wo - 1));
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
+            for (int x = 0; x < 4; ++x) sums[x] = x == e ? s : sums[x];
+        }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) part[(slice * 4 * MB + 4 * m + i) * 64] = output(m, i);
-    __syncthreads();
-    for (int row = slice; row < 4 * MB; row += p.WK) {
-        const int ch = ch_base + 16 * (row >> 2) + (row & 3);
-        f4_t rv = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
-        if (has_resid) rv = load_resid(ch);
-        const float bv = p.bias ? p.bias[min(ch, p.N - 1)] : 0.0f;
-        f4_t v = part[row * 64];
-        for (int s = 1; s < p.WK; ++s) v += part[(s * 4 * MB + row) * 64];
-        store(finish(v, bv, rv), ch);
+        for (int i = 0; i < 4; ++i) {
+            const int ch = ch_base + 16 * m + i;
+            const bool skip = (left_out >> (4 * m + i) & 1) == 0;
+            f4_t rv = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
+            if (has_resid) rv = load_resid(ch);
+            store(finish((f4_t){sums[0][i], sums[1][i], sums[2][i], sums[3][i]}, p.bias ? p.bias[min(ch, p.N - 1)] : 0.0f, rv), ch, skip);
+        }
     }
 }
 

@@ -393,8 +393,9 @@ static void refresh_launch_params(tdc_conv_plan *plan) {
     kp.channel_major = g.channel_major;
     kp.fd_g1 = make_fastdiv(g.channel_major ? g.grid_x : g.grid_y);
     kp.fd_g2 = make_fastdiv(g.channel_major ? g.grid_y : g.grid_x);
-    kp.wpk_bytes = (unsigned)(packed_weight_floats(g) * sizeof(float));
-    kp.w_scale = plan->d_wpk + (packed_weight_floats(g) - g.scale_floats);
+    kp.wpk_bytes = (unsigned)(packed_part_floats(g) * sizeof(float));
+    kp.w_scale = plan->d_wpk + packed_part_floats(g);
+    kp.w_raw = kp.w_scale + g.scale_floats;
 #if defined(TDC_STAMPS) && TDC_STAMPS
     kp.stamps = plan->d_stamps;
 #endif

@@ -73,6 +73,7 @@ struct Geometry {
     // of taps with at most four channels) per filter row.  win_L = window rows of one image, RS / CS = slots per row / octet.
     int units_wg = 0, oct_shift = 0, ksteps = 0, row_taps = 1;
     int scale_floats = 0;            // tile.alg = 8, behind the packed weights: 1 if any of the following is not 1, 3 unused, a factor per (padded) output channel
+    size_t raw_floats = 0;           // tile.alg = 8 and 1 with tw = 0, last: the weights as they came (see direct_block)
     int channel_major = 0;           // which logical workgroup order costs fewer L2 fills (see conv_staged.hip)
     double b_ways = 1.0;             // serialisation of the B-operand LDS read by bank conflicts (1 = none)
 };
@@ -95,7 +96,9 @@ bool model_set_constants(const double *in, int n);
 // w[tile*MT + mblk*mf + l%mf][pass*cch + cg*kc + l/mf][tap], zero outside N x C.
 // tile.alg = 2 regroups the nine taps of a channel group as [taps 0-3][lane][4] [taps 4-7][lane][4] [tap 8][lane];
 // tile.alg = 1 and 5 store the 16 Winograd-domain values U = G g G^T of every (n, c) as [quarter][lane][4].
-size_t packed_weight_floats(const Geometry &g);
+// What follows the packed weights proper: Geometry::scale_floats, then Geometry::raw_floats.
+size_t packed_part_floats(const Geometry &g);         // the packed weights proper
+size_t packed_weight_floats(const Geometry &g);       // all of the buffer
 void pack_weights(const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, const float *w_oihw, float *packed);
 
 // Division of a small non-negative integer by a run-time constant without a branch:
@@ -167,6 +170,7 @@ struct ConvKParams {
     long long in_bstride;      // floats between consecutive images of the input (C*H*W when dense)
     long long out_bstride;     // ... of the output (N*P when dense)
     long long resid_bstride;   // ... of the residual
+    const float *w_raw;        // the weights as they came, OIHW (see Geometry::raw_floats)
 #if defined(TDC_STAMPS) && TDC_STAMPS
     unsigned long long *stamps;   // profiling build: [workgroup][16 waves][8] time stamps, or null
 #endif

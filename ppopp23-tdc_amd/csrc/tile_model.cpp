@@ -224,7 +224,7 @@ static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geome
     g.grid_x = (int)gx;
     g.wslab_floats = t.wm * t.mb * g.ksteps * 3 * 256;
     g.scale_floats = 4 + g.grid_y * g.MT;
-    if ((long long)packed_weight_floats(g) * 4 >= (1LL << 31)) return fail("packed weights exceed 2 GiB");
+    if ((long long)(packed_part_floats(g) + g.scale_floats) * 4 >= (1LL << 31)) return fail("packed weights exceed 2 GiB");
     g.channel_major = channel_major_order(4.0 * d.batch * d.C * d.H * d.W, 6.0 * d.N * d.C * g.taps, n_wg, g.grid_y);
     return true;
 }
@@ -324,6 +324,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         if (units * g.units_image >= (1LL << 32) || units >= (1LL << 30)) return fail("batch too large for tile.alg = 1 with tw = 0");
         if (d.H * d.W < 8) return fail("tile.alg = 1 with tw = 0 needs images of at least 8 pixels");
         g.units = (int)units;
+        g.raw_floats = (size_t)d.N * d.C * 9;
         g.unit_images = std::min(d.batch - 1, 14 / g.units_image + 1);
         g.TW = 2 * std::min(g.TWt, 16 * t.wn);
         g.TH = 2;
@@ -511,9 +512,8 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     return true;
 }
 
-size_t packed_weight_floats(const Geometry &g) {
-    return (size_t)g.grid_y * (size_t)g.nchunks * (size_t)g.wslab_floats + (size_t)g.scale_floats;
-}
+size_t packed_part_floats(const Geometry &g) { return (size_t)g.grid_y * (size_t)g.nchunks * (size_t)g.wslab_floats; }
+size_t packed_weight_floats(const Geometry &g) { return packed_part_floats(g) + (size_t)g.scale_floats + g.raw_floats; }
 
 static uint16_t to_bf16(float v) {   // nearest even; a finite value never becomes infinite
     uint32_t u;
@@ -544,7 +544,7 @@ static float split_channel_scale(const tdc_conv_desc &d, const float *w, int n) 
 }
 
 static void pack_split_weights(const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, const float *w, float *packed) {
-    float *const scales = packed + (packed_weight_floats(g) - g.scale_floats);
+    float *const scales = packed + packed_part_floats(g);
     std::vector<int> shift((size_t)g.scale_floats - 4, 0);
     std::fill(scales, scales + 4, 0.0f);
     for (int n = 0; n < g.scale_floats - 4; ++n) {
@@ -589,6 +589,7 @@ void pack_weights(const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, 
     const int ncg = t.cch / g.kc;
     const int taps = g.taps;
     float *dst = packed;
+    if (g.raw_floats) std::memcpy(packed + (packed_weight_floats(g) - g.raw_floats), w, g.raw_floats * sizeof(float));
     if (t.alg == 8) {
         pack_split_weights(d, t, g, w, packed);
         return;

@@ -1016,6 +1016,28 @@ def test_every_batched_winograd_tile(shape, pad):
         assert (got[:, :4] == 7.0).all() and (got[:, 4 + N:] == 7.0).all()
 
 
+@pytest.mark.parametrize("shape,pad", [((2, 13, 20, 9, 11), 1), ((3, 40, 40, 8, 7), 0), ((5, 33, 17, 4, 4), 1)])
+def test_batched_winograd_tiles_with_special_values(shape, pad):
+    """Infinities and NaN in the input and in the weights reach exactly the outputs whose 3x3 window holds them, and neighbours
+    whose sum overflows in the input transform (four of 1.5e38) come out finite, as plain fp32 sums give them."""
+    B, C, N, H, W = shape
+    g = seeded(8790)
+    x, w = torch.rand(B, C, H, W, generator=g) + 0.1, torch.rand(N, C, 3, 3, generator=g) * 0.2 + 0.1
+    w[3] = -w[3]
+    w[5, 1, 0, 0] = float("inf")
+    x[0, 1, 2, 3], x[0, 2, 3, 0], x[1, 0, 1, 1] = float("inf"), -float("inf"), float("nan")
+    x[1, 4, 2:4, 2:4] = 1.5e38
+    want = torch.nn.functional.conv2d(x.double(), w.double(), None, 1, pad).float()
+    assert torch.isinf(want).any() and torch.isnan(want).any() and (want.abs() > 1e38).any() and torch.isfinite(want).any()
+    # (positive fp32 sums of at most 360 products, a rounding of 2^-24 each: 2.2e-5; Winograd's transforms four times that)
+    tiles = [t for t in tdc_amd.model_enumerate(tdc_amd.conv_desc(B, C, N, H, W, 3, 3, 1, pad)) if t.alg == 1 and t.tw == 0]
+    assert {t.wk for t in tiles} >= {1, 4}
+    for t in tiles:
+        announce("batched winograd special values", shape, pad, t)
+        got = torch.from_numpy(run_conv(x, w, pad=pad, tile=t))
+        assert torch.allclose(got, want, rtol=1e-4, atol=0.0, equal_nan=True), f"{shape} {t}"
+
+
 def split_tiles(B, C, N, H, W, K, stride, pad, dil=1):
     """Every launchable tile of the split-operand kernel (tile.alg = 8), also those the model does not offer at this size."""
     d = tdc_amd.conv_desc(B, C, N, H, W, K, K, stride, pad, dil)
