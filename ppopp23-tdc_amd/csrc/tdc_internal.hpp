@@ -86,6 +86,7 @@ bool check_desc(const tdc_conv_desc &d, std::string *why);
 
 bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &info, std::string *why, int tail_N = 0);
 std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N = 0);
+std::vector<tdc_tile_info> model_choices(const tdc_conv_desc &d, int tail_N = 0);   // what a pick, by price or by timing, is made from
 bool model_select(const tdc_conv_desc &d, tdc_tile_info &info, std::string *why, int tail_N = 0);
 int model_constants(double *out, int cap);            // returns the number of constants
 bool model_set_constants(const double *in, int n);

@@ -168,6 +168,20 @@ def test_batches_keep_the_staged_winograd_tiles(batch, C, N, H, W):
         assert tdc_amd.model_select(d).tile.alg == 1 and tdc_amd.model_select(d).tile.tw > 0
 
 
+@pytest.mark.parametrize("batch,C,N,hw,alg", [(16, 32, 32, 28, (4, 6)), (8, 32, 64, 28, (4, 6)), (48, 16, 112, 12, (4, 6)),
+                                              (64, 64, 64, 7, (4, 6)), (32, 16, 16, 56, (4, 6)), (3, 144, 48, 31, (1,)), (32, 32, 32, 56, (1,))])
+def test_batches_take_winograd_only_where_its_error_is_no_larger(batch, C, N, hw, alg):
+    """Direct kernels whose waves share few input channels have half the rounding error of Winograd: batches keep them there."""
+    assert tdc_amd.model_select(tdc_amd.conv_desc(batch, C, N, hw, hw, 3, 3, 1, 1)).tile.alg in alg
+
+
+@pytest.mark.parametrize("batch,C,N,H,W,wk", [(8, 128, 32, 105, 105, 2), (15, 94, 87, 42, 46, 2), (17, 528, 112, 40, 40, 4)])
+def test_batched_winograd_chains_are_no_longer_than_the_staged_ones(batch, C, N, H, W, wk):
+    """... and where the staged Winograd tile splits the input channels over waves, so do those over the whole batch."""
+    t = tdc_amd.model_select(tdc_amd.conv_desc(batch, C, N, H, W, 3, 3, 1, 1)).tile
+    assert t.alg == 1 and t.wk * t.ks >= wk
+
+
 def test_algorithmic_work_and_roofline_of_config1():
     i = tdc_amd.model_select(conv3(32, 32, 56))
     assert i.flops == 2 * 56 * 56 * 32 * 32 * 9 == 57802752
