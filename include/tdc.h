@@ -92,7 +92,8 @@ typedef struct tdc_tile {
                          With tw = 0 (pad <= 1, images of 8 pixels and more) the output tiles of the whole batch are counted
                          in one row: 16 * mb channels (mb 1 or 2) x 16 tiles per wave, wn = 2 or 4 waves over tiles that
                          share the weights through LDS, wk teams of them over input channels (at most 8 waves; cch = C
-                         rounded up to 8 * wk), input straight into registers; wm = nb = ks = 1, wl = 0, grid_z = 1.
+                         rounded up to 8 * wk), input straight into registers; wm = ks = 1, wl = 0, grid_z = 1.  nb = 2 adds up the sums
+                         in parts of 64 channels (not with mb = wn = 2).
                      2 = direct 3x3 / dilation 1 convolution with the weights read from global memory straight
                          into registers (the LDS holds input only, so a pass can take more input channels);
                          mb = nb = 1, an even number of channel groups per wave and pass.

@@ -31,7 +31,12 @@ typedef float f2u_t __attribute__((ext_vector_type(2), aligned(4)));
 // Outputs that come out infinite or NaN are computed as plain sums (direct_block); the look at them costs at most 0.1 us
 // (60 -> 84 @35 batch 5 10.3 -> 10.4, 128 -> 128 @56 batch 64 within 1 %).
 // ---------------------------------------------------------------------------
-template <int MB, int WN>
+// PARTS: every eight steps (64 channels of the team) the outputs of the sums so far are added up in LDS and the sums start at
+// zero again, 4 * MB KiB per wave.  The error of a chain grows with the root of its length: 528 -> 112 @40 batch 17 in one chain
+// 7.0e-7 and 141 us, staged with four slices 3.6e-7 and 216, two teams in parts 2.7e-7 and 164.  Beside the same tile in one
+// chain 1.05 to 1.06 of the time with four waves, 1.00 to 1.025 with eight (82 to 1024 channels, 63 shapes), so it is a form of
+// its own, for layers whose other tiles have shorter chains than a team.
+template <int MB, int WN, bool PARTS>
 __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKParams p) {
     constexpr int G = 2;                        // groups of four channels per step (four never won: fewer waves fit)
     constexpr int CHUNKS = MB * G * 4;          // KiB of transformed weights per team and step
@@ -228,18 +233,7 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
             }
         }
     };
-    int st = 0;
-    for (; st < steps - 2; ++st) step(st, std::integral_constant<int, 2>{});
-    if (st < steps - 1) step(st++, std::integral_constant<int, 1>{});
-    step(st, std::integral_constant<int, 0>{});
-    barrier();                                  // (the buffers are used again below)
-
     // Y = A^T M A (A^T = [1 1 1 0; 0 1 -1 -1]): lane (k, n) holds channels 4k + i of tile n, all 16 positions
-    const int oy = 2 * ty, ox = 2 * tx;
-    const bool two_cols = ox + 1 < p.Wo, two_rows = oy + 1 < p.Ho;
-    float *__restrict__ out = p.out + ((long long)img * p.out_bstride + (oy * p.Wo + ox));
-    const bool has_resid = p.resid != nullptr;
-    const float *__restrict__ resid = has_resid ? p.resid + ((long long)img * p.resid_bstride + (oy * p.Wo + ox)) : nullptr;
     auto output = [&](int m, int i) {
         float s[2][4];
 #pragma unroll
@@ -250,6 +244,31 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
         }
         return (f4_t){s[0][0] + s[0][1] + s[0][2], s[0][1] - s[0][2] - s[0][3], s[1][0] + s[1][1] + s[1][2], s[1][1] - s[1][2] - s[1][3]};
     };
+    // outputs of the teams and of the parts of their sums: [wn][team][row = 4m + i][lane]
+    f4_t *const part = reinterpret_cast<f4_t *>(lds) + (PARTS ? 2 * ustage : 0) + (size_t)(wn * p.WK) * (4 * MB * 64) + lane;
+    f4_t *const own = part + slice * (4 * MB * 64);
+    int st = 0;
+    for (; st < steps - 2; ++st) {
+        if (PARTS && st > 0 && st % 8 == 0) {
+#pragma unroll
+            for (int m = 0; m < MB; ++m) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) own[(4 * m + i) * 64] = st == 8 ? output(m, i) : own[(4 * m + i) * 64] + output(m, i);
+#pragma unroll
+                for (int x = 0; x < 16; ++x) acc[m][x] = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
+            }
+        }
+        step(st, std::integral_constant<int, 2>{});
+    }
+    if (st < steps - 1) step(st++, std::integral_constant<int, 1>{});
+    step(st, std::integral_constant<int, 0>{});
+    barrier();                                  // (the buffers are used again below)
+
+    const int oy = 2 * ty, ox = 2 * tx;
+    const bool two_cols = ox + 1 < p.Wo, two_rows = oy + 1 < p.Ho;
+    float *__restrict__ out = p.out + ((long long)img * p.out_bstride + (oy * p.Wo + ox));
+    const bool has_resid = p.resid != nullptr;
+    const float *__restrict__ resid = has_resid ? p.resid + ((long long)img * p.resid_bstride + (oy * p.Wo + ox)) : nullptr;
     auto load_resid = [&](int ch) {             // (pixels outside the image repeat the tile's first: never stored)
         const float *r = resid + (long long)min(ch, p.N - 1) * p.P;
         f4_t v;
@@ -287,6 +306,7 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
         }
         return v;
     };
+    const bool parted = PARTS && steps > 10;    // (the last two steps never start a part)
     const int ch_base = by * (16 * MB) + 4 * k;
     if (p.WK == 1) {
 #pragma unroll
@@ -304,17 +324,17 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const f4_t v = output(m, i);
+                f4_t v = output(m, i);
+                if (parted) v += own[(4 * m + i) * 64];
                 store(finish(v, bv[i], rv[i]), ch0 + i, unusual(v, 4 * m + i));
             }
         }
     } else {
-        // the teams leave their outputs in LDS, [wn][team][row = 4m + i][lane], and finish every WK-th row each
-        f4_t *part = reinterpret_cast<f4_t *>(lds) + (size_t)(wn * p.WK) * (4 * MB * 64) + lane;
+        // every wave of a team finishes every WK-th row
 #pragma unroll
         for (int m = 0; m < MB; ++m)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) part[(slice * 4 * MB + 4 * m + i) * 64] = output(m, i);
+            for (int i = 0; i < 4; ++i) own[(4 * m + i) * 64] = parted ? own[(4 * m + i) * 64] + output(m, i) : output(m, i);
         __syncthreads();
         for (int row = slice; row < 4 * MB; row += p.WK) {
             const int ch = ch_base + 16 * (row >> 2) + (row & 3);
@@ -352,8 +372,11 @@ const void *wino_block_kernel_function(const KernelId &k) {
     using kernel_fn = void (*)(ConvKParams);
     kernel_fn fn = nullptr;
     if (k.family == KernelId::BLOCK_WINO) {
-        if (k.p[0] == 1) fn = k.p[1] == 4 ? static_cast<kernel_fn>(tdc_wino3x3_block_kernel<1, 4>) : k.p[1] == 2 ? static_cast<kernel_fn>(tdc_wino3x3_block_kernel<1, 2>) : nullptr;
-        if (k.p[0] == 2) fn = k.p[1] == 4 ? static_cast<kernel_fn>(tdc_wino3x3_block_kernel<2, 4>) : k.p[1] == 2 ? static_cast<kernel_fn>(tdc_wino3x3_block_kernel<2, 2>) : nullptr;
+        const bool parts = k.p[2] != 0, wide = k.p[1] == 4;
+        if (k.p[0] == 1 && wide) fn = parts ? static_cast<kernel_fn>(tdc_wino3x3_block_kernel<1, 4, true>) : tdc_wino3x3_block_kernel<1, 4, false>;
+        if (k.p[0] == 1 && k.p[1] == 2) fn = parts ? static_cast<kernel_fn>(tdc_wino3x3_block_kernel<1, 2, true>) : tdc_wino3x3_block_kernel<1, 2, false>;
+        if (k.p[0] == 2 && wide) fn = parts ? static_cast<kernel_fn>(tdc_wino3x3_block_kernel<2, 4, true>) : tdc_wino3x3_block_kernel<2, 4, false>;
+        if (k.p[0] == 2 && k.p[1] == 2 && !parts) fn = tdc_wino3x3_block_kernel<2, 2, false>;
     }
     return reinterpret_cast<const void *>(fn);
 }

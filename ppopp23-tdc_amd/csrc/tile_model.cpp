@@ -308,8 +308,9 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         // split the input channels, two groups of four channels per step
         if (d.KH != 3 || d.KW != 3 || d.stride != 1 || d.dilation != 1 || d.pad > 1)
             return fail("tile.alg = 1 with tw = 0 needs a 3x3 / stride 1 / dilation 1 / pad <= 1 convolution");
-        if (t.mf != 16 || t.wm != 1 || (t.wn != 2 && t.wn != 4) || t.nb != 1)
-            return fail("tile.alg = 1 with tw = 0 needs mf = 16, wm = nb = 1, wn = 2 or 4");
+        if (t.mf != 16 || t.wm != 1 || (t.wn != 2 && t.wn != 4))
+            return fail("tile.alg = 1 with tw = 0 needs mf = 16, wm = 1, wn = 2 or 4");
+        if (t.nb == 2 && t.mb == 2 && t.wn == 2) return fail("tile.alg = 1 with tw = 0: no sums in parts with mb = wn = 2");
         if (t.wl != 0 || t.ks != 1) return fail("tile.alg = 1 with tw = 0 has no loader waves and no split across workgroups");
         if (tail_N > 0) return fail("tile.alg = 1 cannot carry a fused tail");
         if (t.wk > 4 * t.mb) return fail("tile.alg = 1 with tw = 0: more teams than rows to finish");
@@ -471,8 +472,10 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     // (... and so does the streamed 3x3 kernel with several pixel blocks per wave: all its threads share the final store)
     const long long red_bytes = (t.wk > 1 || t.alg == 1 || t.alg == 5 || ((t.alg == 4 || t.alg == 6) && t.nb > 1)) ? (long long)t.wk * g.MT * g.PT * 4 : 0;
     long long lds = std::max(stage_bytes, red_bytes);
-    if (wino_batch)   // two buffers of transformed weights per team, or the outputs of all teams
-        lds = std::max<long long>(2LL * t.wk * t.mb * 2 * 4096, t.wk > 1 ? (long long)t.wk * t.wn * t.mb * 4096 : 0);
+    if (wino_batch) {   // two buffers of transformed weights per team, or the outputs of all teams (nb = 2: and those of their parts)
+        const long long weights = 2LL * t.wk * t.mb * 2 * 4096, outputs = (long long)t.wk * t.wn * t.mb * 4096;
+        lds = t.nb == 2 ? weights + outputs : std::max(weights, t.wk > 1 ? outputs : 0);
+    }
     if (tail_N > 0) {
         // A fused 1x1 tail needs every output channel of the convolution in one workgroup; its tile is parked
         // in LDS behind the split-K partials with a row stride that keeps the four channel quarters of a
@@ -785,10 +788,10 @@ KernelId kernel_id_for(const tdc_tile &t, int KH, int KW, int dilation, int stri
     }
     if (t.alg == 1 && t.tw == 0) {
         if (extras || KH != 3 || KW != 3 || dilation != 1 || stride != 1 || t.mf != 16 || t.wm != 1 || (t.wn != 2 && t.wn != 4) ||
-            (t.mb != 1 && t.mb != 2) || t.nb != 1)
+            (t.mb != 1 && t.mb != 2) || (t.nb != 1 && t.nb != 2) || (t.nb == 2 && t.mb == 2 && t.wn == 2))
             return k;
         k.family = KernelId::BLOCK_WINO;
-        k.p[0] = t.mb; k.p[1] = t.wn;
+        k.p[0] = t.mb; k.p[1] = t.wn; k.p[2] = t.nb == 2;
         return k;
     }
     if (t.alg == 7) {
@@ -881,7 +884,7 @@ std::string kernel_name(const KernelId &k) {
             std::snprintf(buf, sizeof buf, "tdc_wino3x3_stream_kernel<%d, %d>", k.p[0], k.p[1]);
             break;
         case KernelId::BLOCK_WINO:
-            std::snprintf(buf, sizeof buf, "tdc_wino3x3_block_kernel<%d, %d>", k.p[0], k.p[1]);
+            std::snprintf(buf, sizeof buf, "tdc_wino3x3_block_kernel<%d, %d, %s>", k.p[0], k.p[1], tf[k.p[2] != 0]);
             break;
         case KernelId::BLOCK_1x1:
             std::snprintf(buf, sizeof buf, "tdc_conv1x1_block_kernel<%d, %d, %s, %s>", k.p[0], k.p[1], tf[k.p[2] != 0], tf[k.p[3] != 0]);
@@ -1116,6 +1119,9 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
         if (t.wk > 1) clk += 707.0 + 58.0 * g.waves * t.mb * std::min(wgs_cu, 3.0);
         const double traffic = 4.0 * (d.batch * ((double)d.C * d.H * d.W + (double)d.N * P) + 16.0 * d.C * d.N);
         info.pred_us = 0.85 * (3.12 + clk / (m.clock_ghz * 1e3) + traffic / 4.45e6);
+        // (timed beside nb = 1 on 63 shapes of 82 to 1024 channels: 1.05 to 1.06 with four waves, at most 1.12, and 1.00 to 1.025
+        //  with eight, which leave the vector instructions of a part more room)
+        if (t.nb == 2) info.pred_us *= g.waves > 4 ? 1.02 : 1.06;
         info.pred_l2_bytes = 0.0;
         return true;
     }
@@ -1342,6 +1348,9 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
                     //  workgroups fit the chip at once; 256 -> 256 @7 batch 64 25.8 us against 28.2)
                     if (mb == 2 && wn == 2 && (wk < 4 || g.grid_x * g.grid_y > machine().cus)) continue;
                     out.push_back(t);
+                    // (the same with its sums in parts of eight steps, where there are several)
+                    t.nb = 2;
+                    if (t.cch / (8 * wk) > 10 && make_geometry(d, t, g, nullptr, 0)) out.push_back(t);
                 }
     // Winograd candidates for 3x3 / stride 1 convolutions with enough pixels to fill tile lanes.  Batches keep them beside the
     // tiles above: those stop where batch * tiles * tiles reaches 2^32 (224x224 from 28 images, 512x512 from one), and deep
@@ -1488,6 +1497,7 @@ static double rounding_variance(const tdc_conv_desc &d, const tdc_tile &t) {
     const double n = wino ? d.C : (double)d.C * d.KH * d.KW;
     double chain = n / ((double)t.wk * t.ks);
     if (t.alg == 3) chain = std::min(0.5 * t.cch / t.wk, n);
+    if (t.alg == 1 && t.tw == 0 && t.nb == 2) chain /= 1 + std::max(t.cch / (8 * t.wk) - 3, 0) / 8;   // (a part ends every eight steps but for the last two)
     if ((t.alg == 4 || t.alg == 6) && t.nb == 1) chain *= 0.5;   // (these keep two accumulators)
     const double v = 0.5 * (chain + n / (chain * t.ks) + (t.ks - 1));
     return wino ? 2.84 * v + 13.4 : v;

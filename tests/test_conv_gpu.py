@@ -1073,6 +1073,31 @@ def run_slices(plan, x, resid, N, Ho, Wo):
     return got[:, 4:4 + N].numpy()
 
 
+@pytest.mark.parametrize("shape,pad", [((2, 88, 20, 9, 11), 1), ((3, 81, 33, 8, 7), 0), ((2, 165, 40, 6, 6), 1), ((2, 330, 17, 5, 7), 1),
+                                       ((2, 512, 36, 4, 4), 1)])
+def test_batched_winograd_sums_in_parts(shape, pad):
+    """The form with sums in parts of 64 channels (nb = 2): one part end right before the last two steps, two of them, ragged
+    channels, one to four teams; plain and with the whole epilogue on channel slices.  The error against 64-bit sums stays within
+    1.3 times what chains of 80 channels, the longest, give: 2.5e-8 * sqrt(2.84 * (40 + C / 160) + 13.4) of the norm."""
+    B, C, N, H, W = shape
+    x, w = case(8795 + C, B, C, N, H, W, 3)
+    g = seeded(8796)
+    bias = torch.randn(N, generator=g)
+    exact = torch.nn.functional.conv2d(x.double(), w.double(), None, 1, pad)
+    Ho, Wo = exact.shape[2], exact.shape[3]
+    resid = torch.randn(B, N, Ho, Wo, generator=g)
+    want_full = (exact + bias.view(1, -1, 1, 1) + resid).clamp_min(0).float().numpy()
+    tiles = [t for t in tdc_amd.model_enumerate(tdc_amd.conv_desc(B, C, N, H, W, 3, 3, 1, pad)) if t.alg == 1 and t.tw == 0 and t.nb == 2]
+    assert {t.mb for t in tiles} == {1, 2} and (C < 330 or {t.wk for t in tiles} == {1, 2, 4})
+    for t in tiles:
+        announce("batched winograd in parts", shape, pad, t)
+        got = torch.from_numpy(run_conv(x, w, pad=pad, tile=t)).double()
+        assert (got - exact).norm() <= 1.3 * 2.5e-8 * math.sqrt(2.84 * (40 + C / 160) + 13.4) * exact.norm(), f"{shape} {t}"
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, 3, 3, 1, pad, 1, True, True, tile=t).set_weights(w, bias)
+        assert_close(run_slices(plan, x, resid, N, Ho, Wo), want_full, f"slices {shape} {t}")
+        plan.close()
+
+
 @pytest.mark.parametrize("shape,K,stride,pad,dil", [
     ((3, 20, 24, 7, 5), 1, 1, 0, 1), ((2, 33, 40, 9, 9), 1, 1, 0, 1), ((5, 300, 70, 7, 7), 1, 1, 0, 1), ((9, 64, 130, 2, 2), 1, 1, 0, 1),
     ((3, 70, 17, 1, 3), 1, 1, 0, 1), ((2, 260, 64, 12, 11), 1, 1, 0, 1), ((3, 16, 20, 7, 7), 3, 1, 1, 1), ((2, 40, 36, 13, 9), 3, 2, 1, 1),
