@@ -124,8 +124,8 @@ typedef struct tdc_tile {
                      7 = 1x1 / pad 0 convolution (any stride) for batches: 16 * mb channels x 16 * nb pixels per wave (mb 1 or 2,
                          nb 2 or 4), operands straight into registers one run of 16 channels ahead of the MFMAs; wm x wn
                          waves over channels and pixels, wk over input channels (at most 8 together; cch = C rounded up to
-                         16 * wk); the pixels of all images in one row, so grid_x counts them and grid_z is 1; tw = 1,
-                         ks = 1, wl = 0.  Carries the input affine, not a fused tail.
+                         16 * wk); the pixels of all images in one row, so grid_x counts them and grid_z is 1; tw = 1
+                         or, with the sums in parts of that many channels, 8, 16 or 32; ks = 1, wl = 0.  Carries the input affine, not a fused tail.
                      8 = fp32 as three bf16 parts per operand and six products on v_mfma_f32_16x16x32_bf16, accumulated in fp32
                          (the error against 64-bit sums is below that of the fp32 MFMAs; sums that come out NaN or under 2^-90,
                          where the split does not hold, are computed again without it).  16 * mb channels x 16 * nb pixels per

@@ -50,7 +50,11 @@ struct PixelGroup<2> {
 // 12.9 -> 7.8; even at about 4 us, slower below (0.2-0.3 us of index arithmetic in front of the first request).
 // Blocks of 64 channels per wave (mb = 4) were slower everywhere: too few waves to cover each other's start and end.
 // ---------------------------------------------------------------------------
-template <int MB, int NJ, bool AFF, bool GEN>
+// PART: the products of 8, 16 or 32 channels are summed apart, 0: all of a wave's in one chain, whose error grows with the root
+// of its length.  They cost 1.044, 1.036 and 1.013 of the time of PART = 0 (66 shapes, on average), and are taken where the tile
+// that would run otherwise has shorter chains: 304 -> 176 @53 in one chain 7.4 us and an error of 3.1e-7 against 64-bit sums, on the
+// streamed kernel 9.2 us and 1.1e-7, in parts of 32 7.6 us and 1.2e-7.
+template <int MB, int NJ, bool AFF, bool GEN, int PART>
 __global__ void __launch_bounds__(512, 2) tdc_conv1x1_block_kernel(const ConvKParams p) {
     using G = PixelGroup<NJ>;
     using px_t = typename G::reg_t;
@@ -139,14 +143,28 @@ __global__ void __launch_bounds__(512, 2) tdc_conv1x1_block_kernel(const ConvKPa
         }
         __builtin_amdgcn_sched_barrier(0);      // the requests stay in front of the MFMAs they run under
     };
-    f4_t acc[MB][NJ];
+    // The products of half a run, of one or of two runs are summed by themselves and then added to `acc`: those of single runs,
+    // where they are few MFMAs, a run later, when their sums have long left the matrix pipe.
+    constexpr bool LATE = PART == 16 && MB * NJ <= 4;
+    typedef f4_t Sums[MB][NJ];
+    Sums acc, s0, s1;
+    auto clear = [&](Sums &x) {
 #pragma unroll
-    for (int m = 0; m < MB; ++m)
+        for (int m = 0; m < MB; ++m)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) acc[m][j] = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
-    auto multiply = [&](Run &r) {
+            for (int j = 0; j < NJ; ++j) x[m][j] = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    auto add = [&](const Sums &x) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
+        for (int m = 0; m < MB; ++m)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[m][j] += x[m][j];
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // K-steps first ... first + count - 1 of a run; `fresh`: a part begins
+    auto multiply = [&](Run &r, Sums &sum, bool fresh, int first, int count) {
+#pragma unroll
+        for (int s = first; s < first + count; ++s) {
             if constexpr (AFF) {
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
@@ -157,26 +175,54 @@ __global__ void __launch_bounds__(512, 2) tdc_conv1x1_block_kernel(const ConvKPa
 #pragma unroll
             for (int m = 0; m < MB; ++m)
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.a[m][s], r.b[s][j], acc[m][j], 0, 0, 0);
+                for (int j = 0; j < NJ; ++j)
+                    sum[m][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(r.a[m][s], r.b[s][j], fresh && s == first ? (f4_t){0.0f, 0.0f, 0.0f, 0.0f} : sum[m][j], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
+    // the even and the odd runs of the wave; `last`: no odd run follows
+    auto even = [&](Run &r, bool last) {
+        if constexpr (PART == 0) {
+            multiply(r, acc, false, 0, 4);
+        } else if constexpr (PART == 8) {
+            multiply(r, s0, true, 0, 2);
+            multiply(r, s1, true, 2, 2);
+            add(s0);
+            add(s1);
+        } else {
+            multiply(r, s0, true, 0, 4);
+            if constexpr (LATE) add(s1);
+            else if (PART == 16 || last) add(s0);
+        }
+    };
+    auto odd = [&](Run &r) {
+        if constexpr (PART == 0 || PART == 8) {
+            even(r, true);
+        } else {
+            multiply(r, LATE ? s1 : s0, PART == 16, 0, 4);
+            add(s0);
+        }
+    };
+    clear(acc);
+    if constexpr (LATE) clear(s1);
     if (q_begin < q_end) {
         Run r0, r1;
         load(r0, q_begin);
         int q = q_begin;
         for (; q + 2 < q_end; q += 2) {
             load(r1, q + 1);
-            multiply(r0);
+            even(r0, false);
             load(r0, q + 2);
-            multiply(r1);
+            odd(r1);
         }
         if (q + 1 < q_end) {
             load(r1, q + 1);
-            multiply(r0);
-            multiply(r1);
+            even(r0, false);
+            odd(r1);
+            if constexpr (LATE) add(s1);
         } else {
-            multiply(r0);
+            even(r0, true);
+            if constexpr (LATE) add(s0);
         }
     }
 
@@ -275,21 +321,26 @@ __global__ void __launch_bounds__(512, 2) tdc_conv1x1_block_kernel(const ConvKPa
 
 using kernel_fn = void (*)(ConvKParams);
 
-template <int MB, int NJ>
+template <int MB, int NJ, int PART>
 static kernel_fn pick_block(bool aff, bool gen) {
-    return aff ? (gen ? static_cast<kernel_fn>(tdc_conv1x1_block_kernel<MB, NJ, true, true>) : tdc_conv1x1_block_kernel<MB, NJ, true, false>)
-               : (gen ? static_cast<kernel_fn>(tdc_conv1x1_block_kernel<MB, NJ, false, true>) : tdc_conv1x1_block_kernel<MB, NJ, false, false>);
+    return aff ? (gen ? static_cast<kernel_fn>(tdc_conv1x1_block_kernel<MB, NJ, true, true, PART>) : tdc_conv1x1_block_kernel<MB, NJ, true, false, PART>)
+               : (gen ? static_cast<kernel_fn>(tdc_conv1x1_block_kernel<MB, NJ, false, true, PART>) : tdc_conv1x1_block_kernel<MB, NJ, false, false, PART>);
+}
+
+template <int PART>
+static kernel_fn pick_block(int mb, int nj, bool aff, bool gen) {
+    if (nj == 4) return mb == 1 ? pick_block<1, 4, PART>(aff, gen) : mb == 2 ? pick_block<2, 4, PART>(aff, gen) : nullptr;
+    if (nj == 2) return mb == 1 ? pick_block<1, 2, PART>(aff, gen) : mb == 2 ? pick_block<2, 2, PART>(aff, gen) : nullptr;
+    return nullptr;
 }
 
 const void *block_kernel_function(const KernelId &k) {
-    kernel_fn fn = nullptr;
+    if (k.family != KernelId::BLOCK_1x1) return nullptr;
     const bool aff = k.p[2] != 0, gen = k.p[3] != 0;
-    if (k.family == KernelId::BLOCK_1x1) {
-        if (k.p[1] == 4)
-            fn = k.p[0] == 1 ? pick_block<1, 4>(aff, gen) : k.p[0] == 2 ? pick_block<2, 4>(aff, gen) : nullptr;
-        else if (k.p[1] == 2)
-            fn = k.p[0] == 1 ? pick_block<1, 2>(aff, gen) : k.p[0] == 2 ? pick_block<2, 2>(aff, gen) : nullptr;
-    }
+    const kernel_fn fn = k.p[4] == 0    ? pick_block<0>(k.p[0], k.p[1], aff, gen)
+                         : k.p[4] == 8  ? pick_block<8>(k.p[0], k.p[1], aff, gen)
+                         : k.p[4] == 16 ? pick_block<16>(k.p[0], k.p[1], aff, gen)
+                         : k.p[4] == 32 ? pick_block<32>(k.p[0], k.p[1], aff, gen) : nullptr;
     return reinterpret_cast<const void *>(fn);
 }
 

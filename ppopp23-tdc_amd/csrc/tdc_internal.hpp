@@ -188,7 +188,7 @@ enum : int { TAPS_GENERIC = 0, TAPS_1x1 = 1, TAPS_3x3 = 9, TAPS_3x3G = 10, TAPS_
 //               tdc_conv3x3_stream_rownb_kernel<CG, NB>               p = {CG, 1, 0, NB}   (NB = 2 or 4 pixel blocks per wave)
 //   STREAM_WINO tdc_wino3x3_stream_kernel<CG, MAXW>                   p = {CG, MAXW}
 //   BLOCK_WINO  tdc_wino3x3_block_kernel<MB, WN, PARTS>               p = {MB, WN, PARTS}
-//   BLOCK_1x1   tdc_conv1x1_block_kernel<MB, NJ, AFF, GEN>            p = {MB, NJ, AFF, GEN}
+//   BLOCK_1x1   tdc_conv1x1_block_kernel<MB, NJ, AFF, GEN, PART>      p = {MB, NJ, AFF, GEN, PART}
 //   SPLIT       tdc_conv_split_kernel<MB, NB, MODE, AFF>              p = {MB, NB, MODE, AFF}   (MODE: 0 flat, 1 window, 2 few channels)
 struct KernelId {
     enum Family : int { NONE = 0, STAGED = 1, STREAM_1x1 = 2, STREAM_3x3 = 3, STREAM_WINO = 4, BLOCK_1x1 = 5, BLOCK_WINO = 6, SPLIT = 7 };

@@ -358,7 +358,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
             return fail("tile.alg = 7 takes all input channels in one pass: cch = C rounded up to 16 * wk");
         g.gen = !flat || g.P < t.nb;
         g.units_image = g.gen ? g.P : ceil_div(g.P, t.nb);
-        if (t.tw != 1) return fail("tile.alg = 7 needs tw = 1");
+        if (t.tw != 1 && t.tw != 8 && t.tw != 16 && t.tw != 32) return fail("tile.alg = 7 needs tw = 1, 8, 16 or 32");
         const long long units = (long long)d.batch * g.units_image;
         if (units * g.units_image >= (1LL << 32) || units >= (1LL << 30)) return fail("batch too large for tile.alg = 7");
         g.units = (int)units;
@@ -798,7 +798,7 @@ KernelId kernel_id_for(const tdc_tile &t, int KH, int KW, int dilation, int stri
         // (`extras` here can only mean the input affine)
         if (KH != 1 || KW != 1 || t.mf != 16 || (t.mb != 1 && t.mb != 2) || (t.nb != 2 && t.nb != 4)) return k;
         k.family = KernelId::BLOCK_1x1;
-        k.p[0] = t.mb; k.p[1] = t.nb; k.p[2] = extras; k.p[3] = single_pixels;
+        k.p[0] = t.mb; k.p[1] = t.nb; k.p[2] = extras; k.p[3] = single_pixels; k.p[4] = t.tw >= 8 ? t.tw : 0;
         return k;
     }
     if (t.alg == 5) {
@@ -887,7 +887,7 @@ std::string kernel_name(const KernelId &k) {
             std::snprintf(buf, sizeof buf, "tdc_wino3x3_block_kernel<%d, %d, %s>", k.p[0], k.p[1], tf[k.p[2] != 0]);
             break;
         case KernelId::BLOCK_1x1:
-            std::snprintf(buf, sizeof buf, "tdc_conv1x1_block_kernel<%d, %d, %s, %s>", k.p[0], k.p[1], tf[k.p[2] != 0], tf[k.p[3] != 0]);
+            std::snprintf(buf, sizeof buf, "tdc_conv1x1_block_kernel<%d, %d, %s, %s, %d>", k.p[0], k.p[1], tf[k.p[2] != 0], tf[k.p[3] != 0], k.p[4]);
             break;
         case KernelId::SPLIT:
             std::snprintf(buf, sizeof buf, "tdc_conv_split_kernel<%d, %d, %d, %s>", k.p[0], k.p[1], k.p[2], tf[k.p[3] != 0]);
@@ -1174,6 +1174,8 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
         if (t.wk > 1) clk += 232.0 + 20.5 * g.waves * t.mb * t.nb * std::min(wgs_cu, 4.0);
         const double traffic = 4.0 * (d.batch * P * ((double)d.C + d.N) + (double)d.C * d.N);
         info.pred_us = 0.92 * (2.67 + clk / (m.clock_ghz * 1e3) + traffic / 11.95e6);
+        // (timed beside tw = 1 on 66 shapes: 1.013 on average, at most 1.07; 1.036, at most 1.09; 1.044, at most 1.11)
+        info.pred_us *= t.tw == 32 ? 1.013 : t.tw == 16 ? 1.036 : t.tw == 8 ? 1.044 : 1.0;
         info.pred_l2_bytes = 0.0;   // nothing is staged
         return true;
     }
@@ -1256,7 +1258,15 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
                             if (wm * wn * wk > 8 || wm * wn * wk == 2 || 16 * mb * wm > round_up(d.N, 16 * mb)) continue;
                             tdc_tile t{16, mb, nb, wm, wn, wk, round_up(d.C, 16 * wk), 1, 1, 0, 7};
                             Geometry g;
-                            if (make_geometry(d, t, g, nullptr, 0)) out.push_back(t);
+                            if (!make_geometry(d, t, g, nullptr, 0)) continue;
+                            out.push_back(t);
+                            // (the same with its sums in parts, where a wave has more channels than one of them; from 128 channels on
+                            //  parts of 8 are too many to have the smaller error)
+                            for (int part : {32, 16, 8})
+                                if (t.cch / wk > part && t.cch / wk < 16 * part) {
+                                    t.tw = part;
+                                    out.push_back(t);
+                                }
                         }
     }
     // streamed 3x3 candidates: 1, 2 or 4 groups of four channels per wave, a few shapes of the 16-pixel tile
@@ -1496,9 +1506,16 @@ static double rounding_variance(const tdc_conv_desc &d, const tdc_tile &t) {
     const bool wino = t.alg == 1 || t.alg == 5;
     const double n = wino ? d.C : (double)d.C * d.KH * d.KW;
     double chain = n / ((double)t.wk * t.ks);
-    if (t.alg == 3) chain = std::min(0.5 * t.cch / t.wk, n);
-    if (t.alg == 1 && t.tw == 0 && t.nb == 2) chain /= 1 + std::max(t.cch / (8 * t.wk) - 3, 0) / 8;   // (a part ends every eight steps but for the last two)
-    if ((t.alg == 4 || t.alg == 6) && t.nb == 1) chain *= 0.5;   // (these keep two accumulators)
+    if (t.alg == 3) chain = 0.5 * std::min((double)t.cch / t.wk, n);          // (two accumulators)
+    if (t.alg == 7 || (t.alg == 1 && t.tw == 0)) chain = std::min((double)t.cch / t.wk, n);
+    double parts = 1.0;                                          // ... of a wave's sum
+    if (t.alg == 1 && t.tw == 0 && t.nb == 2) parts += std::max(t.cch / (8 * t.wk) - 3, 0) / 8;   // (one ends every eight steps but for the last two)
+    if (t.alg == 7 && t.tw > 1) parts = std::max(chain / t.tw, 1.0);
+    if (parts > 1.0) {
+        const double v = 0.5 * (chain / parts + parts + t.wk - 1);
+        return wino ? 2.84 * v + 13.4 : v;
+    }
+    if ((t.alg == 4 || t.alg == 6) && t.nb == 1) chain *= 0.5;   // (likewise)
     const double v = 0.5 * (chain + n / (chain * t.ks) + (t.ks - 1));
     return wino ? 2.84 * v + 13.4 : v;
 }
@@ -1506,10 +1523,11 @@ static double rounding_variance(const tdc_conv_desc &d, const tdc_tile &t) {
 // The tiles a pick is made from.  Where the tiles of the other families would take a direct kernel with short chains (several
 // waves share few input channels), Winograd over the tiles of the whole batch is faster, 0.6 to 0.9 of the time, but its error
 // is up to 1.7 times as large (16 -> 112 @12 batch 48 0.9e-7 -> 1.5e-7), and with more input channels per chain than the staged
-// Winograd tile 1.4 times (128 -> 32 @105 batch 8 2.6e-7 -> 3.5e-7): it is taken only where its error is no larger than that of
-// the tile it takes the place of.
+// Winograd tile 1.4 times (128 -> 32 @105 batch 8 2.6e-7 -> 3.5e-7).  So is that of the register-blocked 1x1 kernel, up to 2.7 times
+// (304 -> 176 @53 1.1e-7 -> 3.1e-7 against five waves of 64 channels).  They are taken only where their error is no larger than
+// that of the tile they take the place of.
 static std::vector<tdc_tile_info> choices_within(const tdc_conv_desc &d, int tail_N, double &limit) {
-    auto batched = [](const tdc_tile &t) { return t.alg == 1 && t.tw == 0; };
+    auto batched = [](const tdc_tile &t) { return t.alg == 7 || (t.alg == 1 && t.tw == 0); };
     std::vector<tdc_tile_info> all, choices;
     const tdc_tile_info *plain = nullptr;
     const std::vector<tdc_tile> tiles = model_enumerate(d, tail_N);
@@ -1520,7 +1538,7 @@ static std::vector<tdc_tile_info> choices_within(const tdc_conv_desc &d, int tai
         all.push_back(info);
         if (!batched(t) && t.alg < 7 && (!plain || info.pred_us < plain->pred_us)) plain = &all.back();
     }
-    limit = plain ? 1.02 * rounding_variance(d, plain->tile) : 0.0;
+    limit = plain ? 1.06 * rounding_variance(d, plain->tile) : 0.0;   // (3 % of the error: where channels are padded to whole steps)
     for (const tdc_tile_info &info : all)
         if (!batched(info.tile) || rounding_variance(d, info.tile) <= limit) choices.push_back(info);
     return choices;

@@ -959,6 +959,23 @@ def test_every_blocked_1x1_tile(shape, stride):
         assert_close(out.cpu().numpy(), want_aff, f"input affine {shape} s{stride} {t}")
 
 
+@pytest.mark.parametrize("C", [16, 47, 80, 304])
+def test_blocked_1x1_sums_in_parts(C):
+    """The error of tiles with their sums in parts of 8, 16 or 32 channels stays within 1.3 times what chains of that length give:
+    2.5e-8 * sqrt((part + parts of a wave + waves) / 2) of the norm; single pixels (a stride) and groups, ragged channels."""
+    B, N, H, W = 3, 40, 9, 8
+    x, w = case(8660 + C, B, C, N, H, W, 1)
+    for stride in (1, 2):
+        exact = torch.nn.functional.conv2d(x.double(), w.double(), None, stride)
+        tiles = [t for t in tdc_amd.model_enumerate(tdc_amd.conv_desc(B, C, N, H, W, 1, 1, stride, 0)) if t.alg == 7 and t.tw > 1]
+        assert {t.tw for t in tiles} == {8, 16, 32} - {32 if C <= 32 else 0, 16 if C <= 16 else 0}
+        for t in tiles:
+            announce("blocked 1x1 in parts", C, stride, t)
+            got = torch.from_numpy(run_conv(x, w, stride=stride, tile=t)).double()
+            bound = 1.3 * 2.5e-8 * math.sqrt(0.5 * (t.tw + t.cch / t.wk / t.tw + t.wk))
+            assert (got - exact).norm() <= bound * exact.norm(), f"{C} s{stride} {t}"
+
+
 def test_blocked_1x1_with_images_far_apart():
     """tile.alg = 7 reaches the images of one wave through 32-bit offsets; images 2 GiB apart are launched one by one."""
     from ctypes import c_void_p

@@ -183,6 +183,15 @@ def test_batched_winograd_chains_are_no_longer_than_the_staged_ones(batch, C, N,
     assert t.alg == 1 and (t.wk * t.ks >= wk or (t.tw == 0 and t.nb == 2 and C >= 64 * wk))
 
 
+@pytest.mark.parametrize("batch,C,N,H,W,part", [(1, 304, 176, 53, 53, 32), (8, 160, 128, 28, 28, 32), (9, 80, 224, 18, 18, 16), (17, 41, 1385, 11, 25, 8),
+                                                (8, 704, 128, 14, 14, 704)])
+def test_blocked_1x1_chains_follow_the_kernel_they_replace(batch, C, N, H, W, part):
+    """The register-blocked 1x1 tiles sum in parts where the streamed tile that would run otherwise has short chains, and in one
+    chain where a staged tile with long ones would."""
+    t = tdc_amd.model_select(tdc_amd.conv_desc(batch, C, N, H, W, 1, 1, 1, 0)).tile
+    assert t.alg == 7 and (t.tw if t.tw > 1 else t.cch // t.wk) <= part and (t.tw == 1) == (part == C)
+
+
 def test_algorithmic_work_and_roofline_of_config1():
     i = tdc_amd.model_select(conv3(32, 32, 56))
     assert i.flops == 2 * 56 * 56 * 32 * 32 * 9 == 57802752
