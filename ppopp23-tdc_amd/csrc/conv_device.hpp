@@ -158,13 +158,18 @@ __device__ __forceinline__ ImageBase image_base(const ConvKParams &p, int img) {
     return b;
 }
 
-// A block of 16 channels x 16 pixels as plain fp32 sums over the weights as the caller gave them (p.w_raw, OIHW): for the rare
+// A block of 16 channels x 16 pixels as plain fp32 sums over the weights as the caller gave them (w_raw, OIHW): for the rare
 // outputs that a transform or a split of the operands cannot represent.  Lane (k = l / 16, n = l % 16) names channel `ch` (row n
 // of the block; past N: any) and output pixel (oy, ox) of image `img` (column n); it gets rows 4k .. 4k + 3 of its pixel.  Every
-// lane of the wave must call it.  Padding counts (0 * inf).  AFF: the input affine of a 1x1 convolution.
+// lane of the wave must call it, in a kernel whose only argument is the ConvKParams.  Padding counts (0 * inf).  AFF: the input affine of a 1x1 convolution.
 // Bound: latency, sixteen channels in flight; a wave in which it runs takes several times as long.
 template <bool AFF>
-__device__ __forceinline__ f4_t direct_block(const ConvKParams &p, int ch, int img, int oy, int ox) {
+__device__ __forceinline__ f4_t direct_block(int ch, int img, int oy, int ox) {
+    // (the kernel arguments are read here and now: kept for this from the start they would cost the kernel's ordinary path scalars)
+    typedef const __attribute__((address_space(4))) ConvKParams *args_t;
+    args_t args = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    const auto &p = *args;
     const int k = (threadIdx.x >> 4) & 3;
     const int taps = p.KH * p.KW, plane = p.H * p.W;
     const float *const w = p.w_raw + (size_t)min(ch, p.N - 1) * p.C * taps;

@@ -62,8 +62,10 @@ static __device__ __forceinline__ bool suspect(float sum) { return !(fabsf(sum) 
 //   SPLIT_FEW     at most four input channels (RGB stems): 8 bytes per pixel, a K octet is a pair of neighbouring taps.
 // Infinite and NaN operands (and finite ones above 3.39e38) make the split invalid: an infinity less itself is NaN.  Operands
 // below 2^-110 lose their last bits, because bf16 has no subnormals under 2^-133.  A wave that finds a NaN among its sums, or
-// one under 2^-90 other than zero, computes its outputs again, one by one, in fp32 from the unsplit input.  Channels of very small
-// or very large weights are packed times a power of two (pack_split_weights) and their sums multiplied by p.w_scale.
+// one under 2^-90 other than zero, computes plain fp32 sums of the unsplit operands for its block (direct_block) and takes those
+// for the sums in question: 512 -> 128 @28 batch 32 takes 31 us, with one NaN pixel 122, with nothing but NaN or sums below 2^-90
+// 310 (out of scalar fp32 sums for every output of such a wave 1600 and 3200).  Channels of very small or very large weights are packed times a power of two (pack_split_weights)
+// and their sums multiplied by p.w_scale.
 // AFF: per-channel affine (+ ReLU) on the input of a 1x1 convolution.
 // Bound: no single one.  512 -> 128 @28 batch 32 takes 26 us: 9 us of MFMAs at the 390 TFLOP/s of fp32 products that a bare MFMA
 // loop reaches, 13 us of memory traffic, and between them LDS reads (a half of the MFMA time at mb = 2), the splitting (6
@@ -338,36 +340,11 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
     const int ch_base = mblk0 * 16 + 4 * k;
     const bool scaled = __builtin_amdgcn_readfirstlane(__float_as_int(scaled_flag)) == 0x3f800000;
     const bool has_resid = p.resid != nullptr;
-    // One sum in fp32 from the unsplit input (see above): channel ch, pixel pix of image img.
-    auto exact_sum = [&](int ch, int img, int pix) {
-        const int oy = MODE == SPLIT_FLAT ? 0 : pix / p.Wo, ox = pix - oy * p.Wo;
-        const float *const src = p.in + (long long)img * p.in_bstride;
-        const __bf16 *const w = reinterpret_cast<const __bf16 *>(p.wpk) + (size_t)(ch >> 4) * steps_all * 1536 + (ch & 15) * 8;
-        float sum = 0.0f;
-        for (int c = 0; c < p.C; ++c) {
-            const int chunk = c / p.CCH, cc = c - chunk * p.CCH;
-            for (int tap = 0; tap < p.KH * p.KW; ++tap) {
-                const int kr = tap / p.KW, kx = tap - kr * p.KW;
-                float v;
-                if constexpr (MODE == SPLIT_FLAT) {
-                    v = src[(size_t)c * p.P + pix];
-                } else {
-                    const int y = oy * p.stride + kr * p.dil - p.pad, x = ox * p.stride + kx * p.dil - p.pad;
-                    const bool inside = (unsigned)y < (unsigned)p.H && (unsigned)x < (unsigned)p.W;
-                    v = inside ? src[(size_t)c * (p.H * p.W) + y * p.W + x] : 0.0f;   // (padding counts: 0 * inf)
-                }
-                if constexpr (AFF) {
-                    const float *const a = p.in_aff + (size_t)chunk * 2 * p.CCH + cc;
-                    v = v * a[0] + a[p.CCH];
-                    if (p.in_relu) v = fmaxf(v, 0.0f);
-                }
-                const int idx = MODE == SPLIT_FEW ? kr * p.fd_wtw.d + (kx >> 1) : (tap << no_shift) + (cc >> 3);
-                const int e = MODE == SPLIT_FEW ? (kx & 1) * 4 + c : cc & 7;
-                const __bf16 *const q = w + ((size_t)(chunk * ksteps + (idx >> 2)) * 1536 + (idx & 3) * 128 + e);
-                sum += v * ((float)q[0] + (float)q[512] + (float)q[1024]);
-            }
-        }
-        return sum;
+    // Plain sums for pixel j of this lane's group or block (see above), lane n naming channel `ch`.
+    auto plain = [&](int ch, int j) __attribute__((always_inline)) {
+        const Pixel px = pixel(MODE == SPLIT_FLAT ? 0 : j);
+        const int pix = MODE == SPLIT_FLAT ? px.pix + j : px.fresh ? 0 : px.pix;
+        return direct_block<AFF>(ch, px.img, pix / p.Wo, pix % p.Wo);
     };
 #pragma unroll
     for (int m = 0; m < MB; ++m)
@@ -384,21 +361,18 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
                 for (int i = 0; i < 4; ++i) bad |= suspect(lead[m][j][i]);
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
 #pragma unroll 1
-            for (int r = 0; r < MB * NB * 4; ++r) {
-                const int m = r / (4 * NB), j = (r >> 2) % NB, ch = ch_base + 16 * m + (r & 3);
-                const Pixel px = pixel(j);
-                if ((MODE == SPLIT_FLAT ? j < px.fresh : px.fresh != 0) || ch >= p.N) continue;
-                const int pix = px.pix + (MODE == SPLIT_FLAT ? j : 0);
-                float sum = exact_sum(ch, px.img, pix);
-                if (scaled) sum *= w_scale[ch];
-                if (p.bias) sum += p.bias[ch];
-                if (has_resid) sum += p.resid[(long long)px.img * p.resid_bstride + (long long)ch * p.P + pix];
-                if (p.relu) sum = fmaxf(sum, 0.0f);
-                p.out[(long long)px.img * p.out_bstride + (long long)ch * p.P + pix] = sum;
+            for (int r = 0; r < MB * NB; ++r) {
+                const f4_t sums = plain((mblk0 + r / NB) * 16 + n, r % NB);
+                const f4_t scale = scaled ? (f4_t)*reinterpret_cast<const f4u_t *>(w_scale + ch_base + 16 * (r / NB)) : (f4_t){1.0f, 1.0f, 1.0f, 1.0f};
+#pragma unroll
+                for (int x = 0; x < MB * NB; ++x)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float v = lead[x / NB][x % NB][i];
+                        lead[x / NB][x % NB][i] = x != r ? v : suspect(v) ? sums[i] : v * scale[i];
+                    }
             }
-            return;
-        }
-        if (__builtin_expect(scaled, 0)) {
+        } else if (__builtin_expect(scaled, 0)) {
 #pragma unroll
             for (int m = 0; m < MB; ++m) {
                 const f4_t s = *reinterpret_cast<const f4u_t *>(w_scale + ch_base + 16 * m);   // (padded to whole blocks)
@@ -483,17 +457,25 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
                 for (int j = 0; j < NB; ++j) bad |= suspect(v[i][j]);
             }
-            if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
-#pragma unroll 1
-                for (int r = 0; r < 2 * NB; ++r) {
-                    const float s = exact_sum(min(r < NB ? ch[0] : ch[1], p.N - 1), px.img, px.pix + r % NB);
-#pragma unroll
-                    for (int x = 0; x < 2 * NB; ++x) v[x / NB][x % NB] = x == r ? s : v[x / NB][x % NB];
-                }
-            }
+            float scale[2] = {1.0f, 1.0f};
             if (__builtin_expect(scaled, 0)) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) v[i] *= w_scale[ch[i]];
+                for (int i = 0; i < 2; ++i) scale[i] = w_scale[ch[i]];
+            }
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
+                // (rows 4k and 4k + 1 of the block of plain sums are the two of quarter k here)
+                const int row = slice + min(r0 + (n & 1), rows - 1) * p.WK;
+#pragma unroll 1
+                for (int j = 0; j < NB; ++j) {
+                    const f4_t sums = plain(mblk0 * 16 + 16 * (row >> 2) + (row & 3) + (n & 12), j);
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int x = 0; x < NB; ++x) v[i][x] = x != j ? v[i][x] : suspect(v[i][x]) ? sums[i] : v[i][x] * scale[i];
+                }
+            } else if (__builtin_expect(scaled, 0)) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) v[i] *= scale[i];
             }
             finish(v[0], ch[0], bv[0], rv[0]);
             if (r0 + 1 < rows) finish(v[1], ch[1], bv[1], rv[1]);

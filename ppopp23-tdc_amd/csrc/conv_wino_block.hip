@@ -353,7 +353,7 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
         if (__builtin_amdgcn_ballot_w64((left_out >> (4 * m) & 15) != 0) == 0) continue;
 #pragma unroll 1
         for (int e = 0; e < 4; ++e) {
-            const f4_t s = direct_block<false>(p, ch_base - 4 * k + 16 * m + n, img, min(oy + (e >> 1), p.Ho - 1), min(ox + (e & 1), p.Wo - 1));
+            const f4_t s = direct_block<false>(ch_base - 4 * k + 16 * m + n, img, min(oy + (e >> 1), p.Ho - 1), min(ox + (e & 1), p.Wo - 1));
 #pragma unroll
             for (int x = 0; x < 4; ++x) sums[x] = x == e ? s : sums[x];
         }

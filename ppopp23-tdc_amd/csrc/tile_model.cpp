@@ -224,6 +224,7 @@ static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geome
     g.grid_x = (int)gx;
     g.wslab_floats = t.wm * t.mb * g.ksteps * 3 * 256;
     g.scale_floats = 4 + g.grid_y * g.MT;
+    g.raw_floats = (size_t)d.N * d.C * g.taps;
     if ((long long)(packed_part_floats(g) + g.scale_floats) * 4 >= (1LL << 31)) return fail("packed weights exceed 2 GiB");
     g.channel_major = channel_major_order(4.0 * d.batch * d.C * d.H * d.W, 6.0 * d.N * d.C * g.taps, n_wg, g.grid_y);
     return true;

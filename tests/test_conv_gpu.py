@@ -1190,6 +1190,27 @@ def test_split_tiles_with_special_values(shape, K, stride, pad):
 
 @pytest.mark.parametrize("shape,K,stride,pad", [((2, 40, 36, 8, 8), 1, 1, 0), ((2, 70, 20, 7, 7), 1, 1, 0), ((2, 40, 36, 9, 9), 3, 2, 1),
                                                 ((2, 3, 20, 12, 12), 7, 2, 3)])
+def test_split_tiles_replace_only_the_sums_in_question(shape, K, stride, pad):
+    """One NaN pixel and one channel with a NaN weight: every output that sees neither keeps its bits (with at most four channels
+    taps go in pairs, and the last one's partner, of weight zero, puts outputs one column further in question: they stay close)."""
+    B, C, N, H, W = shape
+    g = seeded(8780)
+    x, w = torch.randn(B, C, H, W, generator=g), torch.randn(N, C, K, K, generator=g)
+    xn, wn = x.clone(), w.clone()
+    xn[0, 1, 3, 4], wn[5, 2, 0, 0] = float("nan"), float("nan")
+    hit = torch.isnan(torch.nn.functional.conv2d(xn.double(), wn.double(), None, stride, pad))
+    assert hit.any() and not hit.all()
+    for t in split_tiles(B, C, N, H, W, K, stride, pad):
+        announce("split replaced sums", shape, K, t)
+        plain, got = run_conv(x, w, stride=stride, pad=pad, tile=t), run_conv(xn, wn, stride=stride, pad=pad, tile=t)
+        assert np.isnan(got[hit.numpy()]).all()
+        if C > 4:
+            assert np.array_equal(got[~hit.numpy()], plain[~hit.numpy()]), f"{shape} {t}"
+        assert_close(got[~hit.numpy()], plain[~hit.numpy()], f"{shape} {t}")
+
+
+@pytest.mark.parametrize("shape,K,stride,pad", [((2, 40, 36, 8, 8), 1, 1, 0), ((2, 70, 20, 7, 7), 1, 1, 0), ((2, 40, 36, 9, 9), 3, 2, 1),
+                                                ((2, 3, 20, 12, 12), 7, 2, 3)])
 def test_split_tiles_with_channels_of_extreme_weights(shape, K, stride, pad):
     """Channels whose weights are next to nothing (also subnormal) or very large come out as accurate as the others, alone and
     beside an input whose own lower parts bf16 cannot hold; weights that replace others reach a captured graph."""
