@@ -29,6 +29,23 @@ struct Group<2> {
     }
 };
 
+// neither zero nor of a magnitude in [2^-90, infinity)
+static __device__ __forceinline__ bool suspect(float sum) {
+    const unsigned twice = __float_as_uint(sum) << 1;   // (without the sign)
+    return twice - 2u * 0x12800000u >= 2u * (0x7f800000u - 0x12800000u) && twice != 0;
+}
+// Whether any of several sums is: two and a half vector instructions each.  (The total may overflow without any of them being
+// infinite; then each is looked at in vain.)
+struct Range {
+    unsigned low = ~0u;
+    float total = 0.0f;
+    __device__ __forceinline__ void add(float sum) {
+        low = min(low, (__float_as_uint(sum) << 1) - 1u);   // (zero: the largest)
+        total += fabsf(sum);
+    }
+    __device__ __forceinline__ bool suspect() const { return low < 2u * 0x12800000u - 1u || !(total < __builtin_inff()); }
+};
+
 // x = h[0] + h[1] + h[2] exactly for finite x (8 bits of the mantissa each), as long as the lowest part stays representable.
 template <int N, typename V>
 static __device__ __forceinline__ void split3(const float (&x)[N], V (&h)[3]) {
@@ -40,8 +57,6 @@ static __device__ __forceinline__ void split3(const float (&x)[N], V (&h)[3]) {
         h[2][i] = (__bf16)(r1 - (float)h[1][i]);
     }
 }
-
-static __device__ __forceinline__ bool suspect(float sum) { return !(fabsf(sum) >= 0x1p-90f) && sum != 0.0f; }
 
 // ---------------------------------------------------------------------------
 // Every operand is split into three bf16 parts that add up to the fp32 value, and a product is the sum of the six partial
@@ -60,12 +75,13 @@ static __device__ __forceinline__ bool suspect(float sum) { return !(fabsf(sum) 
 //                 channels is staged and the K-steps run over its (tap, octet) pairs.  At stride 2 the even and the odd
 //                 columns lie in separate halves of a row, so neighbouring lanes read neighbouring slots.
 //   SPLIT_FEW     at most four input channels (RGB stems): 8 bytes per pixel, a K octet is a pair of neighbouring taps.
-// Infinite and NaN operands (and finite ones above 3.39e38) make the split invalid: an infinity less itself is NaN.  Operands
-// below 2^-110 lose their last bits, because bf16 has no subnormals under 2^-133.  A wave that finds a NaN among its sums, or
-// one under 2^-90 other than zero, computes plain fp32 sums of the unsplit operands for its block (direct_block) and takes those
-// for the sums in question: 512 -> 128 @28 batch 32 takes 31 us, with one NaN pixel 122, with nothing but NaN or sums below 2^-90
-// 310 (out of scalar fp32 sums for every output of such a wave 1600 and 3200).  Channels of very small or very large weights are packed times a power of two (pack_split_weights)
-// and their sums multiplied by p.w_scale.
+// Infinite and NaN operands (and finite ones above 3.39e38) make the split invalid: an infinity less itself is NaN.  Sums near
+// 3.4e38 can overflow in the leading product alone.  Operands below 2^-110 lose their last bits, because bf16 has no subnormals
+// under 2^-133.  A wave that finds an infinity or a NaN among its sums, or one under 2^-90 other than zero, computes plain fp32 sums
+// of the unsplit operands for its block (direct_block) and takes those for the sums in question: 512 -> 128 @28 batch 32 takes
+// 31 us, with one NaN pixel 122, with nothing but NaN or sums below 2^-90 310 (out of scalar fp32 sums for every output of such
+// a wave 1600 and 3200).  Channels of very small or very large weights are packed times a power of two (pack_split_weights) and
+// their sums multiplied by p.w_scale.
 // AFF: per-channel affine (+ ReLU) on the input of a 1x1 convolution.
 // Bound: no single one.  512 -> 128 @28 batch 32 takes 26 us: 9 us of MFMAs at the 390 TFLOP/s of fp32 products that a bare MFMA
 // loop reaches, 13 us of memory traffic, and between them LDS reads (a half of the MFMA time at mb = 2), the splitting (6
@@ -352,13 +368,14 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
         for (int j = 0; j < NB; ++j) lead[m][j] += rest[m][j];
 
     if (MODE != SPLIT_FLAT || p.WK == 1) {
-        bool bad = false;
+        Range range;
 #pragma unroll
         for (int m = 0; m < MB; ++m)
 #pragma unroll
             for (int j = 0; j < NB; ++j)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) bad |= suspect(lead[m][j][i]);
+                for (int i = 0; i < 4; ++i) range.add(lead[m][j][i]);
+        const bool bad = range.suspect();
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
 #pragma unroll 1
             for (int r = 0; r < MB * NB; ++r) {

@@ -1190,6 +1190,25 @@ def test_split_tiles_with_special_values(shape, K, stride, pad):
 
 @pytest.mark.parametrize("shape,K,stride,pad", [((2, 40, 36, 8, 8), 1, 1, 0), ((2, 70, 20, 7, 7), 1, 1, 0), ((2, 40, 36, 9, 9), 3, 2, 1),
                                                 ((2, 3, 20, 12, 12), 7, 2, 3)])
+def test_split_tiles_near_the_largest_numbers(shape, K, stride, pad):
+    """Sums that stay finite in fp32 are not lost to the split: inputs near 1e37 under a channel of tiny weights, which is packed
+    times a power of two, and a product just below the largest number whose leading parts alone exceed it."""
+    B, C, N, H, W = shape
+    g = seeded(8785)
+    x, w = (torch.rand(B, C, H, W, generator=g) + 0.5) * 4e37, (torch.rand(N, C, K, K, generator=g) + 0.5) * 1e-13
+    x[0, :, :, :4], w[1] = 0.0, 0.0
+    x[0, 1, :, :4], w[1, 1, K // 2, K // 2] = 3.385e38, 1.0045
+    want = torch.nn.functional.conv2d(x.double(), w.double(), None, stride, pad)
+    assert (want[:, 1] > 3.4e38).any() and (want < 3.4028e38).all()
+    for t in split_tiles(B, C, N, H, W, K, stride, pad):
+        announce("split near the largest numbers", shape, K, t)
+        got = torch.from_numpy(run_conv(x, w, stride=stride, pad=pad, tile=t)).double()
+        # (positive fp32 sums of at most 360 products, a rounding of 2^-24 each: 2.2e-5)
+        assert ((got - want).abs() <= 2.2e-5 * want).all(), f"{shape} {t}"
+
+
+@pytest.mark.parametrize("shape,K,stride,pad", [((2, 40, 36, 8, 8), 1, 1, 0), ((2, 70, 20, 7, 7), 1, 1, 0), ((2, 40, 36, 9, 9), 3, 2, 1),
+                                                ((2, 3, 20, 12, 12), 7, 2, 3)])
 def test_split_tiles_replace_only_the_sums_in_question(shape, K, stride, pad):
     """One NaN pixel and one channel with a NaN weight: every output that sees neither keeps its bits (with at most four channels
     taps go in pairs, and the last one's partner, of weight zero, puts outputs one column further in question: they stay close)."""
