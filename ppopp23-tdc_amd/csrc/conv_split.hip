@@ -46,6 +46,25 @@ struct Range {
     __device__ __forceinline__ bool suspect() const { return low < 2u * 0x12800000u - 1u || !(total < __builtin_inff()); }
 };
 
+// What a thread has met among the values it split: whether any is below 2^-110 but not zero and,
+// where factors of the weights ask for it, whether any reaches 2^20.  One and a half vector instructions a value (beside six for the split).
+struct Extremes {
+    unsigned low = ~0u;
+    float high = 0.0f;
+    template <int N>
+    __device__ __forceinline__ void add(const float (&x)[N], bool scaled) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) low = min(low, (__float_as_uint(x[i]) << 1) - 1u);   // (zero: the largest)
+        if (__builtin_expect(scaled, 0)) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) high = fmaxf(high, fabsf(x[i]));
+        }
+    }
+    __device__ __forceinline__ bool tiny() const { return low < 2u * 0x08800000u - 1u; }
+    __device__ __forceinline__ bool large() const { return high >= 0x1p20f; }
+};
+constexpr int EXTREMES_FLOATS = 8;   // of LDS, in front of everything else: one word per wave
+
 // x = h[0] + h[1] + h[2] exactly for finite x (8 bits of the mantissa each), as long as the lowest part stays representable.
 template <int N, typename V>
 static __device__ __forceinline__ void split3(const float (&x)[N], V (&h)[3]) {
@@ -78,10 +97,16 @@ static __device__ __forceinline__ void split3(const float (&x)[N], V (&h)[3]) {
 // Infinite and NaN operands (and finite ones above 3.39e38) make the split invalid: an infinity less itself is NaN.  Sums near
 // 3.4e38 can overflow in the leading product alone.  Operands below 2^-110 lose their last bits, because bf16 has no subnormals
 // under 2^-133.  A wave that finds an infinity or a NaN among its sums, or one under 2^-90 other than zero, computes plain fp32 sums
-// of the unsplit operands for its block (direct_block) and takes those for the sums in question: 512 -> 128 @28 batch 32 takes
-// 31 us, with one NaN pixel 122, with nothing but NaN or sums below 2^-90 310 (out of scalar fp32 sums for every output of such
-// a wave 1600 and 3200).  Channels of very small or very large weights are packed times a power of two (pack_split_weights) and
-// their sums multiplied by p.w_scale.
+// of the unsplit operands for the block that holds it (direct_block) and takes those for the sums in question: 512 -> 128 @28
+// batch 32 batch 32 takes 27 us, with one NaN pixel 78, with nothing but NaN or sums below 2^-90 296 (out of scalar fp32 sums for every output
+// of such a wave 1600 and 3200).  Channels of very small or very large weights are packed times a power of two
+// (pack_split_weights) and their sums multiplied by p.w_scale.
+// A sum of 2^-90 or more bears the lost bits of an operand below 2^-110 only while its partner stays under 2^20, and a zero may
+// stand for parts that all vanished.  So the threads note the inputs of either kind (Extremes) and the host the channels with
+// weights below 2^-110 (a negative factor): in question are also zeros where a tiny input or weight took part, sums of channels
+// packed down with a tiny input, and sums of channels with tiny weights beside a large input.  The look at every
+// input takes 1 to 2.5 % (512 -> 128 @28 batch 32 27.1 -> 27.7 us, 3x3 / stride 2 128 -> 128 @56 batch 64 98.1 -> 98.8, stem batch 32
+// 75.4 -> 77.4); one tiny pixel 28.3 us, a weight of 1e-40 in every channel 30.4.
 // AFF: per-channel affine (+ ReLU) on the input of a 1x1 convolution.
 // Bound: no single one.  512 -> 128 @28 batch 32 takes 26 us: 9 us of MFMAs at the 390 TFLOP/s of fp32 products that a bare MFMA
 // loop reaches, 13 us of memory traffic, and between them LDS reads (a half of the MFMA time at mb = 2), the splitting (6
@@ -100,7 +125,8 @@ template <int MB, int NB, int MODE, bool AFF>
 __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParams p) {
     using G = Group<NB>;
     using px_t = typename G::reg_t;
-    extern __shared__ __align__(16) float lds[];
+    extern __shared__ __align__(16) float lds_all[];
+    float *const lds = lds_all + EXTREMES_FLOATS;
     touch_kernel_arguments();
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -173,6 +199,10 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
     bf8_t *const lds8 = reinterpret_cast<bf8_t *>(lds);
     bf4_t *const lds4 = reinterpret_cast<bf4_t *>(lds);
     const int part8 = p.CS << no_shift;         // slots per part
+    Extremes extremes;
+    // whether any factor of the weights is not 1 (read from memory and not passed: new weights may come under a captured graph)
+    const bool scaled = __builtin_amdgcn_readfirstlane(__float_as_int(*p.w_scale)) == 0x3f800000;
+    const float *const w_scale = p.w_scale + 4;
     auto affine = [&](float (&v)[8], int chunk, int c) {
         if constexpr (AFF) {
             const float *const a = p.in_aff + (size_t)chunk * 2 * p.CCH + c;
@@ -213,6 +243,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
             for (int e = 0; e < 8; ++e) v[e] = group[e][x];
             affine(v, st, 8 * f_oct);
             split3(v, h);
+            extremes.add(v, scaled);
 #pragma unroll
             for (int s = 0; s < 3; ++s) lds8[s * part8 + f_oct * p.CS + x * (16 * p.WN) + f_unit] = h[s];
         }
@@ -249,6 +280,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
             for (int i = 0; i < EN; ++i) {
                 if (at[i] < 0) continue;
+                extremes.add(v[i], scaled);
                 if constexpr (MODE == SPLIT_FEW) {
                     bf4_t h[3];
                     split3(v[i], h);
@@ -271,9 +303,6 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
         for (int j = 0; j < NB; ++j) lead[m][j] = rest[m][j] = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
     const int steps_all = p.nchunks * ksteps;
-    // (requested here and looked at behind the last stage.  Read from memory and not passed: new weights may come under a captured graph)
-    const float scaled_flag = *p.w_scale;
-    const float *const w_scale = p.w_scale + 4;
     const int mblk0 = (by * p.WM + wm) * MB;
     struct A {
         bf8_t h[3];
@@ -340,6 +369,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
     if constexpr (MODE == SPLIT_FLAT) request_flat(0);
+    unsigned met_word = 0;
     for (int st = 0; st < p.nchunks; ++st) {
         if (st > 0) barrier();
         if constexpr (MODE == SPLIT_FLAT) {
@@ -348,14 +378,25 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
         } else {
             stage_window(st);
         }
+        if (st + 1 == p.nchunks) {
+            const unsigned met = (__builtin_amdgcn_ballot_w64(extremes.tiny()) ? 1u : 0u) | (__builtin_amdgcn_ballot_w64(extremes.large()) ? 2u : 0u);
+            if (lane == 0) reinterpret_cast<unsigned *>(lds_all)[wave] = met;
+        }
         barrier();
+        met_word = reinterpret_cast<const unsigned *>(lds_all)[lane & 7];   // (comes in under the MFMAs; only the last one counts)
         multiply(st);
     }
 
     // ---- results ---------------------------------------------------------------------------------------------------------
     const int ch_base = mblk0 * 16 + 4 * k;
-    const bool scaled = __builtin_amdgcn_readfirstlane(__float_as_int(scaled_flag)) == 0x3f800000;
+    const unsigned met = lane < 8 && 64 * lane < threads ? met_word : 0u;
+    const bool tiny_input = __builtin_amdgcn_ballot_w64((met & 1u) != 0) != 0, large_input = __builtin_amdgcn_ballot_w64((met & 2u) != 0) != 0;
     const bool has_resid = p.resid != nullptr;
+    // Whether the split may have lost what counts in a sum of a channel with factor `scale` (below 0: it has tiny weights).
+    auto in_question = [&](float sum, float scale) {
+        const bool tiny_weights = scale < 0.0f;
+        return suspect(sum) || (sum == 0.0f && (tiny_input || tiny_weights)) || (tiny_input && fabsf(scale) > 1.0f) || (large_input && tiny_weights);
+    };
     // Plain sums for pixel j of this lane's group or block (see above), lane n naming channel `ch`.
     auto plain = [&](int ch, int j) __attribute__((always_inline)) {
         const Pixel px = pixel(MODE == SPLIT_FLAT ? 0 : j);
@@ -376,25 +417,25 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
                 for (int i = 0; i < 4; ++i) range.add(lead[m][j][i]);
         const bool bad = range.suspect();
-        if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
+        if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0 || tiny_input || scaled, 0)) {
 #pragma unroll 1
             for (int r = 0; r < MB * NB; ++r) {
-                const f4_t sums = plain((mblk0 + r / NB) * 16 + n, r % NB);
-                const f4_t scale = scaled ? (f4_t)*reinterpret_cast<const f4u_t *>(w_scale + ch_base + 16 * (r / NB)) : (f4_t){1.0f, 1.0f, 1.0f, 1.0f};
+                const f4_t scale = scaled ? (f4_t)*reinterpret_cast<const f4u_t *>(w_scale + ch_base + 16 * (r / NB)) : (f4_t){1.0f, 1.0f, 1.0f, 1.0f};   // (padded to whole blocks)
+                f4_t v = lead[0][0];
 #pragma unroll
-                for (int x = 0; x < MB * NB; ++x)
+                for (int x = 1; x < MB * NB; ++x) v = x != r ? v : lead[x / NB][x % NB];
+                bool ask[4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float v = lead[x / NB][x % NB][i];
-                        lead[x / NB][x % NB][i] = x != r ? v : suspect(v) ? sums[i] : v * scale[i];
-                    }
-            }
-        } else if (__builtin_expect(scaled, 0)) {
+                for (int i = 0; i < 4; ++i) ask[i] = in_question(v[i], scale[i]);
 #pragma unroll
-            for (int m = 0; m < MB; ++m) {
-                const f4_t s = *reinterpret_cast<const f4u_t *>(w_scale + ch_base + 16 * m);   // (padded to whole blocks)
+                for (int i = 0; i < 4; ++i) v[i] *= fabsf(scale[i]);
+                if (__builtin_amdgcn_ballot_w64(ask[0] || ask[1] || ask[2] || ask[3]) != 0) {
+                    const f4_t sums = plain((mblk0 + r / NB) * 16 + n, r % NB);
 #pragma unroll
-                for (int j = 0; j < NB; ++j) lead[m][j] *= s;
+                    for (int i = 0; i < 4; ++i) v[i] = ask[i] ? sums[i] : v[i];
+                }
+#pragma unroll
+                for (int x = 0; x < MB * NB; ++x) lead[x / NB][x % NB] = x != r ? lead[x / NB][x % NB] : v;
             }
         }
     }
@@ -475,9 +516,13 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
                 for (int j = 0; j < NB; ++j) bad |= suspect(v[i][j]);
             }
             float scale[2] = {1.0f, 1.0f};
-            if (__builtin_expect(scaled, 0)) {
+            if (__builtin_expect(tiny_input || scaled, 0)) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) scale[i] = w_scale[ch[i]];
+                for (int i = 0; i < 2; ++i) {
+                    if (scaled) scale[i] = w_scale[ch[i]];
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) bad |= in_question(v[i][j], scale[i]);
+                }
             }
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
                 // (rows 4k and 4k + 1 of the block of plain sums are the two of quarter k here)
@@ -488,11 +533,11 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
 #pragma unroll
-                        for (int x = 0; x < NB; ++x) v[i][x] = x != j ? v[i][x] : suspect(v[i][x]) ? sums[i] : v[i][x] * scale[i];
+                        for (int x = 0; x < NB; ++x) v[i][x] = x != j ? v[i][x] : in_question(v[i][x], scale[i]) ? sums[i] : v[i][x] * fabsf(scale[i]);
                 }
             } else if (__builtin_expect(scaled, 0)) {
 #pragma unroll
-                for (int i = 0; i < 2; ++i) v[i] *= scale[i];
+                for (int i = 0; i < 2; ++i) v[i] *= fabsf(scale[i]);
             }
             finish(v[0], ch[0], bv[0], rv[0]);
             if (r0 + 1 < rows) finish(v[1], ch[1], bv[1], rv[1]);

@@ -69,10 +69,9 @@ struct Geometry {
     int gen = 0;                     // single pixels
     int unit_images = 0;             // images that the units of one wave (tile.alg = 8: workgroup) reach past the first one's
     // tile.alg = 8 (units are groups of nb pixels, or output rows): units per workgroup, octets of input channels per stage (as a
-    // power of two), K-steps per stage, taps (pairs
-    // of taps with at most four channels) per filter row.  win_L = window rows of one image, RS / CS = slots per row / octet.
+    // power of two), K-steps per stage, taps (pairs of taps with at most four channels) per filter row.  win_L = window rows of one image, RS / CS = slots per row / octet.
     int units_wg = 0, oct_shift = 0, ksteps = 0, row_taps = 1;
-    int scale_floats = 0;            // tile.alg = 8, behind the packed weights: 1 if any of the following is not 1, 3 unused, a factor per (padded) output channel
+    int scale_floats = 0;            // tile.alg = 8, behind the packed weights: 1 if any of the following is not 1, 3 unused, a factor per (padded) output channel, below 0 with tiny weights
     size_t raw_floats = 0;           // tile.alg = 8 and 1 with tw = 0, last: the weights as they came (see direct_block)
     int channel_major = 0;           // which logical workgroup order costs fewer L2 fills (see conv_staged.hip)
     double b_ways = 1.0;             // serialisation of the B-operand LDS read by bank conflicts (1 = none)

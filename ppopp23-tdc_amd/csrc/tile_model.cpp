@@ -211,6 +211,7 @@ static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geome
     }
     if (units * std::max(g.units_image, 16) >= (1LL << 32) || units >= (1LL << 30)) return fail("batch too large for tile.alg = 8");
     if ((long long)d.H * d.W * (g.c_pad + 8) * 4 >= (1LL << 31)) return fail("image too large for tile.alg = 8");
+    lds += 32;   // a word per wave in front, for what it met among the inputs
     if (lds > machine().lds_bytes_per_cu) return fail("tile needs more than 160 KiB of LDS");
     g.units = (int)units;
     g.lds_bytes = (int)lds;
@@ -538,13 +539,17 @@ static float from_bf16(uint16_t h) {
 // channels of two neighbouring taps of a filter row.
 // The last of the three parts is exact only above 2^-110, and sums below 2^-90 cost the kernel a second pass.  Trained networks
 // hold whole channels that weight decay left near nothing, so a channel whose largest weight is outside 2^-40 ... 2^20 is packed
-// times the power of two that brings it to 1, and its sums are multiplied by the inverse, which follows the weights.
+// times the power of two that brings it to 1, and its sums are multiplied by the inverse, which follows the weights.  The factor
+// is negative where a weight other than zero lies below 2^-110 as packed: the kernel then mistrusts zeros and large inputs.
 static float split_channel_scale(const tdc_conv_desc &d, const float *w, int n) {
     const size_t per = (size_t)d.C * d.KH * d.KW;
     float largest = 0.0f;
     for (size_t i = 0; i < per; ++i)
         if (std::isfinite(w[n * per + i])) largest = std::max(largest, std::fabs(w[n * per + i]));
-    return largest == 0.0f || (largest >= 0x1p-40f && largest <= 0x1p20f) ? 1.0f : std::ldexp(1.0f, std::ilogb(largest));
+    const float scale = largest == 0.0f || (largest >= 0x1p-40f && largest <= 0x1p20f) ? 1.0f : std::ldexp(1.0f, std::ilogb(largest));
+    for (size_t i = 0; i < per; ++i)
+        if (w[n * per + i] != 0.0f && std::fabs((double)w[n * per + i]) < 0x1p-110 * scale) return -scale;
+    return scale;
 }
 
 static void pack_split_weights(const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, const float *w, float *packed) {
@@ -555,7 +560,7 @@ static void pack_split_weights(const tdc_conv_desc &d, const tdc_tile &t, const 
         const float s = n < d.N ? split_channel_scale(d, w, n) : 1.0f;
         scales[4 + n] = s;
         shift[n] = -std::ilogb(s);
-        if (shift[n]) scales[0] = 1.0f;
+        if (s != 1.0f) scales[0] = 1.0f;
     }
     uint16_t *const dst = reinterpret_cast<uint16_t *>(packed);
     const bool few = t.tw != 0 && t.cch == 4;

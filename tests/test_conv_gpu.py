@@ -1262,6 +1262,32 @@ def test_split_tiles_with_channels_of_extreme_weights(shape, K, stride, pad):
         plan.close()
 
 
+@pytest.mark.parametrize("shape,K,stride,pad", [((2, 40, 36, 8, 8), 1, 1, 0), ((2, 70, 20, 7, 7), 1, 1, 0), ((2, 40, 36, 9, 9), 3, 2, 1),
+                                                ((2, 3, 20, 12, 12), 7, 2, 3)])
+def test_split_tiles_with_tiny_operands_beside_large_ones(shape, K, stride, pad):
+    """Operands below 2^-110, whose lower parts bf16 cannot hold, where the partner is so large that the sum is not small, and
+    where every part vanishes: products of both kinds meet nothing but zeros in some columns, and ordinary ones in others."""
+    B, C, N, H, W = shape
+    g = seeded(8788)
+    x, w = torch.rand(B, C, H, W, generator=g) + 0.5, torch.rand(N, C, K, K, generator=g) + 0.5
+    x[0, :, :, :4], x[1, :, :2] = 0.0, 0.0
+    x[0, 0, :, :2] = (torch.rand(H, 2, generator=g) + 1.0) * 2.0 ** 60      # beside tiny weights
+    x[0, 0, :, 2:4] = (torch.rand(H, 2, generator=g) + 1.0) * 2.0 ** -137   # beside large ones
+    x[1, 1, :2] = (torch.rand(2, W, generator=g) + 1.0)                     # beside weights that vanish when packed
+    for n, s in ((1, 2.0 ** -124), (2, 2.0 ** -137), (4, 2.0 ** 50), (5, 2.0 ** 19)):
+        w[n, 0] *= s
+    w[6] *= 2.0 ** 50
+    w[6, 1] *= 2.0 ** -140
+    want = torch.nn.functional.conv2d(x.double(), w.double(), None, stride, pad)
+    assert want.max() < 1e38
+    for t in split_tiles(B, C, N, H, W, K, stride, pad):
+        announce("split tiny beside large", shape, K, t)
+        got = torch.from_numpy(run_conv(x, w, stride=stride, pad=pad, tile=t)).double()
+        # (positive fp32 sums of at most 360 products, a rounding of 2^-24 each: 2.2e-5; a subnormal result is off by 2^-150 at
+        # every rounding)
+        assert ((got - want).abs() <= 2.2e-5 * want + 400 * 2.0 ** -150).all(), f"{shape} {t}"
+
+
 @pytest.mark.parametrize("K,stride,C", [(1, 1, 20), (3, 2, 20), (3, 2, 3)])
 def test_split_tiles_with_images_far_apart(K, stride, C):
     """tile.alg = 8 reaches the images of one workgroup through 32-bit offsets; images 2 GiB apart are launched one by one."""
