@@ -16,7 +16,9 @@ def _stream_ptr():
 # What a single small call costs is the host's work, not the kernel's (an 8.4 us pass around a 2.5 us kernel): the forwards
 # below read the raw stream handle instead of building a Stream object, compare a tensor with the expected shape in one
 # expression, leave the explaining to _dev_check where that fails, and hand ctypes plain integers.
-_raw_stream, _device = torch._C._cuda_getCurrentRawStream, torch._C._cuda_getDevice
+# (Private names, absent from a torch without GPU support, under which the host-only parts work all the same.)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
+_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
 _f32 = torch.float32
 
 

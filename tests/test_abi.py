@@ -3,6 +3,8 @@ points (the tile model) work without a GPU.  No convolution is computed here."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -32,6 +34,18 @@ def test_version_and_error_string():
     assert b"gfx950" in L.tdc_version()
     assert L.tdc_model_select(None, None) == _lib.TDC_ERR_INVALID
     assert b"null" in L.tdc_last_error_string()
+
+
+def test_import_under_a_torch_without_gpu_names():
+    """The host-only parts work where torch lacks the private names by which the forwards read the raw stream."""
+    code = ("import torch\n"
+            "for name in ('_cuda_getCurrentRawStream', '_cuda_getDevice'):\n"
+            "    if hasattr(torch._C, name): delattr(torch._C, name)\n"
+            "import tdc_amd\n"
+            "assert tdc_amd.model_select(tdc_amd.conv_desc(1, 32, 32, 56, 56, 3, 3, 1, 1)).tile.mf == 16\n")
+    env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "ppopp23-tdc_amd"))
+    run = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0, run.stderr
 
 
 def test_struct_layouts_match_the_header():
