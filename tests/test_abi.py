@@ -42,6 +42,7 @@ def test_import_under_a_torch_without_gpu_names():
             "for name in ('_cuda_getCurrentRawStream', '_cuda_getDevice'):\n"
             "    if hasattr(torch._C, name): delattr(torch._C, name)\n"
             "import tdc_amd\n"
+            "assert tdc_amd.Conv2dPlan and tdc_amd.partial_tucker2\n"
             "assert tdc_amd.model_select(tdc_amd.conv_desc(1, 32, 32, 56, 56, 3, 3, 1, 1)).tile.mf == 16\n")
     env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "ppopp23-tdc_amd"))
     run = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=300)
