@@ -42,8 +42,8 @@ def check_features(net, feats, what):
 @pytest.mark.parametrize("B,C,H,W", [(1, 1, 1, 4), (2, 3, 2, 4), (3, 5, 7, 8), (2, 37, 13, 12), (2, 6, 16, 260), (1, 2, 9, 6), (2, 3, 5, 7)])
 def test_max_pool_3x3_stride_2(B, C, H, W):
     """Rows of whole quads (the 128-bit kernel: one quad a row, one row, odd heights, a partly empty last block) and others; the
-    output as a tensor of its own, and as a slice of a wider buffer whose planes may leave it without 8-byte alignment.  Equal to
-    the reference bit for bit, negative values, infinities and signed zeros among them."""
+    output as a tensor of its own, and as a slice of a wider buffer.  Equal to the reference, negative values, infinities and
+    zeros among them."""
     g = torch.Generator().manual_seed(17)
     x = torch.randn(B, C, H, W, generator=g) - 1.0
     x.view(-1)[::7] = float("inf")
@@ -61,6 +61,23 @@ def test_max_pool_3x3_stride_2(B, C, H, W):
     assert torch.equal(out, want) and torch.equal(net.read(a), want)
     got = net.read(cat)
     assert torch.equal(got[:, 1:], want) and torch.equal(got[:, :1], want[:, :1])
+
+
+@pytest.mark.parametrize("B,C,H,W", [(1, 1, 1, 4), (2, 3, 2, 4), (3, 5, 7, 8), (2, 6, 16, 260)])
+def test_max_pool_kernels_agree_bit_for_bit(B, C, H, W):
+    """The kernel for whole quads against the one with an output per lane, which takes the same image with a column more (whose
+    windows are the same up to that column): windows of zeros of both signs, of negative values beside them, and NaN."""
+    g = torch.Generator().manual_seed(18)
+    values = torch.tensor([0.0, -0.0, -0.0, -1.0, float("nan"), -float("inf")])
+    x = values[torch.randint(0, 6, (B, C, H, W), generator=g)]
+    bits = []
+    for v in (x, torch.cat([x, torch.ones(B, C, H, 1)], 3)):
+        net = nets.Net(B, C, H, v.shape[3])
+        a = net.pool(0, "max", 3, 2, 1)
+        net.finalize(a)
+        bits.append(net(v.cuda()).cpu()[..., :W // 2].contiguous().view(torch.int32))
+    assert torch.equal(bits[0], bits[1])
+    assert W < 8 or (bits[0] == -2 ** 31).any() and (bits[0] == 0).any()
 
 
 def test_pool_and_concat_ops():
