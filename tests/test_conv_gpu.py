@@ -1055,6 +1055,32 @@ def test_batched_winograd_tiles_with_special_values(shape, pad):
         assert torch.allclose(got, want, rtol=1e-4, atol=0.0, equal_nan=True), f"{shape} {t}"
 
 
+@pytest.mark.parametrize("C,pad", [(20, 1), (20, 0), (88, 1)])
+def test_batched_winograd_with_images_far_apart(C, pad):
+    """Winograd tiles over the whole batch reach the images of one wave through 32-bit offsets, and check the requests of the last
+    channels against the end of the batch; images 2 GiB apart are launched one by one, each with an end and a first pixel of its own."""
+    from ctypes import c_void_p
+    B, N, H, W = 3, 24, 4, 5
+    x, w = case(8770 + C, B, C, N, H, W, 3)
+    want = ref.conv2d_c(x.numpy(), w.numpy(), pad=pad)
+    far = 1 << 29
+    buf = torch.empty(2 * far + C * H * W, device="cuda")
+    for b in range(B):
+        buf[b * far:b * far + C * H * W] = x[b].reshape(-1).cuda()
+    tiles = [t for t in tdc_amd.model_enumerate(tdc_amd.conv_desc(B, C, N, H, W, 3, 3, 1, pad)) if t.alg == 1 and t.tw == 0]
+    assert {t.mb for t in tiles} == {1, 2} and {t.wk for t in tiles} >= {1, 4} and (C <= 80 or any(t.nb == 2 for t in tiles))
+    for t in tiles:
+        announce("batched winograd far apart", C, pad, t)
+        plan = tdc_amd.Conv2dPlan(B, C, N, H, W, 3, 3, 1, pad, tile=t).set_weights(w)
+        out = torch.full(want.shape, float("nan"), device="cuda")
+        tdc_amd._lib.check(tdc_amd.lib().tdc_conv_forward_strided(
+            plan._h, c_void_p(buf.data_ptr()), far, None, 0, c_void_p(out.data_ptr()), 0,
+            c_void_p(torch.cuda.current_stream().cuda_stream)))
+        torch.cuda.synchronize()
+        plan.close()
+        assert_close(out.cpu().numpy(), want, f"{t}")
+
+
 def split_tiles(B, C, N, H, W, K, stride, pad, dil=1):
     """Every launchable tile of the split-operand kernel (tile.alg = 8), also those the model does not offer at this size."""
     d = tdc_amd.conv_desc(B, C, N, H, W, K, K, stride, pad, dil)
