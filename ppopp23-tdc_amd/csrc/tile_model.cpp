@@ -1532,45 +1532,58 @@ static double rounding_variance(const tdc_conv_desc &d, const tdc_tile &t) {
 // Winograd tile 1.4 times (128 -> 32 @105 batch 8 2.6e-7 -> 3.5e-7).  So is that of the register-blocked 1x1 kernel, up to 2.7 times
 // (304 -> 176 @53 1.1e-7 -> 3.1e-7 against five waves of 64 channels).  They are taken only where their error is no larger than
 // that of the tile they take the place of.
-static std::vector<tdc_tile_info> choices_within(const tdc_conv_desc &d, int tail_N, double &limit) {
+// (Prices and places in `tiles` only: ten thousand tdc_tile_info cost a third of the time of a selection.)
+struct Choice {
+    int tile;
+    double us, handicap;
+};
+static std::vector<Choice> choices_within(const tdc_conv_desc &d, int tail_N, const std::vector<tdc_tile> &tiles, double &limit) {
     auto batched = [](const tdc_tile &t) { return t.alg == 7 || (t.alg == 1 && t.tw == 0); };
-    std::vector<tdc_tile_info> all, choices;
-    const tdc_tile_info *plain = nullptr;
-    const std::vector<tdc_tile> tiles = model_enumerate(d, tail_N);
-    all.reserve(tiles.size());
-    for (const tdc_tile &t : tiles) {
+    std::vector<Choice> choices;
+    choices.reserve(tiles.size());
+    int plain = -1;
+    double plain_us = 0.0;
+    for (int i = 0; i < (int)tiles.size(); ++i) {
         tdc_tile_info info;
-        if (!model_evaluate(d, t, info, nullptr, tail_N)) continue;
-        all.push_back(info);
-        if (!batched(t) && t.alg < 7 && (!plain || info.pred_us < plain->pred_us)) plain = &all.back();
+        if (!model_evaluate(d, tiles[i], info, nullptr, tail_N)) continue;
+        choices.push_back({i, info.pred_us, staged_winograd_handicap(info)});
+        if (batched(tiles[i]) || tiles[i].alg >= 7 || (plain >= 0 && info.pred_us >= plain_us)) continue;
+        plain = i;
+        plain_us = info.pred_us;
     }
-    limit = plain ? 1.06 * rounding_variance(d, plain->tile) : 0.0;   // (3 % of the error: where channels are padded to whole steps)
-    for (const tdc_tile_info &info : all)
-        if (!batched(info.tile) || rounding_variance(d, info.tile) <= limit) choices.push_back(info);
+    limit = plain >= 0 ? 1.06 * rounding_variance(d, tiles[plain]) : 0.0;   // (3 % of the error: where channels are padded to whole steps)
+    choices.erase(std::remove_if(choices.begin(), choices.end(), [&](const Choice &c) { return batched(tiles[c.tile]) && rounding_variance(d, tiles[c.tile]) > limit; }), choices.end());
     return choices;
 }
 std::vector<tdc_tile_info> model_choices(const tdc_conv_desc &d, int tail_N) {
     double limit;
-    return choices_within(d, tail_N, limit);
+    const std::vector<tdc_tile> tiles = model_enumerate(d, tail_N);
+    std::vector<tdc_tile_info> infos;
+    for (const Choice &c : choices_within(d, tail_N, tiles, limit)) {
+        infos.emplace_back();
+        if (!model_evaluate(d, tiles[c.tile], infos.back(), nullptr, tail_N)) infos.pop_back();
+    }
+    return infos;
 }
 
 bool model_select(const tdc_conv_desc &d, tdc_tile_info &best, std::string *why, int tail_N) {
     if (!check_desc(d, why)) return false;
     double limit;
-    const std::vector<tdc_tile_info> cands = choices_within(d, tail_N, limit);
-    const bool batched = std::any_of(cands.begin(), cands.end(), [](const tdc_tile_info &i) { return i.tile.alg == 1 && i.tile.tw == 0; });
-    bool have = false;
+    const std::vector<tdc_tile> tiles = model_enumerate(d, tail_N);
+    const std::vector<Choice> cands = choices_within(d, tail_N, tiles, limit);
+    const bool batched = std::any_of(cands.begin(), cands.end(), [&](const Choice &c) { return tiles[c.tile].alg == 1 && tiles[c.tile].tw == 0; });
+    const Choice *pick = nullptr;
     double best_us = 0.0;
-    for (const tdc_tile_info &info : cands) {
+    for (const Choice &c : cands) {
         // (the handicap takes the pick from a staged tile, but not to a kernel with a larger error)
-        if (batched && info.tile.alg < 7 && rounding_variance(d, info.tile) > limit) continue;
-        const double us = info.pred_us * (batched ? staged_winograd_handicap(info) : 1.0);
-        if (!have || us < best_us) {
-            best = info;
+        if (batched && tiles[c.tile].alg < 7 && rounding_variance(d, tiles[c.tile]) > limit) continue;
+        const double us = c.us * (batched ? c.handicap : 1.0);
+        if (!pick || us < best_us) {
+            pick = &c;
             best_us = us;
-            have = true;
         }
     }
+    const bool have = pick && model_evaluate(d, tiles[pick->tile], best, nullptr, tail_N);
     if (!have && why) {
         // say why the plainest tile cannot be launched: that is the limit the shape runs into
         const tdc_tile plain{16, 1, 1, 1, 1, 1, 4, 1, 1, 0, 0};
