@@ -5,30 +5,6 @@
 
 namespace tdc {
 
-typedef float f2_t __attribute__((ext_vector_type(2)));
-// (pixel groups need not be 16-byte aligned: images with an odd number of pixels, channel slices)
-typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
-typedef float f2u_t __attribute__((ext_vector_type(2), aligned(4)));
-
-template <int NJ>
-struct PixelGroup;
-template <>
-struct PixelGroup<4> {
-    using mem_t = f4u_t;
-    using reg_t = f4_t;
-    static __device__ __forceinline__ reg_t load(__amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
-        return __builtin_bit_cast(reg_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, 0));
-    }
-};
-template <>
-struct PixelGroup<2> {
-    using mem_t = f2u_t;
-    using reg_t = f2_t;
-    static __device__ __forceinline__ reg_t load(__amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
-        return __builtin_bit_cast(reg_t, __builtin_amdgcn_raw_buffer_load_b64(rsrc, voff, soff, 0));
-    }
-};
-
 // ---------------------------------------------------------------------------
 // One wave computes 16*MB output channels x 16*NJ pixels on v_mfma_f32_16x16x4_f32, operands straight from global memory
 // into registers, one run of 16 input channels ahead of the MFMAs.  The batch is flattened: pixel groups are counted
@@ -38,8 +14,8 @@ struct PixelGroup<2> {
 //     would run past the end of its image starts earlier and leaves the pixels of its neighbour alone.  GEN: pixels one by
 //     one (strided convolutions, images of fewer than NJ pixels).
 //   * A operand: the packed weights of the streamed kernel, [16 channels][run][lane][4], one 128-bit request for four K-steps.
-//   * MB*NJ MFMAs per K-step from 1 + MB/4 requests: at MB = NJ = 4 the address path of a compute unit is busy a quarter of
-//     the time the matrix pipe is, where the 16x16 blocks of the streamed kernel need it twice as long as the pipe.
+//   * MB*NJ MFMAs per K-step from 1 + MB/4 requests: at MB = 2, NJ = 4 the address path of a compute unit is busy three eighths
+//     of the time the matrix pipe is, where the 16x16 blocks of the streamed kernel need it twice as long as the pipe.
 // A workgroup is WM x WN waves over channels and pixels (they share operands through the L1), times WK waves that split
 // the input channels and add their partial blocks through LDS in slice order.
 // AFF: per-channel affine (+ ReLU) on the input, in registers.

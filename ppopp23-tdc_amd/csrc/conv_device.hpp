@@ -1,6 +1,6 @@
 // Device-side pieces shared by the convolution kernels: MFMA wrappers, the multiply-high division, the common
 // epilogue of a lane that holds four channels of a pixel, the kernel-argument touch, and the time-stamp macros of
-// the profiling build.  Included by conv_staged.hip and conv_stream.hip only.
+// the profiling build.  Included by every conv_*.hip with kernels.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -34,9 +34,33 @@
 
 namespace tdc {
 
+typedef float f2_t __attribute__((ext_vector_type(2)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef float f16_t __attribute__((ext_vector_type(16)));
+// (for places that need not be aligned: images with an odd number of pixels, channel slices)
+typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f2u_t __attribute__((ext_vector_type(2), aligned(4)));
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
+
+// N neighbouring pixels of a plane, one request.
+template <int N>
+struct PixelGroup;
+template <>
+struct PixelGroup<4> {
+    using mem_t = f4u_t;
+    using reg_t = f4_t;
+    static __device__ __forceinline__ reg_t load(__amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
+        return __builtin_bit_cast(reg_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, 0));
+    }
+};
+template <>
+struct PixelGroup<2> {
+    using mem_t = f2u_t;
+    using reg_t = f2_t;
+    static __device__ __forceinline__ reg_t load(__amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
+        return __builtin_bit_cast(reg_t, __builtin_amdgcn_raw_buffer_load_b64(rsrc, voff, soff, 0));
+    }
+};
 
 template <int MF>
 struct Mfma;

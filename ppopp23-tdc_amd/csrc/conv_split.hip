@@ -5,29 +5,6 @@ namespace tdc {
 
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf4_t __attribute__((ext_vector_type(4)));
-typedef float f2_t __attribute__((ext_vector_type(2)));
-// (pixel groups need not be aligned: images with an odd number of pixels, channel slices)
-typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
-typedef float f2u_t __attribute__((ext_vector_type(2), aligned(4)));
-
-template <int NB>
-struct Group;
-template <>
-struct Group<4> {
-    using mem_t = f4u_t;
-    using reg_t = f4_t;
-    static __device__ __forceinline__ reg_t load(__amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
-        return __builtin_bit_cast(reg_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voff, soff, 0));
-    }
-};
-template <>
-struct Group<2> {
-    using mem_t = f2u_t;
-    using reg_t = f2_t;
-    static __device__ __forceinline__ reg_t load(__amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
-        return __builtin_bit_cast(reg_t, __builtin_amdgcn_raw_buffer_load_b64(rsrc, voff, soff, 0));
-    }
-};
 
 // neither zero nor of a magnitude in [2^-90, infinity)
 static __device__ __forceinline__ bool suspect(float sum) {
@@ -98,7 +75,7 @@ static __device__ __forceinline__ void split3(const float (&x)[N], V (&h)[3]) {
 // 3.4e38 can overflow in the leading product alone.  Operands below 2^-110 lose their last bits, because bf16 has no subnormals
 // under 2^-133.  A wave that finds an infinity or a NaN among its sums, or one under 2^-90 other than zero, computes plain fp32 sums
 // of the unsplit operands for the block that holds it (direct_block) and takes those for the sums in question: 512 -> 128 @28
-// batch 32 batch 32 takes 27 us, with one NaN pixel 78, with nothing but NaN or sums below 2^-90 296 (out of scalar fp32 sums for every output
+// batch 32 takes 27 us, with one NaN pixel 78, with nothing but NaN or sums below 2^-90 296 (out of scalar fp32 sums for every output
 // of such a wave 1600 and 3200).  Channels of very small or very large weights are packed times a power of two
 // (pack_split_weights) and their sums multiplied by p.w_scale.
 // A sum of 2^-90 or more bears the lost bits of an operand below 2^-110 only while its partner stays under 2^20, and a zero may
@@ -123,7 +100,7 @@ enum : int { SPLIT_FLAT = 0, SPLIT_WINDOW = 1, SPLIT_FEW = 2 };
 
 template <int MB, int NB, int MODE, bool AFF>
 __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParams p) {
-    using G = Group<NB>;
+    using G = PixelGroup<NB>;
     using px_t = typename G::reg_t;
     extern __shared__ __align__(16) float lds_all[];
     float *const lds = lds_all + EXTREMES_FLOATS;
@@ -145,7 +122,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
     const int threads = 64 * p.WM * p.WN;
     const unsigned HW4 = (unsigned)(p.H * p.W) * 4u;
     // (see Geometry) slots per output column, octets per stage as a power of two, K-steps per stage
-    const int ss = p.KS, no_shift = p.win_nreq, ksteps = p.win_ns, half = p.win_off;
+    const int ss = p.slots_col, no_shift = p.oct_shift, ksteps = p.ksteps, half = p.odd_columns;
 
     // first unit (group of NB pixels / output row) and first image of the workgroup; column tile of a window
     const int ty = MODE == SPLIT_FLAT ? bx : fdiv(bx, p.fd_ntx);

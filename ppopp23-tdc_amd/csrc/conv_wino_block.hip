@@ -5,9 +5,6 @@
 
 namespace tdc {
 
-typedef float f2_t __attribute__((ext_vector_type(2)));
-typedef float f2u_t __attribute__((ext_vector_type(2), aligned(4)));
-
 // ---------------------------------------------------------------------------
 // 3x3 / stride 1 / dilation 1 / pad <= 1.  The 2x2-pixel output tiles of the whole batch form one row; a wave owns 16 of
 // them (one per pixel lane, so neither image edges nor small images leave lanes idle) and 16*MB output channels.

@@ -21,7 +21,6 @@
 
 namespace tdc {
 
-typedef float f2_t __attribute__((ext_vector_type(2)));
 typedef unsigned u2_t __attribute__((ext_vector_type(2)));
 
 // lane j of a 16-lane row takes the value of lane j + 1 / j + 2 (zero past the row)

@@ -377,8 +377,8 @@ static void refresh_launch_params(tdc_conv_plan *plan) {
     kp.fd_wn = make_fastdiv(plan->tile.wn);
     kp.fd_ks = make_fastdiv(g.ks);
     if (plan->tile.alg == 8) {
-        kp.KS = d.stride;
-        kp.win_nreq = g.oct_shift; kp.win_ns = g.ksteps;
+        kp.slots_col = d.stride;
+        kp.oct_shift = g.oct_shift; kp.ksteps = g.ksteps; kp.odd_columns = g.odd_columns;
         kp.fd_npx = make_fastdiv(std::max(g.nrows * g.ncols, 1));
         kp.fd_hww = make_fastdiv(std::max(g.ncols, 1));
         kp.fd_wtw = make_fastdiv(g.row_taps);

@@ -69,9 +69,12 @@ struct Geometry {
     int gen = 0;                     // single pixels
     int unit_images = 0;             // images that the units of one wave (tile.alg = 8: workgroup) reach past the first one's
     // tile.alg = 8 (units are groups of nb pixels, or output rows): units per workgroup, octets of input channels per stage (as a
-    // power of two), K-steps per stage, taps (pairs of taps with at most four channels) per filter row.  win_L = window rows of one image, RS / CS = slots per row / octet.
-    int units_wg = 0, oct_shift = 0, ksteps = 0, row_taps = 1;
-    int scale_floats = 0;            // tile.alg = 8, behind the packed weights: 1 if any of the following is not 1, 3 unused, a factor per (padded) output channel, below 0 with tiny weights
+    // power of two), K-steps per stage, taps (pairs of taps with at most four channels) per filter row, where the odd columns of
+    // a row start.  win_L = window rows of one image, RS / CS = slots per row / octet.
+    int units_wg = 0, oct_shift = 0, ksteps = 0, row_taps = 1, odd_columns = 0;
+    // tile.alg = 8, behind the packed weights: 1 if any of the following is not 1, 3 unused, a factor per (padded) output channel,
+    // below 0 for channels with tiny weights
+    int scale_floats = 0;
     size_t raw_floats = 0;           // tile.alg = 8 and 1 with tw = 0, last: the weights as they came (see direct_block)
     int channel_major = 0;           // which logical workgroup order costs fewer L2 fills (see conv_staged.hip)
     double b_ways = 1.0;             // serialisation of the B-operand LDS read by bank conflicts (1 = none)
@@ -136,7 +139,11 @@ struct ConvKParams {
     int TW, TH, ntx;
     int WM, WN, WK;
     int CCH, nchunks, CPW;
-    int KS, cps;               // slices across workgroups, passes per slice
+    union {
+        int KS;                // slices across workgroups
+        int slots_col;         // tile.alg = 8: LDS slots per output column
+    };
+    int cps;                   // passes per slice
     int WL;                    // loader waves (the last WL of the workgroup)
     int grid_x, grid_y;        // pixel tiles, channel tiles
     int n_wg;                  // grid_x * grid_y * batch * KS
@@ -154,7 +161,11 @@ struct ConvKParams {
     int head_mblk, head_npb;   // ... 16-row blocks of its output (the core's input channels), 16-pixel blocks of the window
     int head_ww, head_wq;      // ... window width (TW + 2) and pixels ((TH + 2) * (TW + 2))
     int head_ld, head_f_off;   // ... row stride and offset (floats) of its output in LDS
-    int win_rows, win_L, win_nreq, win_ns, win_off;   // tile.alg = 6: the wave-private input window in LDS (see Geometry)
+    int win_rows, win_L;       // tile.alg = 6: the wave-private input window in LDS (see Geometry); tile.alg = 8: window rows of one image
+    union {
+        struct { int win_nreq, win_ns, win_off; };
+        struct { int oct_shift, ksteps, odd_columns; };   // tile.alg = 8 (see Geometry): the odd columns of a row at stride 2 start here
+    };
     FastDiv fd_winL;
     FastDiv fd_hww, fd_hnpb;
     FastDiv fd_npx;            // 16-pixel blocks per tile

@@ -203,8 +203,8 @@ static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geome
         g.ncols = (int)columns;
         g.nrows = (int)rows;
         g.win_L = (int)image_rows;
-        g.win_off = (g.ncols + 1) / 2;
-        g.RS = !few && d.stride == 2 ? 2 * g.win_off : g.ncols;
+        g.odd_columns = (g.ncols + 1) / 2;
+        g.RS = !few && d.stride == 2 ? 2 * g.odd_columns : g.ncols;
         g.CS = g.nrows * g.RS;
         lds = few ? 3LL * g.CS * 8 : (3LL * g.CS * 16) << g.oct_shift;
         cols = ceil_div(g.Wo, g.TW);
@@ -388,7 +388,6 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         g.TW = 2 * g.TWt;
         g.TH = 2 * g.THt;
         g.PT = 4 * lanes;   // pixels the workgroup's lanes stand for
-    } else if (wino_batch) {
     } else if (t.alg == 5) {
         g.ktaps = 16;
         g.TW = 28;
@@ -398,7 +397,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
         g.PT = t.mf * t.nb * t.wn;
         g.TW = std::min(g.PT, g.P);
         g.TH = 1;
-    } else {
+    } else if (!wino_batch) {
         g.PT = t.mf * t.nb * t.wn;
         // (the streamed 1x1 kernel walks the output in runs of 16 consecutive pixels, whatever the image's rows are)
         const bool runs = t.alg == 3 && !flat;
@@ -730,7 +729,7 @@ double *mc_field(int i) {
 
 struct CompiledKernel { const char *name; int regs, sgprs, waves; };
 // hipcc's resource report for the convolution kernels of this build (written by the Makefile from the compile of
-// conv_staged.hip and conv_stream.hip): name, VGPRs + AGPRs per lane, scalar registers, waves per SIMD.
+// every conv_*.hip with kernels): name, VGPRs + AGPRs per lane, scalar registers, waves per SIMD.
 static const CompiledKernel compiled_kernels[] = {
 #include "kernel_registers.inc"
 };
@@ -1136,7 +1135,8 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
         // the L2 need, + LDS reads + the end of every workgroup + launch and memory traffic.  Fitted to 4500 timed tiles of 90
         // 1x1 shapes (6 % mean error, 2.2 % mean loss of the pick within the family) and 4100 tiles of 60 3x3 and 7x7 shapes
         // (6 %, 2.5 %).  The factor in front of the 1x1 and 3x3 forms: as measured, the formulas of the other families are 15 to
-        // 25 % kind to the launches this one competes with (7 us and more), those for the 7x7 stems are not.  At 0.91 no 1x1
+        // 25 % kind to the launches this one competes with (7 us and more; most of all those of the staged kernel at stride 2: 128 -> 128
+        // @28 batch 32 23.5 us for 34.6, 256 -> 256 @14 22.8 for 41.4), those for the 7x7 stems are not.  At 0.91 no 1x1
         // shape of the 90 loses more than 2 % to its former pick and the mean gain is 9 % (0.85: 10 %, but three lose 8 to 12 %;
         // 1.0: 6 %); the lines fall at 7 to 9 us from 64 channels up, and about 25 us at 3x3 / stride 2.
         const bool flat = t.tw == 0;
