@@ -23,18 +23,17 @@ struct Range {
     __device__ __forceinline__ bool suspect() const { return low < 2u * 0x12800000u - 1u || !(total < __builtin_inff()); }
 };
 
-// What a thread has met among the values it split: whether any is below 2^-110 but not zero and,
-// where factors of the weights ask for it, whether any reaches 2^20.  One and a half vector instructions a value (beside six for the split).
+// What a thread has met among the values it split: whether any is below 2^-110 but not zero, and whether any reaches 2^20.  Two
+// vector instructions a value (beside six for the split).
 struct Extremes {
     unsigned low = ~0u;
     float high = 0.0f;
     template <int N>
-    __device__ __forceinline__ void add(const float (&x)[N], bool scaled) {
+    __device__ __forceinline__ void add(const float (&x)[N]) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) low = min(low, (__float_as_uint(x[i]) << 1) - 1u);   // (zero: the largest)
-        if (__builtin_expect(scaled, 0)) {
-#pragma unroll
-            for (int i = 0; i < N; ++i) high = fmaxf(high, fabsf(x[i]));
+        for (int i = 0; i < N; i += 2) {
+            low = min(min(low, (__float_as_uint(x[i]) << 1) - 1u), (__float_as_uint(x[i + 1]) << 1) - 1u);   // (zero: the largest)
+            asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(high) : "v"(high), "v"(x[i]), "v"(x[i + 1]));   // (fmaxf would quiet each value first)
         }
     }
     __device__ __forceinline__ bool tiny() const { return low < 2u * 0x08800000u - 1u; }
@@ -75,15 +74,16 @@ static __device__ __forceinline__ void split3(const float (&x)[N], V (&h)[3]) {
 // 3.4e38 can overflow in the leading product alone.  Operands below 2^-110 lose their last bits, because bf16 has no subnormals
 // under 2^-133.  A wave that finds an infinity or a NaN among its sums, or one under 2^-90 other than zero, computes plain fp32 sums
 // of the unsplit operands for the block that holds it (direct_block) and takes those for the sums in question: 512 -> 128 @28
-// batch 32 takes 27 us, with one NaN pixel 78, with nothing but NaN or sums below 2^-90 296 (out of scalar fp32 sums for every output
+// batch 32 takes 28 us, with one NaN pixel 79, with nothing but NaN or sums below 2^-90 296 (out of scalar fp32 sums for every output
 // of such a wave 1600 and 3200).  Channels of very small or very large weights are packed times a power of two
 // (pack_split_weights) and their sums multiplied by p.w_scale.
 // A sum of 2^-90 or more bears the lost bits of an operand below 2^-110 only while its partner stays under 2^20, and a zero may
 // stand for parts that all vanished.  So the threads note the inputs of either kind (Extremes) and the host the channels with
 // weights below 2^-110 (a negative factor): in question are also zeros where a tiny input or weight took part, sums of channels
 // packed down with a tiny input, and sums of channels with tiny weights beside a large input.  The look at every
-// input takes 1 to 2.5 % (512 -> 128 @28 batch 32 27.1 -> 27.7 us, 3x3 / stride 2 128 -> 128 @56 batch 64 98.1 -> 98.8, stem batch 32
-// 75.4 -> 77.4); one tiny pixel 28.3 us, a weight of 1e-40 in every channel 30.4.
+// input takes 0.5 to 2.5 % (512 -> 128 @28 batch 32 27.9 -> 28.5 us, 3x3 / stride 2 128 -> 128 @56 batch 64 98.6 -> 98.9, stem batch 32
+// 78.5 -> 79.9); one tiny pixel 28.7 us, a weight of 1e-40 in every channel 31.  That some factor is not 1 is looked at behind the
+// last stage: waiting for it in front of the first one, behind weights that come from memory, cost the networks 0.8 %.
 // AFF: per-channel affine (+ ReLU) on the input of a 1x1 convolution.
 // Bound: no single one.  512 -> 128 @28 batch 32 takes 26 us: 9 us of MFMAs at the 390 TFLOP/s of fp32 products that a bare MFMA
 // loop reaches, 13 us of memory traffic, and between them LDS reads (a half of the MFMA time at mb = 2), the splitting (6
@@ -177,9 +177,6 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
     bf4_t *const lds4 = reinterpret_cast<bf4_t *>(lds);
     const int part8 = p.CS << no_shift;         // slots per part
     Extremes extremes;
-    // whether any factor of the weights is not 1 (read from memory and not passed: new weights may come under a captured graph)
-    const bool scaled = __builtin_amdgcn_readfirstlane(__float_as_int(*p.w_scale)) == 0x3f800000;
-    const float *const w_scale = p.w_scale + 4;
     auto affine = [&](float (&v)[8], int chunk, int c) {
         if constexpr (AFF) {
             const float *const a = p.in_aff + (size_t)chunk * 2 * p.CCH + c;
@@ -220,7 +217,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
             for (int e = 0; e < 8; ++e) v[e] = group[e][x];
             affine(v, st, 8 * f_oct);
             split3(v, h);
-            extremes.add(v, scaled);
+            extremes.add(v);
 #pragma unroll
             for (int s = 0; s < 3; ++s) lds8[s * part8 + f_oct * p.CS + x * (16 * p.WN) + f_unit] = h[s];
         }
@@ -257,7 +254,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
             for (int i = 0; i < EN; ++i) {
                 if (at[i] < 0) continue;
-                extremes.add(v[i], scaled);
+                extremes.add(v[i]);
                 if constexpr (MODE == SPLIT_FEW) {
                     bf4_t h[3];
                     split3(v[i], h);
@@ -280,6 +277,9 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
         for (int j = 0; j < NB; ++j) lead[m][j] = rest[m][j] = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
     const int steps_all = p.nchunks * ksteps;
+    // (requested here and looked at behind the last stage.  Read from memory and not passed: new weights may come under a captured graph)
+    const float scaled_flag = *p.w_scale;
+    const float *const w_scale = p.w_scale + 4;
     const int mblk0 = (by * p.WM + wm) * MB;
     struct A {
         bf8_t h[3];
@@ -366,6 +366,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 
     // ---- results ---------------------------------------------------------------------------------------------------------
     const int ch_base = mblk0 * 16 + 4 * k;
+    const bool scaled = __builtin_amdgcn_readfirstlane(__float_as_int(scaled_flag)) == 0x3f800000;
     const unsigned met = lane < 8 && 64 * lane < threads ? met_word : 0u;
     const bool tiny_input = __builtin_amdgcn_ballot_w64((met & 1u) != 0) != 0, large_input = __builtin_amdgcn_ballot_w64((met & 2u) != 0) != 0;
     const bool has_resid = p.resid != nullptr;
