@@ -239,30 +239,26 @@ __global__ void __launch_bounds__(512, 2) tdc_conv1x1_block_kernel(const ConvKPa
     };
     const int ch_base = (by * p.WM + wm) * (16 * MB) + 4 * k;
     if (p.WK == 1) {
+        float bv[4 * MB];
+        px_t rv[4 * MB];
 #pragma unroll
-        for (int m = 0; m < MB; ++m) {
-            const int ch0 = ch_base + 16 * m;
-            float bv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            px_t rv[4];
-            if (p.bias) {
+        for (int r = 0; r < 4 * MB; ++r) bv[r] = p.bias ? p.bias[min(ch_base + 16 * (r >> 2) + (r & 3), p.N - 1)] : 0.0f;
+        if (has_resid) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) bv[i] = p.bias[min(ch0 + i, p.N - 1)];
+            for (int r = 0; r < 4 * MB; ++r) rv[r] = load_resid(ch_base + 16 * (r >> 2) + (r & 3));
+        }
+        settle(bv);
+        settle(rv);
+#pragma unroll
+        for (int r = 0; r < 4 * MB; ++r) {
+            px_t v;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                v[j] = acc[r >> 2][j][r & 3] + bv[r];
+                if (has_resid) v[j] += rv[r][j];
+                if (p.relu) v[j] = fmaxf(v[j], 0.0f);
             }
-            if (has_resid) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i) rv[i] = load_resid(ch0 + i);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                px_t v;
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) {
-                    v[j] = acc[m][j][i] + bv[i];
-                    if (has_resid) v[j] += rv[i][j];
-                    if (p.relu) v[j] = fmaxf(v[j], 0.0f);
-                }
-                store(v, ch0 + i);
-            }
+            store(v, ch_base + 16 * (r >> 2) + (r & 3));
         }
         return;
     }
@@ -277,21 +273,32 @@ __global__ void __launch_bounds__(512, 2) tdc_conv1x1_block_kernel(const ConvKPa
             for (int j = 0; j < NJ; ++j) v[j] = acc[m][j][i];
             part[(slice * 4 * MB + 4 * m + i) * 64] = v;
         }
+    const int rows = (4 * MB - slice + p.WK - 1) / p.WK;
+    float bv[2 * MB];
+    px_t rv[2 * MB];
+#pragma unroll
+    for (int r = 0; r < 2 * MB; ++r) {
+        if (r >= rows) break;
+        const int row = slice + r * p.WK, ch = ch_base + 16 * (row >> 2) + (row & 3);
+        bv[r] = p.bias ? p.bias[min(ch, p.N - 1)] : 0.0f;
+        if (has_resid) rv[r] = load_resid(ch);
+    }
     __syncthreads();
-    for (int row = slice; row < 4 * MB; row += p.WK) {
-        const int ch = ch_base + 16 * (row >> 2) + (row & 3);
-        px_t rv;
-        if (has_resid) rv = load_resid(ch);
-        const float bv = p.bias ? p.bias[min(ch, p.N - 1)] : 0.0f;
+    settle(bv);
+    settle(rv);
+#pragma unroll
+    for (int r = 0; r < 2 * MB; ++r) {
+        if (r >= rows) break;
+        const int row = slice + r * p.WK;
         px_t v = part[row * 64];
         for (int s = 1; s < p.WK; ++s) v += part[(s * 4 * MB + row) * 64];
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
-            v[j] += bv;
-            if (has_resid) v[j] += rv[j];
+            v[j] += bv[r];
+            if (has_resid) v[j] += rv[r][j];
             if (p.relu) v[j] = fmaxf(v[j], 0.0f);
         }
-        store(v, ch);
+        store(v, ch_base + 16 * (row >> 2) + (row & 3));
     }
 }
 

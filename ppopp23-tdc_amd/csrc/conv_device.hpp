@@ -144,13 +144,42 @@ __device__ __forceinline__ void finish_four_channels(const f4_t &acc, int ch0, i
     }
 }
 
+// Loads and stores of a wave are counted together and in order, and bias and residual are loaded in branches: where a value of
+// theirs is first used behind a store, the compiler waits for that store too, a memory round trip (about 1 us) per block of
+// outputs.  So kernels whose lanes finish several blocks request all of them first and settle them here, in front of the
+// first store: the one wait stands here, and nothing behind it needs another.  (Tucker block 512-128-128-512 @28 batch 32 121.6 ->
+// 116.1 us, Tucker ResNet-18 batch 32 822 -> 800.)
+template <int N>
+__device__ __forceinline__ void settle(float (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+}
+template <int N, typename V>
+__device__ __forceinline__ void settle(V (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" : "+v"(v[i]));
+}
+
+// Four consecutive channels (from ch0) of one pixel with addends that are in registers (see settle).
+__device__ __forceinline__ void store_four_channels(const f4_t &acc, int ch0, int N, long long P, long long pix, const float (&bias)[4],
+                                                    bool has_resid, const float (&resid)[4], int relu, float *__restrict__ out) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (ch0 + i >= N) continue;
+        float val = acc[i] + bias[i];
+        if (has_resid) val += resid[i];
+        if (relu) val = fmaxf(val, 0.0f);
+        store_out(out + ((long long)(ch0 + i) * P + pix), val);
+    }
+}
+
 // The kernel arguments (about 530 bytes) are read through the scalar cache.  Left alone, the compiler fetches them in
 // several dependent batches, and every batch that touches a cache line for the first time costs a round trip to L2
 // before the first request can go out.  Touch every line of the argument block at once: whatever order the compiler
 // then loads the values in, it hits the scalar cache.
 __device__ __forceinline__ void touch_kernel_arguments() {
     if constexpr (TDC_TOUCH_KERNARGS) {
-        static_assert(sizeof(ConvKParams) > 8 * 64 && sizeof(ConvKParams) <= 9 * 64, "touch exactly the lines of the argument block");
+        static_assert(sizeof(ConvKParams) > 8 * 64 && sizeof(ConvKParams) <= 9 * 64 + 8 * TDC_STAMPS, "touch exactly the lines of the argument block");
         const auto kargs = __builtin_amdgcn_kernarg_segment_ptr();
         unsigned t0, t1, t2, t3, t4, t5, t6, t7, t8;
         asm volatile(
@@ -182,6 +211,15 @@ __device__ __forceinline__ ImageBase image_base(const ConvKParams &p, int img) {
     return b;
 }
 
+// The kernel arguments, read when they are used: what only the end of a kernel needs would otherwise be loaded at its start and cost
+// scalar registers all the way.  (In a kernel whose only argument is the ConvKParams.)
+typedef const __attribute__((address_space(4))) ConvKParams *late_args_t;
+__device__ __forceinline__ late_args_t late_arguments() {
+    late_args_t args = (late_args_t)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    return args;
+}
+
 // A block of 16 channels x 16 pixels as plain fp32 sums over the weights as the caller gave them (w_raw, OIHW): for the rare
 // outputs that a transform or a split of the operands cannot represent.  Lane (k = l / 16, n = l % 16) names channel `ch` (row n
 // of the block; past N: any) and output pixel (oy, ox) of image `img` (column n); it gets rows 4k .. 4k + 3 of its pixel.  Every
@@ -189,11 +227,7 @@ __device__ __forceinline__ ImageBase image_base(const ConvKParams &p, int img) {
 // Bound: latency, sixteen channels in flight; a wave in which it runs takes several times as long.
 template <bool AFF>
 __device__ __forceinline__ f4_t direct_block(int ch, int img, int oy, int ox) {
-    // (the kernel arguments are read here and now: kept for this from the start they would cost the kernel's ordinary path scalars)
-    typedef const __attribute__((address_space(4))) ConvKParams *args_t;
-    args_t args = (args_t)__builtin_amdgcn_kernarg_segment_ptr();
-    asm volatile("" : "+s"(args));
-    const auto &p = *args;
+    const auto &p = *late_arguments();
     const int k = (threadIdx.x >> 4) & 3;
     const int taps = p.KH * p.KW, plane = p.H * p.W;
     const float *const w = p.w_raw + (size_t)min(ch, p.N - 1) * p.C * taps;

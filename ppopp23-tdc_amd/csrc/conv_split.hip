@@ -1,57 +1,8 @@
 // fp32 convolution on the bf16 matrix pipe (tile.alg = 8, tdc_conv_split_kernel).
 #include "conv_device.hpp"
+#include "conv_split_device.hpp"
 
 namespace tdc {
-
-typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
-typedef __bf16 bf4_t __attribute__((ext_vector_type(4)));
-
-// neither zero nor of a magnitude in [2^-90, infinity)
-static __device__ __forceinline__ bool suspect(float sum) {
-    const unsigned twice = __float_as_uint(sum) << 1;   // (without the sign)
-    return twice - 2u * 0x12800000u >= 2u * (0x7f800000u - 0x12800000u) && twice != 0;
-}
-// Whether any of several sums is: two and a half vector instructions each.  (The total may overflow without any of them being
-// infinite; then each is looked at in vain.)
-struct Range {
-    unsigned low = ~0u;
-    float total = 0.0f;
-    __device__ __forceinline__ void add(float sum) {
-        low = min(low, (__float_as_uint(sum) << 1) - 1u);   // (zero: the largest)
-        total += fabsf(sum);
-    }
-    __device__ __forceinline__ bool suspect() const { return low < 2u * 0x12800000u - 1u || !(total < __builtin_inff()); }
-};
-
-// What a thread has met among the values it split: whether any is below 2^-110 but not zero, and whether any reaches 2^20.  Two
-// vector instructions a value (beside six for the split).
-struct Extremes {
-    unsigned low = ~0u;
-    float high = 0.0f;
-    template <int N>
-    __device__ __forceinline__ void add(const float (&x)[N]) {
-#pragma unroll
-        for (int i = 0; i < N; i += 2) {
-            low = min(min(low, (__float_as_uint(x[i]) << 1) - 1u), (__float_as_uint(x[i + 1]) << 1) - 1u);   // (zero: the largest)
-            asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(high) : "v"(high), "v"(x[i]), "v"(x[i + 1]));   // (fmaxf would quiet each value first)
-        }
-    }
-    __device__ __forceinline__ bool tiny() const { return low < 2u * 0x08800000u - 1u; }
-    __device__ __forceinline__ bool large() const { return high >= 0x1p20f; }
-};
-constexpr int EXTREMES_FLOATS = 8;   // of LDS, in front of everything else: one word per wave
-
-// x = h[0] + h[1] + h[2] exactly for finite x (8 bits of the mantissa each), as long as the lowest part stays representable.
-template <int N, typename V>
-static __device__ __forceinline__ void split3(const float (&x)[N], V (&h)[3]) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        h[0][i] = (__bf16)x[i];
-        const float r1 = x[i] - (float)h[0][i];
-        h[1][i] = (__bf16)r1;
-        h[2][i] = (__bf16)(r1 - (float)h[1][i]);
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Every operand is split into three bf16 parts that add up to the fp32 value, and a product is the sum of the six partial
@@ -370,11 +321,6 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
     const unsigned met = lane < 8 && 64 * lane < threads ? met_word : 0u;
     const bool tiny_input = __builtin_amdgcn_ballot_w64((met & 1u) != 0) != 0, large_input = __builtin_amdgcn_ballot_w64((met & 2u) != 0) != 0;
     const bool has_resid = p.resid != nullptr;
-    // Whether the split may have lost what counts in a sum of a channel with factor `scale` (below 0: it has tiny weights).
-    auto in_question = [&](float sum, float scale) {
-        const bool tiny_weights = scale < 0.0f;
-        return suspect(sum) || (sum == 0.0f && (tiny_input || tiny_weights)) || (tiny_input && fabsf(scale) > 1.0f) || (large_input && tiny_weights);
-    };
     // Plain sums for pixel j of this lane's group or block (see above), lane n naming channel `ch`.
     auto plain = [&](int ch, int j) __attribute__((always_inline)) {
         const Pixel px = pixel(MODE == SPLIT_FLAT ? 0 : j);
@@ -404,7 +350,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
                 for (int x = 1; x < MB * NB; ++x) v = x != r ? v : lead[x / NB][x % NB];
                 bool ask[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) ask[i] = in_question(v[i], scale[i]);
+                for (int i = 0; i < 4; ++i) ask[i] = in_question(v[i], scale[i], tiny_input, large_input);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) v[i] *= fabsf(scale[i]);
                 if (__builtin_amdgcn_ballot_w64(ask[0] || ask[1] || ask[2] || ask[3]) != 0) {
@@ -440,26 +386,22 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
             }
         };
         if (p.WK == 1) {
+            float bv[4 * MB];
+            px_t rv[4 * MB];
 #pragma unroll
-            for (int m = 0; m < MB; ++m) {
-                const int ch0 = ch_base + 16 * m;
-                float bv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-                px_t rv[4];
-                if (p.bias) {
+            for (int r = 0; r < 4 * MB; ++r) bv[r] = p.bias ? p.bias[min(ch_base + 16 * (r >> 2) + (r & 3), p.N - 1)] : 0.0f;
+            if (has_resid) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) bv[i] = p.bias[min(ch0 + i, p.N - 1)];
-                }
-                if (has_resid) {
+                for (int r = 0; r < 4 * MB; ++r) rv[r] = load_resid(ch_base + 16 * (r >> 2) + (r & 3));
+            }
+            settle(bv);
+            settle(rv);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) rv[i] = load_resid(ch0 + i);
-                }
+            for (int r = 0; r < 4 * MB; ++r) {
+                px_t v;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    px_t v;
-#pragma unroll
-                    for (int j = 0; j < NB; ++j) v[j] = lead[m][j][i];
-                    finish(v, ch0 + i, bv[i], rv[i]);
-                }
+                for (int j = 0; j < NB; ++j) v[j] = lead[r >> 2][j][r & 3];
+                finish(v, ch_base + 16 * (r >> 2) + (r & 3), bv[r], rv[r]);
             }
             return;
         }
@@ -477,17 +419,27 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
             }
         barrier();
         const int rows = 4 * MB / p.WK;          // (WK divides 4 * MB)
-        for (int r0 = 0; r0 < rows; r0 += 2) {   // two at a time, bias and residual requested before they are needed
-            float bv[2] = {0.0f, 0.0f};
-            px_t rv[2], v[2];
+        float bv[2 * MB];
+        px_t rv[2 * MB];
+#pragma unroll
+        for (int r = 0; r < 2 * MB; ++r) {
+            if (r >= rows) break;
+            const int row = slice + r * p.WK, ch = ch_base + 16 * (row >> 2) + (row & 3);
+            bv[r] = p.bias ? p.bias[min(ch, p.N - 1)] : 0.0f;
+            if (has_resid) rv[r] = load_resid(ch);
+        }
+        settle(bv);
+        settle(rv);
+#pragma unroll
+        for (int r0 = 0; r0 < 2 * MB; r0 += 2) {   // two at a time
+            if (r0 >= rows) break;
+            px_t v[2];
             int ch[2];
             bool bad = false;
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
                 const int row = slice + min(r0 + i, rows - 1) * p.WK;
                 ch[i] = ch_base + 16 * (row >> 2) + (row & 3);
-                if (p.bias) bv[i] = p.bias[min(ch[i], p.N - 1)];
-                if (has_resid) rv[i] = load_resid(ch[i]);
                 v[i] = part[row * 64];
                 for (int s = 1; s < p.WK; ++s) v[i] += part[(s * 4 * MB + row) * 64];
 #pragma unroll
@@ -499,7 +451,7 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
                 for (int i = 0; i < 2; ++i) {
                     if (scaled) scale[i] = w_scale[ch[i]];
 #pragma unroll
-                    for (int j = 0; j < NB; ++j) bad |= in_question(v[i][j], scale[i]);
+                    for (int j = 0; j < NB; ++j) bad |= in_question(v[i][j], scale[i], tiny_input, large_input);
                 }
             }
             if (__builtin_expect(__builtin_amdgcn_ballot_w64(bad) != 0, 0)) {
@@ -511,24 +463,41 @@ __global__ void __launch_bounds__(512, 2) tdc_conv_split_kernel(const ConvKParam
 #pragma unroll
                     for (int i = 0; i < 2; ++i)
 #pragma unroll
-                        for (int x = 0; x < NB; ++x) v[i][x] = x != j ? v[i][x] : in_question(v[i][x], scale[i]) ? sums[i] : v[i][x] * fabsf(scale[i]);
+                        for (int x = 0; x < NB; ++x) v[i][x] = x != j ? v[i][x] : in_question(v[i][x], scale[i], tiny_input, large_input) ? sums[i] : v[i][x] * fabsf(scale[i]);
                 }
             } else if (__builtin_expect(scaled, 0)) {
 #pragma unroll
                 for (int i = 0; i < 2; ++i) v[i] *= fabsf(scale[i]);
             }
-            finish(v[0], ch[0], bv[0], rv[0]);
-            if (r0 + 1 < rows) finish(v[1], ch[1], bv[1], rv[1]);
+            finish(v[0], ch[0], bv[r0], rv[r0]);
+            if (r0 + 1 < rows) finish(v[1], ch[1], bv[r0 + 1], rv[r0 + 1]);
         }
     } else {
+        const auto &q = *late_arguments();
+        float bias[MB][4];
+#pragma unroll
+        for (int m = 0; m < MB; ++m) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) bias[m][i] = q.bias ? q.bias[min(ch_base + 16 * m + i, q.N - 1)] : 0.0f;
+            settle(bias[m]);
+        }
 #pragma unroll
         for (int j = 0; j < NB; ++j) {
             const Pixel px = pixel(j);
             if (px.fresh) continue;
-            float *__restrict__ const out = p.out + (long long)px.img * p.out_bstride;
-            const float *__restrict__ const resid = has_resid ? p.resid + (long long)px.img * p.resid_bstride : nullptr;
+            float resid[MB][4];
+            if (q.resid) {                    // (a column of blocks at a time: all of them would not fit the registers)
+                const float *__restrict__ const from = q.resid + ((long long)px.img * q.resid_bstride + px.pix);
 #pragma unroll
-            for (int m = 0; m < MB; ++m) finish_four_channels(lead[m][j], ch_base + 16 * m, p.N, p.P, px.pix, p.bias, resid, p.relu, out);
+                for (int m = 0; m < MB; ++m)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) resid[m][i] = from[(long long)min(ch_base + 16 * m + i, q.N - 1) * q.P];
+#pragma unroll
+                for (int m = 0; m < MB; ++m) settle(resid[m]);
+            }
+            float *__restrict__ const out = q.out + (long long)px.img * q.out_bstride;
+#pragma unroll
+            for (int m = 0; m < MB; ++m) store_four_channels(lead[m][j], ch_base + 16 * m, q.N, q.P, px.pix, bias[m], q.resid != nullptr, resid[m], q.relu, out);
         }
     }
 }

@@ -306,25 +306,21 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
     const bool parted = PARTS && steps > 10;    // (the last two steps never start a part)
     const int ch_base = by * (16 * MB) + 4 * k;
     if (p.WK == 1) {
+        float bv[4 * MB];
+        f4_t rv[4 * MB];
 #pragma unroll
-        for (int m = 0; m < MB; ++m) {
-            const int ch0 = ch_base + 16 * m;
-            float bv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            f4_t rv[4];
-            if (p.bias) {
+        for (int r = 0; r < 4 * MB; ++r) bv[r] = p.bias ? p.bias[min(ch_base + 16 * (r >> 2) + (r & 3), p.N - 1)] : 0.0f;
+        if (has_resid) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i) bv[i] = p.bias[min(ch0 + i, p.N - 1)];
-            }
-            if (has_resid) {
+            for (int r = 0; r < 4 * MB; ++r) rv[r] = load_resid(ch_base + 16 * (r >> 2) + (r & 3));
+        }
+        settle(bv);
+        settle(rv);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) rv[i] = load_resid(ch0 + i);
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                f4_t v = output(m, i);
-                if (parted) v += own[(4 * m + i) * 64];
-                store(finish(v, bv[i], rv[i]), ch0 + i, unusual(v, 4 * m + i));
-            }
+        for (int r = 0; r < 4 * MB; ++r) {
+            f4_t v = output(r >> 2, r & 3);
+            if (parted) v += own[r * 64];
+            store(finish(v, bv[r], rv[r]), ch_base + 16 * (r >> 2) + (r & 3), unusual(v, r));
         }
     } else {
         // every wave of a team finishes every WK-th row
@@ -332,15 +328,26 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
         for (int m = 0; m < MB; ++m)
 #pragma unroll
             for (int i = 0; i < 4; ++i) own[(4 * m + i) * 64] = parted ? own[(4 * m + i) * 64] + output(m, i) : output(m, i);
+        const int rows = 4 * MB / p.WK;         // (WK = 2 or 4)
+        float bv[2 * MB];
+        f4_t rv[2 * MB];
+#pragma unroll
+        for (int r = 0; r < 2 * MB; ++r) {
+            if (r >= rows) break;
+            const int row = slice + r * p.WK, ch = ch_base + 16 * (row >> 2) + (row & 3);
+            bv[r] = p.bias ? p.bias[min(ch, p.N - 1)] : 0.0f;
+            if (has_resid) rv[r] = load_resid(ch);
+        }
         __syncthreads();
-        for (int row = slice; row < 4 * MB; row += p.WK) {
-            const int ch = ch_base + 16 * (row >> 2) + (row & 3);
-            f4_t rv = (f4_t){0.0f, 0.0f, 0.0f, 0.0f};
-            if (has_resid) rv = load_resid(ch);
-            const float bv = p.bias ? p.bias[min(ch, p.N - 1)] : 0.0f;
+        settle(bv);
+        settle(rv);
+#pragma unroll
+        for (int r = 0; r < 2 * MB; ++r) {
+            if (r >= rows) break;
+            const int row = slice + r * p.WK;
             f4_t v = part[row * 64];
             for (int s = 1; s < p.WK; ++s) v += part[(s * 4 * MB + row) * 64];
-            store(finish(v, bv, rv), ch, unusual(v, row));
+            store(finish(v, bv[r], rv[r]), ch_base + 16 * (row >> 2) + (row & 3), unusual(v, row));
         }
     }
     if (__builtin_expect(__builtin_amdgcn_ballot_w64(left_out != 0) == 0, 1)) return;
