@@ -74,7 +74,7 @@ typedef struct tdc_tile {
                      also 4)                                                     */
     int32_t nb;   /* MFMA blocks per wave along pixels (1 or 2; alg 4 and 6 also 4: the
                      workgroup's tile is nb 16-pixel blocks side by side along a row;
-                     alg 7: 2 or 4; alg 8: 4, with tw = 0 also 2)                */
+                     alg 7 and 8: 2 or 4)                                        */
     int32_t wm;   /* waves along output channels                               */
     int32_t wn;   /* waves along pixels                                        */
     int32_t wk;   /* waves along input channels (in-workgroup split-K)          */
@@ -131,10 +131,11 @@ typedef struct tdc_tile {
                          where the split does not hold, are computed again without it).  16 * mb channels x 16 * nb pixels per
                          wave.  tw = 0: 1x1 / stride 1 / pad 0, the pixels of all images in one row of groups of nb, wk
                          waves over input channels (mb 1 or 2, cch = 32 * wm * wk, at most 8 waves).  tw > 0: filters larger than
-                         1x1, any stride and dilation, nb = 4, wk = 1: tiles of tw columns and as many output rows, counted through the
-                         batch, as fit in 64 * wn pixels; cch = 8, 16 or 32 input channels per pass, or 4 (at most four
-                         input channels, even stride, dilation 1).  ks = 1, wl = 0.  The 1x1 form carries the input
-                         affine; no fused tail.
+                         1x1, any stride and dilation: tiles of tw columns and as many output rows, counted through the
+                         batch, as fit in 16 * nb * wn pixels.  nb = 4: wk = 1, cch = 8, 16 or 32 input channels per pass, or 4 (at
+                         most four input channels, even stride, dilation 1).  nb = 2: cch = 8 to 128, a power of two, and wk
+                         waves over the steps of a pass (ceil(KH * KW * cch / 32), a multiple of wk).  ks = 1, wl = 0.  The
+                         1x1 form carries the input affine; no fused tail.
                      The model offers 3 to 6 where launch and latency dominate (few channels or few pixels); the
                      staged paths keep the layers whose operands are worth sharing through the LDS. */
 } tdc_tile;

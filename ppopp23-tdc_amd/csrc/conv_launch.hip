@@ -8,14 +8,15 @@
 
 namespace tdc {
 
-// The kernels live in six translation units (conv_staged.hip, conv_stream.hip, conv_wino_stream.hip, conv_block.hip,
-// conv_wino_block.hip, conv_split.hip); each maps the KernelIds of its families to its instantiations.
+// The kernels live in seven translation units (conv_staged.hip, conv_stream.hip, conv_wino_stream.hip, conv_block.hip,
+// conv_wino_block.hip, conv_split.hip, conv_core_split.hip); each maps the KernelIds of its families to its instantiations.
 const void *kernel_function(const KernelId &k) {
     return k.family == KernelId::STAGED        ? staged_kernel_function(k)
            : k.family == KernelId::STREAM_WINO ? wino_stream_kernel_function(k)
            : k.family == KernelId::BLOCK_1x1   ? block_kernel_function(k)
            : k.family == KernelId::BLOCK_WINO  ? wino_block_kernel_function(k)
            : k.family == KernelId::SPLIT       ? split_kernel_function(k)
+           : k.family == KernelId::SPLIT_CORE  ? core_split_kernel_function(k)
                                                : stream_kernel_function(k);
 }
 

@@ -200,8 +200,9 @@ enum : int { TAPS_GENERIC = 0, TAPS_1x1 = 1, TAPS_3x3 = 9, TAPS_3x3G = 10, TAPS_
 //   BLOCK_WINO  tdc_wino3x3_block_kernel<MB, WN, PARTS>               p = {MB, WN, PARTS}
 //   BLOCK_1x1   tdc_conv1x1_block_kernel<MB, NJ, AFF, GEN, PART>      p = {MB, NJ, AFF, GEN, PART}
 //   SPLIT       tdc_conv_split_kernel<MB, NB, MODE, AFF>              p = {MB, NB, MODE, AFF}   (MODE: 0 flat, 1 window, 2 few channels)
+//   SPLIT_CORE  tdc_core_split_kernel<MB>                             p = {MB}
 struct KernelId {
-    enum Family : int { NONE = 0, STAGED = 1, STREAM_1x1 = 2, STREAM_3x3 = 3, STREAM_WINO = 4, BLOCK_1x1 = 5, BLOCK_WINO = 6, SPLIT = 7 };
+    enum Family : int { NONE = 0, STAGED = 1, STREAM_1x1 = 2, STREAM_3x3 = 3, STREAM_WINO = 4, BLOCK_1x1 = 5, BLOCK_WINO = 6, SPLIT = 7, SPLIT_CORE = 8 };
     int family = NONE;
     int p[6] = {0, 0, 0, 0, 0, 0};
 };
@@ -221,13 +222,14 @@ int kernel_vgprs(const KernelId &k);
 int kernel_waves_per_simd(const KernelId &k);
 // The function itself (nullptr if not instantiated).
 const void *kernel_function(const KernelId &k);
-// (its parts, one per translation unit that holds kernels: conv_staged.hip, conv_stream.hip, conv_wino_stream.hip, conv_block.hip, conv_wino_block.hip, conv_split.hip)
+// (its parts, one per translation unit that holds kernels: conv_staged.hip, conv_stream.hip, conv_wino_stream.hip, conv_block.hip, conv_wino_block.hip, conv_split.hip, conv_core_split.hip)
 const void *staged_kernel_function(const KernelId &k);
 const void *stream_kernel_function(const KernelId &k);
 const void *wino_stream_kernel_function(const KernelId &k);
 const void *block_kernel_function(const KernelId &k);
 const void *wino_block_kernel_function(const KernelId &k);
 const void *split_kernel_function(const KernelId &k);
+const void *core_split_kernel_function(const KernelId &k);
 inline const void *conv_kernel_for(const tdc_tile &t, int KH, int KW, int dilation, int stride, bool extras, bool single_pixels) {
     return kernel_function(kernel_id_for(t, KH, KW, dilation, stride, extras, single_pixels));
 }

@@ -119,18 +119,19 @@ static int channel_major_order(double in_bytes, double w_bytes, long long n_wg, 
     return channel_major < pixel_major ? 1 : 0;
 }
 
-// tile.alg = 8: fp32 operands as three bf16 parts each (conv_split.hip).
+// tile.alg = 8: fp32 operands as three bf16 parts each (conv_split.hip, conv_core_split.hip).
 static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::string *why, int tail_N) {
     auto fail = [&](const char *m) {
         if (why) *why = m;
         return false;
     };
     const bool flat = t.tw == 0, few = t.cch == 4, one = d.KH == 1 && d.KW == 1;
-    if (t.mf != 16 || (t.nb != 4 && !(t.nb == 2 && flat)) || (t.mb != 1 && t.mb != 2 && t.mb != 4))
-        return fail("tile.alg = 8 needs mf = 16, mb = 1, 2 or 4, nb = 4 (with tw = 0 also 2)");
+    const bool core = !flat && t.nb == 2;       // (conv_core_split.hip)
+    if (t.mf != 16 || (t.nb != 4 && t.nb != 2) || (core && few) || (t.mb != 1 && t.mb != 2 && t.mb != 4))
+        return fail("tile.alg = 8 needs mf = 16, mb = 1, 2 or 4, nb = 2 or 4 (4 with cch = 4)");
     if (t.wm < 1 || t.wn < 1 || t.wk < 1 || (long long)t.wm * t.wn * t.wk > 8) return fail("tile.alg = 8 needs 1 to 8 waves");
-    if ((t.wk != 1 && !flat) || t.ks != 1 || t.wl != 0)
-        return fail("tile.alg = 8 has no split across workgroups and no loader waves, and splits input channels over waves only with tw = 0");
+    if ((t.wk != 1 && !flat && !core) || t.ks != 1 || t.wl != 0)
+        return fail("tile.alg = 8 has no split across workgroups and no loader waves, and splits input channels over waves only with tw = 0 or nb = 2");
     if (tail_N > 0) return fail("tile.alg = 8 cannot carry a fused tail");
     g = Geometry();
     g.Ho = (d.H + 2 * d.pad - d.dilation * (d.KH - 1) - 1) / d.stride + 1;
@@ -175,8 +176,8 @@ static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geome
         if (few) {
             if (d.C > 4 || d.dilation != 1 || d.stride % 2 != 0)
                 return fail("tile.alg = 8 with cch = 4 needs at most four input channels, an even stride and dilation 1");
-        } else if (t.cch != 8 && t.cch != 16 && t.cch != 32) {
-            return fail("tile.alg = 8 needs cch = 8, 16 or 32 (4: at most four input channels)");
+        } else if (t.cch != 8 && t.cch != 16 && t.cch != 32 && !(core && (t.cch == 64 || t.cch == 128))) {
+            return fail("tile.alg = 8 needs cch = 8, 16 or 32, with nb = 2 also 64 or 128 (4: at most four input channels)");
         }
         if (one) return fail("tile.alg = 8 takes 1x1 convolutions with tw = 0 only");
         if (t.tw < 1 || t.tw > g.PT || t.tw > g.Wo) return fail("tile.alg = 8: tile.tw does not fit");
@@ -188,6 +189,7 @@ static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geome
         while ((8 << g.oct_shift) < t.cch) ++g.oct_shift;
         g.row_taps = few ? ceil_div(d.KW, 2) : d.KW;
         g.ksteps = few ? ceil_div(d.KH * g.row_taps, 4) : ceil_div(g.taps << g.oct_shift, 4);
+        if (g.ksteps % t.wk != 0) return fail("tile.alg = 8: wk does not divide the K-steps of a stage");
         const long long columns = (long long)(g.TW - 1) * d.stride + (few ? 2 * g.row_taps : (d.KW - 1) * d.dilation + 1);
         const long long image_rows = (long long)(g.Ho - 1) * d.stride + (long long)(d.KH - 1) * d.dilation + 1;
         // the most window rows any tile of output rows needs (the tiles repeat their place in the images after Ho of them)
@@ -206,7 +208,9 @@ static bool make_split_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geome
         g.odd_columns = (g.ncols + 1) / 2;
         g.RS = !few && d.stride == 2 ? 2 * g.odd_columns : g.ncols;
         g.CS = g.nrows * g.RS;
-        lds = few ? 3LL * g.CS * 8 : (3LL * g.CS * 16) << g.oct_shift;
+        // (whole rounds of the LDS banks from octet to octet, where they fit)
+        if (core && ((48LL * round_up(g.CS, 16)) << g.oct_shift) + 32 <= machine().lds_bytes_per_cu) g.CS = round_up(g.CS, 16);
+        lds = few ? 3LL * g.CS * 8 : std::max((48LL * g.CS) << g.oct_shift, t.wk > 1 ? 1024LL * g.waves * t.mb * t.nb : 0LL);   // (the sums of all waves)
         cols = ceil_div(g.Wo, g.TW);
     }
     if (units * std::max(g.units_image, 16) >= (1LL << 32) || units >= (1LL << 30)) return fail("batch too large for tile.alg = 8");
@@ -269,7 +273,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     g.taps = d.KH * d.KW;
     g.ktaps = g.taps;
     g.MT = t.mf * t.mb * t.wm;
-    if (t.alg < 0 || t.alg > 7) return fail("tile.alg must be in [0, 8]");
+    if (t.alg < 0 || t.alg > 7) return fail("tile.alg must be in [0, 9]");
     if (t.alg == 5) {
         // Winograd F(2x2,3x3) streamed from global memory: 16*wm channels of one tile row block (2 rows x 28 columns) per
         // workgroup, the input channels split over wk waves in groups of four, everything in one pass
@@ -784,11 +788,12 @@ KernelId kernel_id_for(const tdc_tile &t, int KH, int KW, int dilation, int stri
         if (t.mf != 16 || (t.nb != 2 && t.nb != 4) || (t.mb != 1 && t.mb != 2 && t.mb != 4)) return k;
         // (`extras` here can only mean the input affine of a 1x1 convolution)
         const int mode = t.tw == 0 ? 0 : t.cch == 4 ? 2 : 1;
-        if (mode == 0 ? t.mb > 2 : t.nb != 4) return k;
+        if (mode == 0 ? t.mb > 2 : mode == 2 && t.nb != 4) return k;
         if ((mode == 0) != (KH == 1 && KW == 1)) return k;
         if ((mode != 0 && extras) || (mode == 2 && dilation != 1)) return k;
-        k.family = KernelId::SPLIT;
-        k.p[0] = t.mb; k.p[1] = t.nb; k.p[2] = mode; k.p[3] = extras;
+        k.p[0] = t.mb;
+        k.family = mode == 1 && t.nb == 2 ? KernelId::SPLIT_CORE : KernelId::SPLIT;
+        if (k.family == KernelId::SPLIT) k.p[1] = t.nb, k.p[2] = mode, k.p[3] = extras;
         return k;
     }
     if (t.alg == 1 && t.tw == 0) {
@@ -897,6 +902,9 @@ std::string kernel_name(const KernelId &k) {
         case KernelId::SPLIT:
             std::snprintf(buf, sizeof buf, "tdc_conv_split_kernel<%d, %d, %d, %s>", k.p[0], k.p[1], k.p[2], tf[k.p[3] != 0]);
             break;
+        case KernelId::SPLIT_CORE:
+            std::snprintf(buf, sizeof buf, "tdc_core_split_kernel<%d>", k.p[0]);
+            break;
         default: return "";
     }
     return buf;
@@ -909,6 +917,32 @@ std::string kernel_name(const KernelId &k) {
 int kernel_vgprs(const KernelId &k) {
     const CompiledKernel *c = compiled_kernel(k);
     return c ? (c->regs + 7) / 8 * 8 : 0;
+}
+
+// Price of the split-operand tiles for filters of several taps, in us: a power mean of what a SIMD has to issue (MFMAs, K-steps,
+// staging, stores), of the rounds of workgroups that each take their own chain of stages, and of the weights' way through the
+// L1s, + launch + memory traffic.  `staged`: bytes of LDS per pixel (pair) and octet.
+struct SplitPrice {
+    double pipe_mfma, pipe_step, pipe_stage, pipe_block;
+    double start, stage, stage_entry, step, mfma, block;
+    double weights, launch_us, traffic, power, fragment;
+    double staged;
+};
+static const SplitPrice split_core_price = {0.739, 191.1, 460.1, 600.3, 2930, 2593, 1098, 303.2, 0.8651, 417.2, 1.009, 3.726, 34.35, 2.024, 0.3892, 48};
+static double split_price(const SplitPrice &q, const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, int wg_per_cu) {
+    const double wgs = (double)g.grid_x * g.grid_y / machine().cus;
+    const double load = 0.5 * (std::ceil(wgs) + std::max(wgs, 1.0)), simd = (double)g.waves / machine().simds_per_cu;
+    const double steps = (double)g.nchunks * g.ksteps / t.wk, blocks = t.mb * t.nb, mfmas = steps * blocks * 96.0;
+    const double entries = (g.lds_bytes - 32) / q.staged / g.threads;
+    const double stores = blocks * (1.0 + q.fragment * (16.0 / std::min(t.tw, 16) - 1.0));   // (short rows make short stores)
+    const double shared = std::max(1.0, 0.75 * std::min(std::min((double)wg_per_cu, std::max(1.0, std::ceil(wgs))) * simd, 2.0));
+    const double pipe = load * simd * (q.pipe_mfma * mfmas + q.pipe_step * steps + q.pipe_stage * g.nchunks * entries + q.pipe_block * stores);
+    const double chain = std::ceil(wgs / wg_per_cu) *
+                         (q.start + g.nchunks * (q.stage + q.stage_entry * entries) + q.step * steps + q.mfma * mfmas * shared + q.block * stores);
+    const double l1 = q.weights * load * simd * 4.0 * steps * t.mb * 3072.0 / 56.0;
+    const double clk = std::pow(std::pow(pipe, q.power) + std::pow(chain, q.power) + std::pow(l1, q.power), 1.0 / q.power);
+    const double traffic = 4.0 * d.batch * ((double)d.C * d.H * d.W + (double)d.N * g.P) + 6.0 * d.C * d.N * g.ktaps;
+    return q.launch_us + clk / (machine().clock_ghz * 1e3) + traffic / (q.traffic * 1e6);
 }
 
 bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &info, std::string *why, int tail_N) {
@@ -1130,6 +1164,15 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
         info.pred_l2_bytes = 0.0;
         return true;
     }
+    if (t.alg == 8 && t.tw > 0 && t.nb == 2) {
+        // Fitted to 15000 timed tiles of 1000 shapes (most at 3x3 / stride 2): 6 % mean error, 2.5 % mean loss of the pick within the
+        // family.  At 0.86 one shape in eight gains more than 2 % over its former pick (its time falls by 18 % in the mean, most where
+        // the staged kernel took it), and three in a thousand lose more, 5 to 8 % (0.80: 16 % gain, 3 % lose; 0.92: 6 % and 0.3 %):
+        // the line falls at about 12 us at stride 2.
+        info.pred_us = 0.86 * split_price(split_core_price, d, t, g, wg_per_cu);
+        info.pred_l2_bytes = 0.0;
+        return true;
+    }
     if (t.alg == 8) {
         // Split operands on the bf16 matrix pipe: the largest of what the matrix pipes, a workgroup's own chain of stages and
         // the L2 need, + LDS reads + the end of every workgroup + launch and memory traffic.  Fitted to 4500 timed tiles of 90
@@ -1252,6 +1295,25 @@ std::vector<tdc_tile> model_enumerate(const tdc_conv_desc &d, int tail_N) {
                                 if ((cch == 4) == few && cch < 2 * d.C + 8) offer({16, mb, 4, wm, wn, 1, cch, tw, 1, 0, 8});
                     }
                 }
+        if (!one && d.C >= 32 && flops < 2.5e10) {
+            // The form of 32 pixels per wave.  From about 3e10 on the matrix work of 64 channels x 64 pixels per wave is worth more
+            // (448 -> 64 @90 / stride 2 batch 33, 33 Gflop: 338 us against 318); under 32 channels its sums are no more accurate.
+            for (int mb : {1, 2, 4})
+                for (int wm : {1, 2, 4, 8})
+                    for (int wn : {1, 2, 4})
+                        for (int wk : {1, 2, 4}) {
+                            if ((wm * wn * wk != 4 && wm * wn * wk != 8) || 16 * mb * wm > round_up(d.N, 16 * mb)) continue;
+                            std::vector<int> widths;
+                            for (int tw : {Wo, ceil_div(Wo, 2), ceil_div(Wo, 4), 8, 16}) {
+                                if (tw > std::min(Wo, 32 * wn) || std::find(widths.begin(), widths.end(), tw) != widths.end()) continue;
+                                const double rows = (double)d.batch * Ho, th = std::min(32.0 * wn / tw, rows);
+                                if (rows * Wo >= 0.7 * 32 * wn * std::ceil(rows / std::floor(th)) * ceil_div(Wo, tw)) widths.push_back(tw);
+                            }
+                            for (int tw : widths)
+                                for (int cch : {8, 16, 32, 64, 128})
+                                    if (cch < 2 * d.C + 8 && (cch >= 32 || cch >= d.C)) offer({16, mb, 2, wm, wn, wk, cch, tw, 1, 0, 8});
+                        }
+        }
     }
     // register-blocked 1x1 candidates
     if (d.KH == 1 && d.KW == 1 && d.pad == 0 && tail_N == 0 && !std::getenv("TDC_EXPERIMENT_NO_BLOCKED_1X1")) {

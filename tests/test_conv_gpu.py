@@ -1,4 +1,5 @@
 """GPU parity of the single-convolution entry points (tdc_conv_*) against the CPU oracle."""
+import itertools
 import math
 import sys
 
@@ -1183,6 +1184,40 @@ def test_every_split_tile(shape, K, stride, pad, dil):
             got = plan.forward(x.cuda()).cpu().numpy()
             assert_close(got, want_aff, f"input affine {shape} {t}")
         plan.close()
+
+
+@pytest.mark.parametrize("shape,K,stride,pad,dil", [((3, 130, 40, 9, 7), 3, 2, 1, 1), ((2, 70, 72, 30, 29), 3, 2, 1, 1), ((2, 64, 17, 12, 9), 2, 3, 0, 1),
+                                                    ((3, 100, 20, 11, 11), 3, 1, 2, 2), ((1, 40, 130, 64, 5), 5, 1, 2, 1)])
+def test_split_tiles_of_large_stages(shape, K, stride, pad, dil):
+    """Larger filters, stages of 64 and 128 channels (one and several, ragged; windows of more entries than the threads request in
+    one round) and K-steps dealt to two and four waves, with the whole epilogue on channel slices.  The error against 64-bit sums
+    is bounded by 2e-7 of the norm: six products add up from zero, and one rounding of a sum remains per 32 of them (measured over
+    K = 36 ... 4608: 0.7e-7 ... 1.4e-7)."""
+    B, C, N, H, W = shape
+    x, w = case(8710 + C + N + H, B, C, N, H, W, K)
+    g = seeded(8711)
+    bias = torch.randn(N, generator=g)
+    exact = torch.nn.functional.conv2d(x.double(), w.double(), None, stride, pad, dil)
+    Ho, Wo = exact.shape[2], exact.shape[3]
+    resid = torch.randn(B, N, Ho, Wo, generator=g)
+    want_full = (exact + bias.view(1, -1, 1, 1) + resid).clamp_min(0).float().numpy()
+    d = tdc_amd.conv_desc(B, C, N, H, W, K, K, stride, pad, dil)
+    seen = set()
+    for mb, (wm, wn, wk) in itertools.product((1, 2, 4), ((1, 4, 1), (2, 1, 4), (1, 2, 2), (4, 1, 2), (1, 1, 4))):
+        for cch, tw in itertools.product((64, 128), sorted({Wo, -(-Wo // 4)})):
+            t = tdc_amd.Tile(16, mb, 2, wm, wn, wk, cch, tw, 1, 0, 8)
+            try:
+                tdc_amd.model_evaluate(d, t)
+            except tdc_amd.TdcError:
+                continue
+            seen.add((cch, wk))
+            announce("split large stages", shape, K, stride, dil, t)
+            got = torch.from_numpy(run_conv(x, w, stride=stride, pad=pad, dil=dil, tile=t)).double()
+            assert (got - exact).norm() <= 2e-7 * exact.norm(), f"{shape} {t}"
+            plan = tdc_amd.Conv2dPlan(B, C, N, H, W, K, K, stride, pad, dil, True, True, tile=t).set_weights(w, bias)
+            assert_close(run_slices(plan, x, resid, N, Ho, Wo), want_full, f"slices {shape} {t}")
+            plan.close()
+    assert {wk for _, wk in seen} >= {2, 4} and {cch for cch, _ in seen} == {64, 128}
 
 
 @pytest.mark.parametrize("shape,K,stride,pad", [((2, 40, 36, 8, 8), 1, 1, 0), ((2, 70, 20, 7, 7), 1, 1, 0), ((2, 40, 36, 9, 9), 3, 2, 1),
