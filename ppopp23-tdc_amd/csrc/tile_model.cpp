@@ -273,7 +273,7 @@ bool make_geometry(const tdc_conv_desc &d, const tdc_tile &t, Geometry &g, std::
     g.taps = d.KH * d.KW;
     g.ktaps = g.taps;
     g.MT = t.mf * t.mb * t.wm;
-    if (t.alg < 0 || t.alg > 7) return fail("tile.alg must be in [0, 9]");
+    if (t.alg < 0 || t.alg > 7) return fail("tile.alg must be in [0, 8]");
     if (t.alg == 5) {
         // Winograd F(2x2,3x3) streamed from global memory: 16*wm channels of one tile row block (2 rows x 28 columns) per
         // workgroup, the input channels split over wk waves in groups of four, everything in one pass
