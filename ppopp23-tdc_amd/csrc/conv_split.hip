@@ -45,7 +45,9 @@ namespace tdc {
 // 338 -> 176, 128 -> 128 @56 batch 64 164 -> 101, 64 -> 64 @56 batch 32 30 -> 23.  Not faster where a launch takes under 7 us, and
 // at 3x3 / stride 1, where Winograd saves more (128 -> 128 @56 batch 64 274 us against 267).
 // Not kept: requesting weights four blocks ahead and pixel operands one K-step ahead (0 to 10 % slower: fewer waves fit);
-// 64 channels x 32 pixels per wave in the 1x1 form (best nowhere by more than 3 %, often 10 % behind).
+// 64 channels x 32 pixels per wave in the 1x1 form (best nowhere by more than 3 %, often 10 % behind); four channel blocks with the
+// weights reloaded in place a K-step ahead and the six products of a K-step from zero (218 -> 124 @90 / stride 2 batch 27 162 -> 165,
+// 256 -> 256 @56 / stride 2 batch 40 177 -> 176, networks with the stem unchanged).
 // ---------------------------------------------------------------------------
 enum : int { SPLIT_FLAT = 0, SPLIT_WINDOW = 1, SPLIT_FEW = 2 };
 
