@@ -328,7 +328,7 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
         for (int m = 0; m < MB; ++m)
 #pragma unroll
             for (int i = 0; i < 4; ++i) own[(4 * m + i) * 64] = parted ? own[(4 * m + i) * 64] + output(m, i) : output(m, i);
-        const int rows = 4 * MB / p.WK;         // (WK = 2 or 4)
+        const int rows = (4 * MB - slice + p.WK - 1) / p.WK;   // (WK need not divide them: 3 is taken too)
         float bv[2 * MB];
         f4_t rv[2 * MB];
 #pragma unroll

@@ -1142,6 +1142,32 @@ def test_batched_winograd_sums_in_parts(shape, pad):
         plan.close()
 
 
+@pytest.mark.parametrize("shape,K,tile", [((2, 48, 40, 14, 9), 3, (1, 1, 1, 2, 3, 48, 0, 1)), ((2, 48, 40, 14, 9), 3, (2, 1, 1, 2, 3, 48, 0, 1)),
+                                          ((3, 280, 20, 6, 7), 3, (1, 2, 1, 2, 3, 288, 0, 1)), ((2, 280, 36, 5, 6), 3, (2, 1, 1, 2, 3, 288, 0, 1)),
+                                          ((2, 100, 40, 9, 7), 1, (1, 2, 1, 2, 3, 144, 1, 7)), ((2, 100, 40, 9, 7), 1, (2, 4, 1, 1, 3, 144, 1, 7)),
+                                          ((2, 300, 72, 5, 6), 1, (2, 2, 1, 1, 5, 320, 8, 7)), ((2, 300, 72, 5, 6), 1, (2, 4, 1, 1, 7, 336, 1, 7))])
+def test_rows_that_the_teams_do_not_divide(shape, K, tile):
+    """Three, five and seven teams (waves over input channels) share the 4 or 8 rows of a block unevenly: every row is finished, also
+    with the whole epilogue and where its sums come out infinite (as plain fp32 sums give them).  The model offers 1, 2, 4 and 8."""
+    B, C, N, H, W = shape
+    mb, nb, wm, wn, wk, cch, tw, alg = tile
+    t = tdc_amd.Tile(16, mb, nb, wm, wn, wk, cch, tw, 1, 0, alg)
+    announce("uneven rows", shape, K, t)
+    x, w = case(8797 + C, B, C, N, H, W, K)
+    g = seeded(8798)
+    bias, resid = torch.randn(N, generator=g), torch.randn(B, N, H, W, generator=g)
+    assert_close(run_conv(x, w, pad=K // 2, tile=t), ref.conv2d_c(x.numpy(), w.numpy(), pad=K // 2), f"{shape} {t}")
+    plan = tdc_amd.Conv2dPlan(B, C, N, H, W, K, K, 1, K // 2, 1, True, True, tile=t).set_weights(w, bias)
+    want = ref.conv2d_c(x.numpy(), w.numpy(), bias.numpy(), resid.numpy(), pad=K // 2, relu=True)
+    assert_close(run_slices(plan, x, resid, N, H, W), want, f"slices {shape} {t}")
+    plan.close()
+    x, w = x.abs() + 0.1, w.abs() + 0.1
+    x[0, 1, 2, 3] = float("inf")
+    want = torch.nn.functional.conv2d(x.double(), w.double(), None, 1, K // 2).float()
+    # (positive fp32 sums of at most 2520 products, a rounding of 2^-24 each: 1.5e-4; measured far below)
+    assert torch.allclose(torch.from_numpy(run_conv(x, w, pad=K // 2, tile=t)), want, rtol=1.5e-4, atol=0.0), f"inf {shape} {t}"
+
+
 @pytest.mark.parametrize("shape,K,stride,pad,dil", [
     ((3, 20, 24, 7, 5), 1, 1, 0, 1), ((2, 33, 40, 9, 9), 1, 1, 0, 1), ((5, 300, 70, 7, 7), 1, 1, 0, 1), ((9, 64, 130, 2, 2), 1, 1, 0, 1),
     ((3, 70, 17, 1, 3), 1, 1, 0, 1), ((2, 260, 64, 12, 11), 1, 1, 0, 1), ((3, 16, 20, 7, 7), 3, 1, 1, 1), ((2, 40, 36, 13, 9), 3, 2, 1, 1),
