@@ -921,19 +921,20 @@ int kernel_vgprs(const KernelId &k) {
 
 // Price of the split-operand tiles for filters of several taps, in us: a power mean of what a SIMD has to issue (MFMAs, K-steps,
 // staging, stores), of the rounds of workgroups that each take their own chain of stages, and of the weights' way through the
-// L1s, + launch + memory traffic.  `staged`: bytes of LDS per pixel (pair) and octet.
+// L1s, + launch + memory traffic.  `last`: share of a last, partly filled round of workgroups that counts as a whole one; `idle`: what a
+// launch of fewer workgroups than compute units saves.
 struct SplitPrice {
     double pipe_mfma, pipe_step, pipe_stage, pipe_block;
     double start, stage, stage_entry, step, mfma, block;
     double weights, launch_us, traffic, power, fragment;
-    double staged;
+    double last, idle;
 };
-static const SplitPrice split_core_price = {0.739, 191.1, 460.1, 600.3, 2930, 2593, 1098, 303.2, 0.8651, 417.2, 1.009, 3.726, 34.35, 2.024, 0.3892, 48};
+static const SplitPrice split_core_price = {0.739, 191.1, 460.1, 600.3, 2930, 2593, 1098, 303.2, 0.8651, 417.2, 1.009, 3.726, 34.35, 2.024, 0.3892, 0.5, 0.0};
 static double split_price(const SplitPrice &q, const tdc_conv_desc &d, const tdc_tile &t, const Geometry &g, int wg_per_cu) {
     const double wgs = (double)g.grid_x * g.grid_y / machine().cus;
-    const double load = 0.5 * (std::ceil(wgs) + std::max(wgs, 1.0)), simd = (double)g.waves / machine().simds_per_cu;
+    const double load = q.last * std::ceil(wgs) + (1.0 - q.last) * std::max(wgs, 1.0), simd = (double)g.waves / machine().simds_per_cu;
     const double steps = (double)g.nchunks * g.ksteps / t.wk, blocks = t.mb * t.nb, mfmas = steps * blocks * 96.0;
-    const double entries = (g.lds_bytes - 32) / q.staged / g.threads;
+    const double entries = (g.lds_bytes - 32) / 48.0 / g.threads;
     const double stores = blocks * (1.0 + q.fragment * (16.0 / std::min(t.tw, 16) - 1.0));   // (short rows make short stores)
     const double shared = std::max(1.0, 0.75 * std::min(std::min((double)wg_per_cu, std::max(1.0, std::ceil(wgs))) * simd, 2.0));
     const double pipe = load * simd * (q.pipe_mfma * mfmas + q.pipe_step * steps + q.pipe_stage * g.nchunks * entries + q.pipe_block * stores);
@@ -942,8 +943,10 @@ static double split_price(const SplitPrice &q, const tdc_conv_desc &d, const tdc
     const double l1 = q.weights * load * simd * 4.0 * steps * t.mb * 3072.0 / 56.0;
     const double clk = std::pow(std::pow(pipe, q.power) + std::pow(chain, q.power) + std::pow(l1, q.power), 1.0 / q.power);
     const double traffic = 4.0 * d.batch * ((double)d.C * d.H * d.W + (double)d.N * g.P) + 6.0 * d.C * d.N * g.ktaps;
-    return q.launch_us + clk / (machine().clock_ghz * 1e3) + traffic / (q.traffic * 1e6);
+    return std::pow(std::min(wgs, 1.0), q.idle) * (q.launch_us + clk / (machine().clock_ghz * 1e3) + traffic / (q.traffic * 1e6));
 }
+
+static bool is_core_split(const tdc_tile &t) { return t.alg == 8 && t.tw > 0 && t.nb == 2; }   // (conv_core_split.hip)
 
 bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &info, std::string *why, int tail_N) {
     Geometry g;
@@ -1164,11 +1167,10 @@ bool model_evaluate(const tdc_conv_desc &d, const tdc_tile &t, tdc_tile_info &in
         info.pred_l2_bytes = 0.0;
         return true;
     }
-    if (t.alg == 8 && t.tw > 0 && t.nb == 2) {
+    if (is_core_split(t)) {
         // Fitted to 15000 timed tiles of 1000 shapes (most at 3x3 / stride 2): 6 % mean error, 2.5 % mean loss of the pick within the
-        // family.  At 0.86 one shape in eight gains more than 2 % over its former pick (its time falls by 18 % in the mean, most where
-        // the staged kernel took it), and three in a thousand lose more, 5 to 8 % (0.80: 16 % gain, 3 % lose; 0.92: 6 % and 0.3 %):
-        // the line falls at about 12 us at stride 2.
+        // family.  The factor in front: the formula of the staged tiles is 40 % kind in the mean to those it meets.  What a pick by this
+        // price gains and loses stands at core_split_takes.
         info.pred_us = 0.86 * split_price(split_core_price, d, t, g, wg_per_cu);
         info.pred_l2_bytes = 0.0;
         return true;
@@ -1628,15 +1630,45 @@ std::vector<tdc_tile_info> model_choices(const tdc_conv_desc &d, int tail_N) {
     return infos;
 }
 
+// Whether the split-operand form of 32 pixels per wave, the cheaper one by price, takes the place of the best other tile.  Timed in turn
+// with the tile it would displace, over the 3252 of 20400 random layers (2x2 to 7x7, strides 1 to 3, dilation 2; batch 1 to 64, 16 to
+// 1024 channels, 0.3 to 25 Gflop) where that price is the lower one:
+//   staged direct tiles (1492 layers): 0.74 of their time in the mean; 41 are more than 2 % slower, up to 16 %, most of them at 10 to 14 us,
+//     and no limit on the price or the length of a launch parts those from more than three times as many that gain.
+//   the form of 64 pixels per wave (1683): 0.96, but 408 are slower, up to 38 %: one stage only, or eight waves that share no K-steps, or
+//     a launch that the larger tiles fill better.  The two formulas are 7 % apart in what they make of such pairs; so this choice goes by one
+//     formula fitted to 3800 and 1800 timed tiles of both (5 %), and the new form has to be 2 % lower: it takes 1065 of the layers at 0.92
+//     of their time, 43 of them more than 2 % slower (up to 19 %), and leaves 618, on which it would need 1.045.
+//   streamed and Winograd tiles (77): 0.985, 29 slower, up to 22 %: left alone.
+// The error against 64-bit sums is at most 0.97 of that of the tile displaced.
+static bool core_split_takes(const tdc_conv_desc &d, const tdc_tile &core, const tdc_tile &other) {
+    if (other.alg == 0 || other.alg == 2) return true;
+    if (other.alg != 8) return false;
+    static const SplitPrice of_core = {0.0, 197.3, 138.8, 934.7, 3074, 1993, 2116, 34.23, 0.101, 0.0, 1.432, 2.812, 37.84, 1.517, 0.2695, 0.6759, 0.1105};
+    static const SplitPrice of_other = {0.0, 211.6, 763.8, 635.5, 0.0, 3036, 1168, 294.7, 0.7946, 231.1, 2.445, 3.297, 45.78, 2.322, 0.4946, 0.6586, 0.1059};
+    auto price = [&](const SplitPrice &q, const tdc_tile &t) {
+        Geometry g;
+        tdc_tile_info info;
+        make_geometry(d, t, g, nullptr, 0);
+        model_evaluate(d, t, info, nullptr, 0);
+        return split_price(q, d, t, g, info.wg_per_cu);
+    };
+    return price(of_core, core) < 0.98 * price(of_other, other);
+}
+
 bool model_select(const tdc_conv_desc &d, tdc_tile_info &best, std::string *why, int tail_N) {
     if (!check_desc(d, why)) return false;
     double limit;
     const std::vector<tdc_tile> tiles = model_enumerate(d, tail_N);
     const std::vector<Choice> cands = choices_within(d, tail_N, tiles, limit);
     const bool batched = std::any_of(cands.begin(), cands.end(), [&](const Choice &c) { return tiles[c.tile].alg == 1 && tiles[c.tile].tw == 0; });
-    const Choice *pick = nullptr;
+    const Choice *pick = nullptr, *core = nullptr;
     double best_us = 0.0;
     for (const Choice &c : cands) {
+        if (is_core_split(tiles[c.tile])) {
+            if (!core || c.us < core->us) core = &c;
+            continue;
+        }
         // (the handicap takes the pick from a staged tile, but not to a kernel with a larger error)
         if (batched && tiles[c.tile].alg < 7 && rounding_variance(d, tiles[c.tile]) > limit) continue;
         const double us = c.us * (batched ? c.handicap : 1.0);
@@ -1645,6 +1677,7 @@ bool model_select(const tdc_conv_desc &d, tdc_tile_info &best, std::string *why,
             best_us = us;
         }
     }
+    if (core && (!pick || (core->us < best_us && core_split_takes(d, tiles[core->tile], tiles[pick->tile])))) pick = core;
     const bool have = pick && model_evaluate(d, tiles[pick->tile], best, nullptr, tail_N);
     if (!have && why) {
         // say why the plainest tile cannot be launched: that is the limit the shape runs into

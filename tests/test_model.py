@@ -192,6 +192,25 @@ def test_blocked_1x1_chains_follow_the_kernel_they_replace(batch, C, N, H, W, pa
     assert t.alg == 7 and (t.tw if t.tw > 1 else t.cch // t.wk) <= part and (t.tw == 1) == (part == C)
 
 
+# (timed in turn: us of the tile that was displaced, us of the split-operand form of 32 pixels per wave)
+@pytest.mark.parametrize("batch,C,N,H,W,K,stride,dil,wins", [
+    (36, 32, 96, 82, 82, 2, 1, 1, False),     # 58.8, 80.9: the form of 64 pixels per wave
+    (61, 32, 96, 66, 66, 3, 2, 1, False),     # 42.3, 56.1: likewise
+    (22, 228, 77, 30, 32, 3, 1, 2, False),    # 58.3, 74.0: likewise
+    (24, 126, 139, 75, 32, 3, 3, 1, False),   # 32.6, 41.6: likewise
+    (10, 50, 134, 49, 25, 3, 2, 1, False),    # 11.0, 13.4: streamed
+    (1, 63, 163, 65, 45, 3, 1, 1, False),     # 11.1, 13.0: streamed
+    (46, 256, 480, 11, 11, 3, 2, 1, True),    # 55.5, 34.4: the form of 64 pixels per wave
+    (11, 192, 242, 33, 40, 3, 2, 1, True),    # 43.7, 29.6: likewise
+    (26, 256, 240, 22, 22, 3, 2, 1, True),    # 86.8, 37.6: staged
+    (33, 103, 240, 19, 17, 3, 2, 1, True),    # 43.0, 20.1: staged, weights from memory
+    (21, 256, 64, 17, 17, 5, 1, 1, True),     # 112.4, 45.9: staged
+])
+def test_split_operands_at_32_pixels_per_wave_only_where_they_are_faster(batch, C, N, H, W, K, stride, dil, wins):
+    t = tdc_amd.model_select(tdc_amd.conv_desc(batch, C, N, H, W, K, K, stride, K // 2 * dil, dil)).tile
+    assert (t.alg == 8 and t.tw > 0 and t.nb == 2) == wins, t
+
+
 def test_algorithmic_work_and_roofline_of_config1():
     i = tdc_amd.model_select(conv3(32, 32, 56))
     assert i.flops == 2 * 56 * 56 * 32 * 32 * 9 == 57802752
