@@ -38,8 +38,8 @@ def _short(name):
 
 
 def _is_conv(name):
-    """A dispatch of one of the convolution kernels (staged, streamed, streamed Winograd)."""
-    return "tdc_conv" in name or "tdc_wino" in name
+    """A dispatch of one of the convolution kernels."""
+    return any(part in name for part in ("tdc_conv", "tdc_wino", "tdc_core_split"))
 
 
 def kernel_summary(path, out=sys.stdout):

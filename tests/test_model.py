@@ -297,3 +297,12 @@ def test_model_register_table_matches_the_compiled_kernels():
         assert regs == (real + 7) // 8 * 8, f"{name}: model assumes {regs} registers per lane, compiled kernel uses {real}"
         # the compiler's own waves-per-SIMD figure (vector and scalar register limits) is the model's
         assert compiled[name]["waves_per_simd"] == waves, f"{name}: {compiled[name]} against the model's {waves} waves per SIMD"
+
+
+def test_profile_summaries_know_the_kernel_of_every_tile():
+    from tdc_amd import _lib, profsum
+    names = set()
+    for d in (conv3(128, 128, 56), tdc_amd.conv_desc(8, 64, 64, 56, 56, 3, 3, 1, 1), tdc_amd.conv_desc(8, 256, 64, 56, 56, 1, 1, 1, 0)):
+        names |= {_lib.model_kernel_info(d, t, False)[0] for t in tdc_amd.model_enumerate(d)}
+    assert len({n.split("<")[0] for n in names}) == 9   # (all families)
+    assert all(profsum._is_conv(n) for n in names), [n for n in names if not profsum._is_conv(n)]
