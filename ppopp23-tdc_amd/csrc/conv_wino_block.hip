@@ -328,12 +328,12 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
         for (int m = 0; m < MB; ++m)
 #pragma unroll
             for (int i = 0; i < 4; ++i) own[(4 * m + i) * 64] = parted ? own[(4 * m + i) * 64] + output(m, i) : output(m, i);
-        const int rows = (4 * MB - slice + p.WK - 1) / p.WK;   // (WK need not divide them: 3 is taken too)
+        // (WK need not divide the rows: 3 is taken too)
         float bv[2 * MB];
         f4_t rv[2 * MB];
 #pragma unroll
         for (int r = 0; r < 2 * MB; ++r) {
-            if (r >= rows) break;
+            if (slice + r * p.WK >= 4 * MB) break;
             const int row = slice + r * p.WK, ch = ch_base + 16 * (row >> 2) + (row & 3);
             bv[r] = p.bias ? p.bias[min(ch, p.N - 1)] : 0.0f;
             if (has_resid) rv[r] = load_resid(ch);
@@ -343,7 +343,7 @@ __global__ void __launch_bounds__(512, 2) tdc_wino3x3_block_kernel(const ConvKPa
         settle(rv);
 #pragma unroll
         for (int r = 0; r < 2 * MB; ++r) {
-            if (r >= rows) break;
+            if (slice + r * p.WK >= 4 * MB) break;
             const int row = slice + r * p.WK;
             f4_t v = part[row * 64];
             for (int s = 1; s < p.WK; ++s) v += part[(s * 4 * MB + row) * 64];
