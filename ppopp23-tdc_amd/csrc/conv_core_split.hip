@@ -13,29 +13,35 @@ namespace tdc {
 // stage, which run over its (tap, octet) pairs, are divided among the WK waves; their sums meet in LDS.  At stride 2 the even and
 // the odd columns lie in separate halves of a row, so that neighbouring lanes read neighbouring slots.
 // Bound: the latencies of one workgroup's chain and the issue slots of the SIMDs, not the matrix pipes: 128 -> 128 @28 / stride 2
-// batch 32 has 4.7 us of MFMAs at the rate a bare loop reaches and 3.1 us of memory traffic, and takes 22.8.  Hence
+// batch 32 has 5.0 us of MFMAs and 3.1 us of memory traffic.  Of the 19.7 us of its kernel (time stamps) a wave takes 2.5 until its
+// first requests are out, 2.4 until they have landed and are split, 0.7 at the barrier, 10.3 for its 18 K-steps, 1.7 until the sums of
+// the slices are added and 1.0 for the stores.  Hence
 //   - the next stage is requested in front of the MFMAs of this one (four entries a thread; what a larger stage has beyond that
 //     comes in rounds of its own), and the weights of a K-step are reloaded in place right behind the MFMAs that read them, a K-step
 //     ahead: a ring that copies registers would make every copy wait for what was requested last;
-//   - the three parts of a slot lie together, 48 bytes, one address for three reads, and octets a multiple of 16 slots apart,
-//     so the four lane quarters, an octet each, meet in no bank;
+//   - the three parts of a slot lie together, 48 bytes, one address for three reads, and octets a multiple of 16 slots, whole rounds
+//     of the banks, apart, so that all four lane quarters meet the same banks.  Conflicts still take half of the cycles in which the LDS is active
+//     (48 to 55 % in three layers), but waves wait for it in 1 to 2 % of their time only;
 //   - all six products of a K-step start from zero and are added to the sums once: a single chain per block and half the
 //     accumulators.  The error against 64-bit sums at 3x3 and 64, 128 and 512 channels is 0.9, 1.2 and 2.2e-7 of the norm
 //     (with two accumulators that take the leading and the small products 1.3, 1.9 and 3.9e-7; one for all six throughout 3.7e-7
 //     at 128), at 16 channels 7.0e-8 (6.6e-8).
 // Two pixel blocks per wave: three to four waves per SIMD at mb = 1 and 2.  Four blocks, 24 operand registers more, are better where
-// a launch has more matrix work than latency: from about 30 Gflop, by 5 % with this staging, by 15 to 30 % with the four channel
-// blocks and smaller stages of conv_split.hip's form.
-// Measured (launch to launch, one box, us; before: the best of the other families, or that form): 3x3 / stride 2 128 -> 128 @28
-// batch 32 34.0 -> 22.8, 64 -> 64 @56 batch 32 27.1 -> 25.3, 256 -> 256 @14 batch 32 41.3 -> 27.8, 5x5 64 -> 96 @40 batch 16 65.9 ->
-// 58.0.  At 3x3 / stride 1 Winograd saves more.
+// a launch has more matrix work than latency, or only one stage, behind which nothing can be requested: conv_split.hip's form keeps those
+// layers (core_split_takes in tile_model.cpp).
+// Measured (in one graph, in turn with the best of the other tiles, us): 3x3 / stride 2 128 -> 128 @28 batch 32 30.0 -> 20.1, 64 -> 64
+// @56 batch 32 22.7 -> 21.9, 256 -> 256 @14 batch 32 36.7 -> 24.6, 5x5 64 -> 96 @40 batch 16 60.8 -> 53.1; over 2557 random layers that take
+// it 0.81 of the time.  At 3x3 / stride 1 Winograd saves more.
 // ---------------------------------------------------------------------------
 template <int MB>
 __global__ void __launch_bounds__(512, 2) tdc_core_split_kernel(const ConvKParams p) {
     constexpr int NB = 2;
     extern __shared__ __align__(16) float lds_all[];
     float *const lds = lds_all + EXTREMES_FLOATS;
+    TDC_STAMP_DECL;
+    TDC_STAMP(0);   // entry
     touch_kernel_arguments();
+    TDC_STAMP(7);   // every line of the kernel arguments is in the scalar cache
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -238,19 +244,24 @@ __global__ void __launch_bounds__(512, 2) tdc_core_split_kernel(const ConvKParam
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     };
     request_stage(0);
+    TDC_STAMP(1);   // first stage and first weights requested
 #pragma unroll 1
     for (int st = 0; st < p.nchunks; ++st) {
         if (st > 0) barrier();
         park_stage(st);
+        if (st == 0) TDC_STAMP(2);   // my part of the first stage has landed and is split
         if (st + 1 == p.nchunks) {
             const unsigned met = (__builtin_amdgcn_ballot_w64(extremes.tiny()) ? 1u : 0u) | (__builtin_amdgcn_ballot_w64(extremes.large()) ? 2u : 0u);
             if (lane == 0) reinterpret_cast<unsigned *>(lds_all)[wave] = met;
         }
         barrier();
+        if (st == 0) TDC_STAMP(3);   // everybody's is
         request_stage(st + 1);                  // (past the last stage: nothing but offsets out of range)
         __builtin_amdgcn_sched_barrier(0);
         multiply(st);
     }
+
+    TDC_STAMP(4);   // all stages multiplied
 
     // ---- results ---------------------------------------------------------------------------------------------------------
     const unsigned met_word = reinterpret_cast<const unsigned *>(lds_all)[lane & 7];
@@ -276,6 +287,7 @@ __global__ void __launch_bounds__(512, 2) tdc_core_split_kernel(const ConvKParam
                 acc[m][j] = v;
             }
     }
+    TDC_STAMP(5);   // sums of all slices added
     auto mine = [&](int r) { return p.WK == 1 || r % p.WK == slice; };
     Range range;
 #pragma unroll
@@ -342,6 +354,8 @@ __global__ void __launch_bounds__(512, 2) tdc_core_split_kernel(const ConvKParam
         for (int m = 0; m < MB; ++m)
             if (mine(m * NB + j)) store_four_channels(acc[m][j], ch_base + 16 * m, p.N, p.P, px.pix, bias[m], has_resid, resid[m * NB + j], p.relu, out);
     }
+    TDC_STAMP(6);   // stores issued
+    TDC_STAMP_FLUSH(p, logical, wave, lane);
 }
 
 const void *core_split_kernel_function(const KernelId &k) {

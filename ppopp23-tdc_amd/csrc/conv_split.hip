@@ -37,7 +37,7 @@ namespace tdc {
 // last stage: waiting for it in front of the first one, behind weights that come from memory, cost the networks 0.8 %.
 // AFF: per-channel affine (+ ReLU) on the input of a 1x1 convolution.
 // Bound: no single one.  512 -> 128 @28 batch 32 takes 26 us: 9 us of MFMAs at the 390 TFLOP/s of fp32 products that a bare MFMA
-// loop reaches, 13 us of memory traffic, and between them LDS reads (a half of the MFMA time at mb = 2), the splitting (6
+// loop reaches, 13 us of memory traffic, and between them LDS reads (a half of the MFMA time at mb = 2), the splitting (5
 // vector operations an element) and two barriers a stage, which two to four waves per SIMD overlap only in part.
 // Against the best tile of the other families (launch-to-launch, one box, us): 512 -> 128 @28 batch 32 38 -> 26, 128 -> 512 @28
 // batch 32 46 -> 28, 256 -> 2048 @7 batch 64 44 -> 28, 2048 -> 256 @7 batch 64 43 -> 32, 976 -> 866 @40 batch 5 138 -> 85, 256 -> 128

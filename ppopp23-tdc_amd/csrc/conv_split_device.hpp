@@ -25,7 +25,7 @@ struct Range {
 };
 
 // What a thread has met among the values it split: whether any is below 2^-110 but not zero, and whether any reaches 2^20.  Two
-// vector instructions a value (beside six for the split).
+// vector instructions a value (beside five for the split).
 struct Extremes {
     unsigned low = ~0u;
     float high = 0.0f;
